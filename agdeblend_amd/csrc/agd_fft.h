@@ -7,7 +7,7 @@
 // array stays in VGPRs, and every twiddle is a compile-time constant folded
 // into the instruction stream (no table loads). Radix order: 4s, then 2,
 // then odd primes; radix 2/3/4/5 butterflies are specialised, other primes
-// use a direct butterfly with constant roots.
+// use the DFT on symmetric pairs with constant roots.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -140,22 +140,33 @@ __device__ __forceinline__ void butterfly(float2 (&v)[R]) {
     v[2] = c_add(r2, i2);
     v[3] = c_sub(r2, i2);
   } else {
-    float2 o[R];
+    // odd R: pairs v_k +- v_{R-k} against cos and sin, half the products of
+    // the plain sum
+    constexpr int H = (R - 1) / 2;
+    float2 a[H], b[H];
+    float2 const x0 = v[0];
+    float2 sum = x0;
 #pragma unroll
-    for (int q = 0; q < R; ++q) {
-      float2 a = v[0];
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        if ((q * r) % R == 0) {
-          a = c_add(a, v[r]);
-        } else {
-          a = c_add(a, c_mul(v[r], root<R, S>(q * r)));
-        }
-      }
-      o[q] = a;
+    for (int k = 1; k <= H; ++k) {
+      a[k - 1] = c_add(v[k], v[R - k]);
+      b[k - 1] = c_sub(v[k], v[R - k]);
+      sum = c_add(sum, a[k - 1]);
     }
+    v[0] = sum;
 #pragma unroll
-    for (int q = 0; q < R; ++q) v[q] = o[q];
+    for (int q = 1; q <= H; ++q) {
+      float2 c = x0, d = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int k = 1; k <= H; ++k) {
+        float2 const w = root<R, S>(q * k);
+        c.x += w.x * a[k - 1].x;
+        c.y += w.x * a[k - 1].y;
+        d.x += w.y * b[k - 1].x;
+        d.y += w.y * b[k - 1].y;
+      }
+      v[q] = make_float2(c.x - d.y, c.y + d.x);
+      v[R - q] = make_float2(c.x + d.y, c.y - d.x);
+    }
   }
 }
 

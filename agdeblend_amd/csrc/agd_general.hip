@@ -1,0 +1,736 @@
+// Transforms of any window size, up to four space dims (HIP kernels and their
+// launchers, declared in agd_general.h).
+//
+// A patch whose size is not a multiple of its half windows gets windows one
+// or a few samples longer than asked for, so padded lengths such as 23, 42
+// or 43 are the usual case, not the exception. These kernels take the
+// lengths at run time. Every 1-D transform is a line held by one thread in
+// registers (line_dft): the DFT of P values on the pairs
+//   a_k = x_k + x_{P-k},  b_k = x_k - x_{P-k},   0 < k < P / 2,
+//   X_q, X_{P-q} = (x_0 + (-1)^q x_{P/2} + sum a_k cos(2 pi q k / P))
+//                  +- i S sum b_k sin(2 pi q k / P),
+// i.e. P^2 real multiply-adds for P complex outputs, half of the plain sum,
+// with coefficients that are the same for every thread and come through
+// the scalar cache as instruction operands. No roots, divisions or LDS
+// traffic inside a line, and no dependence on how P factors. Lengths without
+// a prime factor above 13 take a register FFT instead (codelets).
+//
+// Measured (MI355X) on a 45 x 333 x 1500 volume in two patches, windows of
+// 17-18 x 24-25 x 200 (P = 22, 23 x 30, 32, Pt = 250; model 1.15 GB), us per
+// iteration: spatial transforms and update 15480 by the LDS-resident kernels
+// (radix passes through LDS with table roots, forward and adjoint apart) ->
+// 1640 lines as above -> 1620 with the codelets -> 990 with reciprocals for
+// integer divisions; it moves 3.9 GB, 820 us at this card's copy rate. Time
+// transforms 1460 and 1670 -> 480 and 500. Prefetching the model's values
+// ahead of the transforms changed nothing (the lines' registers are worth
+// more as waves).
+#include <hip/hip_runtime.h>
+
+#include "agd_fft.h"
+#include "agd_general.h"
+#include "agd_launch.h"
+
+namespace agdgen {
+
+// coefficient tables are read through the scalar cache (constant address
+// space, block-uniform addresses)
+typedef float __attribute__((address_space(4))) cfloat;
+__device__ __forceinline__ cfloat const *uniform(float const *p, int off) {
+  return (cfloat const *)(uintptr_t)(p + __builtin_amdgcn_readfirstlane(off));
+}
+
+// rows of the coefficient table of length P: for q = 1 .. (P - 1) / 2 the
+// pairs cos, sin(2 pi q k / P), k = 1 .., padded with zeros to whole groups
+// of 4 pairs (built by the host, dft_get)
+__device__ __forceinline__ int table_row(int P) { return 2 * (((P - 1) / 2 + 3) & ~3); }
+
+// One line's inputs as the pairs a, b (and x_0, x_{P/2}).
+template <int HB>
+struct Line {
+  float2 a[HB], b[HB], x0, xh;
+
+  // the line ln[k st], k < P: the inputs k >= nin are zero. P - 1 <= 2 HB.
+  // Everything but ln is uniform over the block.
+  __device__ __forceinline__ void load(float2 const *ln, int st, int P, int nin) {
+    int const h = (P - 1) >> 1;
+    x0 = ln[0];
+    xh = make_float2(0.f, 0.f);
+    if (!(P & 1) && P / 2 < nin) xh = ln[(P / 2) * st];
+#pragma unroll
+    for (int c = 0; c < HB; c += 4) {
+      if (c < h) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          int const k = c + u + 1;
+          // clamped loads, values outside the line or its inputs unused
+          float2 const p = ln[min(k, nin - 1) * st];
+          float2 const m = ln[max(0, min(P - k, nin - 1)) * st];
+          bool const hp = k <= h && k < nin, hm = k <= h && P - k < nin;
+          float2 const x = make_float2(hp ? p.x : 0.f, hp ? p.y : 0.f);
+          float2 const y = make_float2(hm ? m.x : 0.f, hm ? m.y : 0.f);
+          a[c + u] = make_float2(x.x + y.x, x.y + y.y);
+          b[c + u] = make_float2(x.x - y.x, x.y - y.y);
+        }
+      }
+    }
+  }
+
+  // DFT of sign S: the outputs of part `part` of `parts` (uniform over the
+  // wave) below nout to out(q, X_q)
+  template <int S, class Out>
+  __device__ __forceinline__ void dft(int P, int nout, cfloat const *tab, int part, int parts,
+                                      Out const &out) const {
+    int const h = (P - 1) >> 1;
+    if (part == 0) {
+      float2 sum = x0, alt = x0;
+#pragma unroll
+      for (int c = 0; c < HB; c += 4) {
+        if (c < h) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            sum.x += a[c + u].x;
+            sum.y += a[c + u].y;
+            if (u & 1) {  // k = c + u + 1 is even
+              alt.x += a[c + u].x;
+              alt.y += a[c + u].y;
+            } else {
+              alt.x -= a[c + u].x;
+              alt.y -= a[c + u].y;
+            }
+          }
+        }
+      }
+      out(0, make_float2(sum.x + xh.x, sum.y + xh.y));
+      if (!(P & 1) && P / 2 < nout) {
+        float const s = (P / 2) & 1 ? -1.f : 1.f;
+        out(P / 2, make_float2(alt.x + s * xh.x, alt.y + s * xh.y));
+      }
+    }
+    int const row = table_row(P), q1 = 1 + h * (part + 1) / parts;
+    int q = 1 + h * part / parts;
+    for (tab += (q - 1) * row; q < q1; ++q, tab += row) {
+      float const s = q & 1 ? -1.f : 1.f;
+      float cr = x0.x + s * xh.x, ci = x0.y + s * xh.y, sr = 0.f, si = 0.f;
+#pragma unroll
+      for (int c = 0; c < HB; c += 4) {
+        if (c < h) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            float const co = tab[2 * (c + u)], sn = tab[2 * (c + u) + 1];
+            cr += co * a[c + u].x;
+            ci += co * a[c + u].y;
+            sr += sn * b[c + u].x;
+            si += sn * b[c + u].y;
+          }
+        }
+      }
+      if (S < 0) {
+        sr = -sr;
+        si = -si;
+      }
+      // C +- i S (sr + i si)
+      if (q < nout) out(q, make_float2(cr - si, ci + sr));
+      if (P - q < nout) out(P - q, make_float2(cr + si, ci - sr));
+    }
+  }
+};
+
+// The DFTs of `total` lines in place, 64 to a wave: line l at at(l), output
+// q of it through put(l, line, q, value). Up to 64 (128) lines are shared by
+// four (two) waves, each computing a part of every line's outputs, so that
+// short batches still use the whole block; a barrier then separates the
+// waves' loads from the first output. Ends with a barrier.
+template <int HB, int S, class At, class Put>
+__device__ __forceinline__ void block_lines(int total, int st, int P, int nin, int nout,
+                                            cfloat const *tab, At const &at, Put const &put) {
+  int const lane = threadIdx.x & 63;
+  int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Line<HB> ln;
+  if (total <= 128) {
+    int const parts = total <= 64 ? 4 : 2, part = total <= 64 ? wave : wave >> 1;
+    int const l = total <= 64 ? lane : (wave & 1) * 64 + lane;
+    auto const z = at(min(l, total - 1));
+    ln.load(z.p, st, P, nin);
+    __syncthreads();
+    if (l < total)
+      ln.template dft<S>(P, nout, tab, part, parts, [&](int q, float2 v) { put(z, q, v); });
+  } else {
+    for (int l = threadIdx.x; l < total; l += 256) {
+      auto const z = at(l);
+      ln.load(z.p, st, P, nin);
+      ln.template dft<S>(P, nout, tab, 0, 1, [&](int q, float2 v) { put(z, q, v); });
+    }
+  }
+  __syncthreads();
+}
+
+// a / d of small non-negative integers (a < 2^14 or so), inv = 1.f / d
+__device__ __forceinline__ int quot(int a, float inv) {
+  return (int)(((float)a + 0.5f) * inv);
+}
+
+// ---------------------------------------------------------------------------
+// Spatial transforms: one block holds nk time-frequency planes of one (window,
+// time window) in LDS, each a padded [P_0]..[P_{n-1}] array with rows of
+// (P_{n-1} | 1) values (an odd pitch: the lanes of a row transform read
+// distinct banks). Lines along a dim are transformed in place, one thread per
+// line; the model is read and written once, coalesced, between the adjoint's
+// dims (last to first) and the next forward's (first to last).
+// ---------------------------------------------------------------------------
+typedef int i4 __attribute__((ext_vector_type(AGD_MAXSP)));
+struct Planes {
+  int nsp, rows, pitch, rp;  // rows of a plane, row pitch, values of a plane
+  i4 ext, str, P, W;         // per space dim
+};
+
+// a[i], uniform, without indexed registers
+__device__ __forceinline__ int pick(i4 a, int i) {
+  static_assert(AGD_MAXSP == 4, "four space dims");
+  return i == 0 ? a.x : i == 1 ? a.y : i == 2 ? a.z : a.w;
+}
+
+// Padded lengths with a register codelet: no prime factor above 13, where the
+// factored transform takes a third to a fifth of P^2 multiply-adds. The
+// codelet knows the window length (W = 4 P / 5, rounded down: P = ceil(5 W /
+// 4)): S < 0 reads W values and writes P, S > 0 the other way.
+template <int P, int S>
+__device__ __forceinline__ void codelet(float2 *ln, int st) {
+  constexpr int W = P * 4 / 5, NIN = S < 0 ? W : P, NOUT = S < 0 ? P : W;
+  float2 v[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) v[k] = k < NIN ? ln[k * st] : make_float2(0.f, 0.f);
+  agdfft::fft<P, S>(v);
+#pragma unroll
+  for (int k = 0; k < NOUT; ++k) ln[k * st] = v[k];
+}
+// codelet P of the list Ps run on every line, or false
+template <int S, class At>
+__device__ __forceinline__ bool codelets(int, int, int, At const &) {
+  return false;
+}
+template <int S, int N, int... Ps, class At>
+__device__ __forceinline__ bool codelets(int P, int total, int st, At const &at) {
+  if (P == N) {
+    for (int l = threadIdx.x; l < total; l += 256) codelet<N, S>(at(l).p, st);
+    __syncthreads();
+    return true;
+  }
+  return codelets<S, Ps...>(P, total, st, at);
+}
+
+// transforms every line along dim d of the nk planes in place; the other
+// dims run over their current extents g.ext
+template <int HB, int S>
+__device__ __forceinline__ void lines(float2 *sm, Planes &g, int nk, int d, int nin, int nout,
+                                      cfloat const *tab) {
+  int cnt = 1;
+#pragma unroll
+  for (int e = 0; e < AGD_MAXSP; ++e)
+    if (e < g.nsp && e != d) cnt *= g.ext[e];
+  int const total = nk * cnt, st = pick(g.str, d), P = pick(g.P, d);
+  float const inv = 1.f / (float)cnt;
+  struct At {
+    float2 *p;
+  };
+  auto const at = [&](int l) {
+    int const k = quot(l, inv);
+    int r = l - k * cnt, off = k * g.rp;
+#pragma unroll
+    for (int e = AGD_MAXSP - 1; e >= 0; --e) {
+      if (e < g.nsp && e != d) {
+        int const q = quot(r, 1.f / (float)g.ext[e]);
+        off += (r - q * g.ext[e]) * g.str[e];
+        r = q;
+      }
+    }
+    return At{sm + off};
+  };
+  bool done = codelets<S, 8, 9, 10, 12, 13, 14, 15>(P, total, st, at);
+  if constexpr (HB >= 16)
+    if (!done) done = codelets<S, 18, 20, 22, 24, 25, 27, 28, 30, 32, 33>(P, total, st, at);
+  if constexpr (HB >= 24)
+    if (!done) done = codelets<S, 35, 39, 40, 42, 44, 45, 48, 49>(P, total, st, at);
+  if constexpr (HB >= 32)
+    if (!done) done = codelets<S, 50, 52, 54, 55, 60, 63, 64, 65>(P, total, st, at);
+  if (!done)
+    block_lines<HB, S>(total, st, P, nin, nout, tab, at,
+                       [&](At const &z, int q, float2 v) { z.p[q * st] = v; });
+#pragma unroll
+  for (int e = 0; e < AGD_MAXSP; ++e)
+    if (e == d) g.ext[e] = nout;
+}
+
+// the window's traces of the nk planes, between LDS and the tiles of U / V
+// ([tile of 16 traces][Ft][16] per time window): a tile's nk planes are
+// contiguous. Indices by reciprocals (an integer division is ~35
+// instructions, and these two loops were most of the kernel's).
+template <bool TO_LDS>
+__device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr, int Ft,
+                                           float2 *utw, int k0, int nk) {
+  constexpr int NB = 8;  // loads issued together
+  int const span = nk * 16, total = ((ntr + 15) >> 4) * span;
+  float const is = 1.f / (float)span;
+  float const i1 = 1.f / (float)g.W.y, i2 = 1.f / (float)g.W.z, i3 = 1.f / (float)g.W.w;
+  for (int i0 = threadIdx.x; i0 < total; i0 += NB * 256) {
+    float2 v[NB];
+    int lp[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      int const i = min(i0 + b * 256, total - 1);
+      int const t = quot(i, is), rem = i - t * span, k = rem >> 4;
+      int const tr = t * 16 + (rem & 15);
+      float2 *const u = utw + ((unsigned)t * (unsigned)Ft + (unsigned)k0) * 16u + (unsigned)rem;
+      int r = tr, off = k * g.rp;
+      if (g.nsp > 3) {
+        int const q = quot(r, i3);
+        off += (r - q * g.W.w) * g.str.w;
+        r = q;
+      }
+      if (g.nsp > 2) {
+        int const q = quot(r, i2);
+        off += (r - q * g.W.z) * g.str.z;
+        r = q;
+      }
+      if (g.nsp > 1) {
+        int const q = quot(r, i1);
+        off += (r - q * g.W.y) * g.str.y;
+        r = q;
+      }
+      off += r * g.str.x;
+      lp[b] = i0 + b * 256 < total && tr < ntr ? off : -1;
+      if (TO_LDS)
+        v[b] = *u;
+      else if (lp[b] >= 0)
+        *u = sm[off];
+    }
+    if (TO_LDS) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        if (lp[b] >= 0) sm[lp[b]] = v[b];
+    }
+  }
+}
+
+// mode -1: forward only (X -> U); 0..4 as k_adj_spatial_t's MODE, followed by
+// the forward transform of the new model when fuse is set
+template <int HB>
+__global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_spatial_g(
+    AgdWin const *__restrict__ wins, AgdTask const *__restrict__ tasks, int task0,
+    float const *__restrict__ dft, float2 const *__restrict__ V, float2 *__restrict__ X,
+    float2 *__restrict__ U, float alpha, float lamb, float const *__restrict__ lamb_dev, int mode,
+    int fuse, unsigned int *__restrict__ maxbits) {
+  extern __shared__ float2 sm[];
+  if (lamb_dev != nullptr) lamb = lamb_dev[0];
+  AgdTask const t = tasks[task0 + blockIdx.x];
+  AgdWin const &w = wins[t.win];
+  int const nk = t.nk, nsp = w.nsp, last = w.P[nsp - 1];
+  Planes g;
+  g.nsp = nsp;
+  g.rows = w.S / last;
+  g.pitch = last | 1;
+  g.rp = g.rows * g.pitch;
+  {
+    int st = 1;
+#pragma unroll
+    for (int e = AGD_MAXSP - 1; e >= 0; --e) {
+      if (e < nsp) {
+        g.P[e] = w.P[e];
+        g.W[e] = w.W[e];
+        g.str[e] = st;
+        st *= e == nsp - 1 ? g.pitch : w.P[e];
+      } else {
+        g.P[e] = g.W[e] = g.str[e] = 1;
+      }
+    }
+  }
+  int64_t const uoff = w.u_off + (int64_t)t.tw * ((w.ntr + 15) / 16) * w.Ft * 16;
+  float2 *const x = X + w.x_off + ((int64_t)t.tw * w.Ft + t.k0) * w.S;
+  int const total = nk * w.S;
+  bool const has_x = mode == -1 || mode == 0 || mode == 2;
+  if (mode >= 0) {
+#pragma unroll
+    for (int e = 0; e < AGD_MAXSP; ++e) g.ext[e] = g.W[e];
+    tiles_copy<true>(sm, g, w.ntr, w.Ft, const_cast<float2 *>(V) + uoff, t.k0, nk);
+    __syncthreads();
+    for (int d = nsp - 1; d >= 0; --d)
+      lines<HB, -1>(sm, g, nk, d, pick(g.W, d), pick(g.P, d), uniform(dft, w.sdft[d]));
+  }
+  // value i sits at LDS offset i + (row of i) (pitch - last)
+  {
+    int const pad = g.pitch - last;
+    int const dr = 256 / last, dc = 256 - dr * last;
+    int row = threadIdx.x / last, col = threadIdx.x - row * last;
+    float mx = 0.f;
+    constexpr int NB = 8;  // loads issued together
+    for (int i0 = threadIdx.x; i0 < total; i0 += NB * 256) {
+    float2 v[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      if (has_x) v[b] = x[min(i0 + b * 256, total - 1)];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      int const i = i0 + b * 256;
+      if (i < total) {
+        float2 *const s = sm + i + row * pad;
+        float2 nv;
+        if (mode == -1) {
+          nv = v[b];
+        } else {
+          float2 const gv = *s;
+          if (mode == 3) {
+            nv = gv;
+          } else if (mode == 1 || mode == 4) {
+            nv = make_float2(0.f - alpha * gv.x, 0.f - alpha * gv.y);
+            mx = fmaxf(mx, nv.x * nv.x + nv.y * nv.y);
+          } else {
+            nv = make_float2(v[b].x - alpha * gv.x, v[b].y - alpha * gv.y);
+            if (mode == 0) {
+              // x (|x| - lamb) / |x| when |x| > lamb, else 0
+              float const q = nv.x * nv.x + nv.y * nv.y;
+              float const sh = fmaxf(1.f - lamb * __builtin_amdgcn_rsqf(q), 0.f);
+              nv.x *= sh;
+              nv.y *= sh;
+            }
+          }
+          if (mode != 4) x[i] = nv;
+        }
+        if (mode == -1 || fuse) *s = nv;
+      }
+      row += dr;
+      col += dc;
+      if (col >= last) {
+        col -= last;
+        ++row;
+      }
+    }
+    }
+    if (mode == 1 || mode == 4) {
+      __shared__ float red[4];
+      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        float m = red[0];
+        for (int q = 1; q < 4; ++q) m = fmaxf(m, red[q]);
+        atomicMax(maxbits, __float_as_uint(m));
+      }
+    }
+  }
+  if (mode == -1 || fuse) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < AGD_MAXSP; ++e) g.ext[e] = g.P[e];
+    for (int d = 0; d < nsp; ++d)
+      lines<HB, +1>(sm, g, nk, d, pick(g.P, d), pick(g.W, d), uniform(dft, w.sdft[d]));
+    tiles_copy<false>(sm, g, w.ntr, w.Ft, U + uoff, t.k0, nk);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Time transforms of any even window length. Pt = M1 M2 (host: gtime), as the
+// complex transform of pairs of neighbouring traces, z = x_a + i x_b: no
+// unpack twiddles, and odd Pt costs the same as even. A block takes a tile of
+// 16 traces (8 pairs) and its time windows [tw0, tw1) as the specialised
+// kernels do; per time window the M1 phase, twiddle and M2 phase run in place
+// on one LDS tile [8][pitch], pitch = 4 mod 8 (the pairs of a load or store
+// fall in distinct banks). Output n = n1 + M1 n2 sits at n1 M2 + n2 (pos).
+// Short lines, so the loads and barriers bound these kernels, and blocks per
+// CU hide them: a register prefetch of the next tile in the forward, which
+// takes a wave per SIMD, ran 656 against 484 us on the volume above.
+// ---------------------------------------------------------------------------
+constexpr int kPairs = 8;
+__host__ __device__ constexpr int time_pitch(int Pt) { return (Pt + 3) / 8 * 8 + 4; }
+
+struct TimeTables {
+  float2 *Z, *TW;
+  unsigned short *pos;
+};
+
+template <int S>
+__device__ __forceinline__ void time_tables(TimeTables const &t, float2 const *roots, int N,
+                                            int M1, int M2) {
+  float const i1 = 1.f / (float)M1;
+  for (int m = threadIdx.x; m < N; m += 256) {
+    // TW[k2 M1 + n1] = exp(S 2 pi i n1 k2 / N)
+    int const k2 = quot(m, i1), n1 = m - k2 * M1;
+    float2 const r = roots[n1 * k2];  // n1 k2 < N
+    t.TW[m] = make_float2(r.x, S > 0 ? -r.y : r.y);
+    t.pos[m] = (unsigned short)(n1 * M2 + k2);  // of output m = n1 + M1 n2, n2 = k2
+  }
+}
+
+template <int HB, int S>
+__device__ __forceinline__ void time_fft(TimeTables const &t, int pitch, int M1, int M2,
+                                         float const *dft, int d1, int d2) {
+  struct At {
+    float2 *p;
+    float2 const *tw;
+  };
+  if (M1 > 1) {
+    float const i2 = 1.f / (float)M2;
+    block_lines<HB, S>(
+        kPairs * M2, M2, M1, M1, M1, uniform(dft, d1),
+        [&](int l) {
+          int const p = quot(l, i2), k2 = l - p * M2;
+          return At{t.Z + p * pitch + k2, t.TW + k2 * M1};
+        },
+        [&](At const &z, int q, float2 v) {
+          z.p[q * M2] = q == 0 ? v : agdfft::c_mul(v, z.tw[q]);
+        });
+  }
+  float const i1 = 1.f / (float)M1;
+  block_lines<HB, S>(
+      kPairs * M1, 1, M2, M2, M2, uniform(dft, d2),
+      [&](int l) {
+        int const p = quot(l, i1), n1 = l - p * M1;
+        return At{t.Z + p * pitch + n1 * M2, nullptr};
+      },
+      [&](At const &z, int q, float2 v) { z.p[q] = v; });
+}
+
+template <int HB>
+__global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_fwd_time_g(
+    AgdWin const *__restrict__ wins, int const *__restrict__ blocks, int block0,
+    float const *__restrict__ dft, AgdFftPlan const *__restrict__ plans,
+    float2 const *__restrict__ roots, float const *__restrict__ tapers,
+    float const *__restrict__ tscale, float2 const *__restrict__ U, float *__restrict__ T) {
+  extern __shared__ float2 sm[];
+  int const *const bl = blocks + TB_INTS * (block0 + blockIdx.x);
+  AgdWin const &w = wins[bl[0]];
+  int const t0 = bl[1], nt = min(2 * kPairs, w.ntr - t0);
+  int const tw0 = bl[2], tw1 = bl[3];
+  int const twa = tw0 > 0 ? tw0 - 1 : 0;
+  int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2;
+  int const nconv = w.nconv, ntw = w.ntw, pitch = time_pitch(N);
+  TimeTables t;
+  t.Z = sm;
+  t.TW = t.Z + kPairs * pitch;
+  float *const TP = (float *)(t.TW + N);    // [Wt] time taper
+  float *const CA = TP + Wt;                // [16][half] overlap carry
+  t.pos = (unsigned short *)(CA + 2 * kPairs * half);
+  int const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = 4;
+  time_tables<+1>(t, roots + plans[w.tplan_full].roots_off, N, M1, M2);
+  for (int i = tid; i < Wt; i += 256) TP[i] = tapers[w.tt_off + i];
+  for (int i = tid; i < 2 * kPairs * half; i += 256) CA[i] = 0.f;
+  float *const Tb = T + w.t_off + (int64_t)t0 * nconv;
+  int64_t const tw_step = (int64_t)((w.ntr + 15) / 16) * Ft * kPairs;  // float4
+  float4 const *tile = (float4 const *)(U + w.u_off) + (int64_t)(t0 / 16) * Ft * kPairs;
+  for (int tw = twa; tw < tw1; ++tw) {
+    float4 const *u = tile + tw * tw_step;
+    // Hermitian halves of both traces of a pair into z = x_a + i x_b (DC and
+    // Nyquist imaginary parts ignored); traces beyond the window are zero
+    constexpr int NB = 4;
+    for (int i0 = tid; i0 < Ft * kPairs; i0 += NB * 256) {
+      float4 v[NB];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) v[b] = u[min(i0 + b * 256, Ft * kPairs - 1)];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        int const i = i0 + b * 256;
+        if (i < Ft * kPairs) {
+          int const k = i >> 3, p = i & 7;
+          float2 xa = make_float2(v[b].x, v[b].y), xb = make_float2(v[b].z, v[b].w);
+          if (2 * p >= nt) xa = make_float2(0.f, 0.f);
+          if (2 * p + 1 >= nt) xb = make_float2(0.f, 0.f);
+          if (k == 0 || 2 * k == N) xa.y = xb.y = 0.f;
+          float2 *const z = t.Z + p * pitch;
+          z[k] = make_float2(xa.x - xb.y, xa.y + xb.x);
+          if (k > 0 && 2 * k < N) z[N - k] = make_float2(xa.x + xb.y, xb.x - xa.y);
+        }
+      }
+    }
+    __syncthreads();
+    time_fft<HB, +1>(t, pitch, M1, M2, dft, w.tdft1, w.tdft2);
+    // overlap-add: samples [0, half) complete this window's first half
+    for (int p = wave; p < kPairs; p += nw) {
+      if (2 * p >= nt) break;
+      float const sa = tscale[w.trace0 + t0 + 2 * p];
+      float const sb = tscale[w.trace0 + t0 + min(2 * p + 1, nt - 1)];
+      float2 const *const z = t.Z + p * pitch;
+      float *const ca = CA + 2 * p * half, *const cb = ca + half;
+      float *const ta = Tb + (int64_t)2 * p * nconv + tw * half, *const tb = ta + nconv;
+      for (int s = lane; s < half; s += 64) {
+        float2 const z0 = z[t.pos[s]], z1 = z[t.pos[s + half]];
+        float const w0 = TP[s], w1 = TP[s + half];
+        if (tw >= tw0) {
+          ta[s] = ca[s] + z0.x * sa * w0;
+          if (2 * p + 1 < nt) tb[s] = cb[s] + z0.y * sb * w0;
+        }
+        ca[s] = z1.x * sa * w1;
+        cb[s] = z1.y * sb * w1;
+      }
+    }
+    __syncthreads();
+  }
+  if (tw1 < ntw) return;
+  for (int j = wave; j < nt; j += nw) {
+    float *const tj = Tb + (int64_t)j * nconv;
+    for (int s = lane; s < half; s += 64)
+      if (ntw * half + s < nconv) tj[ntw * half + s] = CA[j * half + s];
+    // zero the capacity beyond the data portion (wavelet input padding)
+    for (int s = (ntw + 1) * half + lane; s < nconv; s += 64) tj[s] = 0.f;
+  }
+}
+
+template <int HB>
+__global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_adj_time_g(
+    AgdWin const *__restrict__ wins, int const *__restrict__ blocks, int block0,
+    float const *__restrict__ dft, AgdFftPlan const *__restrict__ plans,
+    float2 const *__restrict__ roots, float const *__restrict__ tapers,
+    float const *__restrict__ tscale, AgdEntry const *__restrict__ went,
+    float const *__restrict__ rec, float const *__restrict__ Tin, float2 *__restrict__ V,
+    int plain, int const *__restrict__ order) {
+  extern __shared__ float2 sm[];
+  // the launch order of the specialised kernel (neighbouring windows' blocks
+  // of the same traces on one XCD)
+  int const bid = order ? order[block0 + xcd_chunk(blockIdx.x, gridDim.x)] : block0 + blockIdx.x;
+  int const *const bl = blocks + TB_INTS * bid;
+  AgdWin const &w = wins[bl[0]];
+  int const t0 = bl[1], nt = min(2 * kPairs, w.ntr - t0);
+  int const tw0 = bl[2], tw1 = bl[3];
+  int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2;
+  int const nconv = w.nconv, pitch = time_pitch(N);
+  TimeTables t;
+  t.Z = sm;
+  t.TW = t.Z + kPairs * pitch;
+  float *const TP = (float *)(t.TW + N);
+  t.pos = (unsigned short *)(TP + Wt);
+  int const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = 4;
+  time_tables<-1>(t, roots + plans[w.tplan_full].roots_off, N, M1, M2);
+  for (int i = tid; i < Wt; i += 256) TP[i] = plain ? 1.f : tapers[w.tt_off + i];
+  __syncthreads();
+  // one source: the record through the blend entries, or a trace buffer; a
+  // wave takes two pairs of traces, whose entries and scales stay in registers
+  float const *const src = Tin != nullptr ? Tin : rec;
+  constexpr int NP = kPairs / 4;
+  int64_t at[NP][2];
+  int start[NP][2], cnt[NP][2];
+  float sc[NP][2];
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      int const j = 2 * (wave + 4 * i) + q, jc = min(j, nt - 1);
+      AgdEntry const e = went[w.trace0 + t0 + jc];
+      float const ts = tscale[w.trace0 + t0 + jc];
+      at[i][q] = Tin != nullptr ? w.t_off + (int64_t)(t0 + jc) * nconv : e.rec;
+      start[i][q] = Tin != nullptr ? 0 : e.trace_start;
+      cnt[i][q] = j >= nt ? 0 : Tin != nullptr ? nconv : e.n;
+      sc[i][q] = plain ? w.scaler : ts;
+    }
+  // unconditional loads (index clamped into the trace's range), zeroed
+  // outside it, so that they stay in flight together
+  auto sample = [&](int i, int q, int t, bool in) -> float {
+    int const i2 = t - start[i][q];
+    bool const ok = in && (unsigned)i2 < (unsigned)cnt[i][q];
+    float const v = src[at[i][q] + (ok ? i2 : 0)];
+    return ok ? v : 0.f;
+  };
+  float const two = plain ? 1.f : 2.f;
+  int const kmax2 = (N - 1) / 2;
+  float4 *const vt = (float4 *)(V + w.u_off) + (int64_t)(t0 / 16) * Ft * kPairs;
+  int64_t const tw_step = (int64_t)((w.ntr + 15) / 16) * Ft * kPairs;
+  for (int tw = tw0; tw < tw1; ++tw) {
+    constexpr int NB = 2;
+    for (int s0 = lane; s0 < N; s0 += 64 * NB) {
+      float x[NP][NB][2];
+#pragma unroll
+      for (int i = 0; i < NP; ++i)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            int const s = s0 + 64 * b;
+            x[i][b][q] = sample(i, q, tw * half + s, s < Wt);
+          }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        int const s = s0 + 64 * b;
+        float const tp = TP[min(s, Wt - 1)];
+        if (s < N) {
+#pragma unroll
+          for (int i = 0; i < NP; ++i)
+            t.Z[(wave + 4 * i) * pitch + s] =
+                make_float2(x[i][b][0] * sc[i][0] * tp, x[i][b][1] * sc[i][1] * tp);
+        }
+      }
+    }
+    __syncthreads();
+    time_fft<HB, -1>(t, pitch, M1, M2, dft, w.tdft1, w.tdft2);
+    // half spectra of the two real traces of a pair, x2 on the interior bins
+    float4 *const vo = vt + tw * tw_step;
+    for (int i = tid; i < Ft * kPairs; i += 256) {
+      int const k = i >> 3, p = i & 7;
+      float2 const *const z = t.Z + p * pitch;
+      float2 const z1 = z[t.pos[k]], z2 = z[t.pos[k ? N - k : 0]];
+      float const s = (k >= 1 && k <= kmax2) ? 0.5f * two : 0.5f;
+      vo[i] = make_float4(s * (z1.x + z2.x), s * (z1.y - z2.y), s * (z1.y + z2.y),
+                          s * (z2.x - z1.x));
+    }
+    __syncthreads();
+  }
+}
+
+// Instances of the run-time sized kernels by the coefficient pairs HB a line
+// holds in registers (lengths up to 2 HB + 1): the fewer, the more waves
+// share a SIMD. The host picks the smallest that fits a window's lines.
+template <int HB>
+static int launch_spatial_g(AgdDev const *g, AgdClass const &c, float2 *X, float alpha,
+                            float lamb, int mode, int fuse) {
+  static int const lds_ok = allow_lds((void const *)k_spatial_g<HB>);
+  (void)lds_ok;
+  int first;
+  int const n = class_range(g, c, &first);
+  if (n <= 0) return 0;
+  return launch(mode < 0 ? "fwd_spatial" : "adj_spatial", k_spatial_g<HB>, dim3(n),
+                dim3(NTHR), c.lds, g->win, g->tasks, first, g->dft, (float2 const *)g->V, X,
+                (float2 *)g->U, alpha, lamb, (float const *)g->lamb_dev, mode, fuse, g->scalar);
+}
+int spatial_general(AgdDev const *g, AgdClass const &c, float2 *X, float alpha,
+                           float lamb, int mode, int fuse) {
+  switch (c.hb) {
+    case 8: return launch_spatial_g<8>(g, c, X, alpha, lamb, mode, fuse);
+    case 16: return launch_spatial_g<16>(g, c, X, alpha, lamb, mode, fuse);
+    case 24: return launch_spatial_g<24>(g, c, X, alpha, lamb, mode, fuse);
+    case 32: return launch_spatial_g<32>(g, c, X, alpha, lamb, mode, fuse);
+    case 48: return launch_spatial_g<48>(g, c, X, alpha, lamb, mode, fuse);
+    default: return launch_spatial_g<64>(g, c, X, alpha, lamb, mode, fuse);
+  }
+}
+template <int HB>
+static int launch_fwd_time_g(AgdDev const *g, AgdClass const &c, int first, int n) {
+  static int const lds_ok = allow_lds((void const *)k_fwd_time_g<HB>);
+  (void)lds_ok;
+  return launch("fwd_time", k_fwd_time_g<HB>, dim3(n), dim3(NTHR), c.lds, g->win,
+                g->tblocks, first, g->dft, g->plans, (float2 const *)g->roots, g->tapers,
+                g->tscale, (float2 const *)g->U, g->T);
+}
+int fwd_time_general(AgdDev const *g, AgdClass const &c, int first, int n) {
+  switch (c.hb) {
+    case 8: return launch_fwd_time_g<8>(g, c, first, n);
+    case 16: return launch_fwd_time_g<16>(g, c, first, n);
+    case 32: return launch_fwd_time_g<32>(g, c, first, n);
+    default: return launch_fwd_time_g<64>(g, c, first, n);
+  }
+}
+template <int HB>
+static int launch_adj_time_g(AgdDev const *g, AgdClass const &c, int first, int n,
+                             float const *Tin, int plain) {
+  static int const lds_ok = allow_lds((void const *)k_adj_time_g<HB>);
+  (void)lds_ok;
+  return launch("adj_time", k_adj_time_g<HB>, dim3(n), dim3(NTHR), c.lds, g->win,
+                g->tblocks, first, g->dft, g->plans, (float2 const *)g->roots, g->tapers,
+                g->tscale, g->went, (float const *)g->r, Tin, (float2 *)g->V, plain,
+                first == c.begin && n == c.count ? g->tadj : (int const *)nullptr);
+}
+int adj_time_general(AgdDev const *g, AgdClass const &c, int first, int n,
+                            float const *Tin, int plain) {
+  switch (c.hb) {
+    case 8: return launch_adj_time_g<8>(g, c, first, n, Tin, plain);
+    case 16: return launch_adj_time_g<16>(g, c, first, n, Tin, plain);
+    case 32: return launch_adj_time_g<32>(g, c, first, n, Tin, plain);
+    default: return launch_adj_time_g<64>(g, c, first, n, Tin, plain);
+  }
+}
+
+}  // namespace agdgen

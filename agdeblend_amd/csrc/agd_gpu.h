@@ -28,6 +28,7 @@ typedef struct {
   AgdWin const *win;          /* [n_win] */
   AgdFftPlan const *plans;    /* FFT plans */
   float const *roots;         /* complex roots pool (interleaved) */
+  float const *dft;           /* line_dft coefficient pool */
   float const *tapers;        /* time taper pool */
   float const *tscale;        /* per global window trace: scaler * space tapers */
   float const *tconst;        /* per global window trace: space tapers only */

@@ -558,6 +558,7 @@ static void trace_coord(BlendCfg const *c, long shot, int ntimes, int channel,
 typedef struct {
   vec plans; /* AgdFftPlan */
   vec roots; /* float pairs */
+  vec dft;   /* line_dft coefficients (floats) */
 } PlanSet;
 
 static int planset_get(PlanSet *s, int n) {
@@ -584,6 +585,7 @@ static int planset_get(PlanSet *s, int n) {
       rem /= f;
     }
   }
+  np_.dft_off = -1;
   np_.roots_off = (int)(s->roots.n);
   for (f = 0; f < n; f++) {
     float *r = (float *)vec_push(&s->roots);
@@ -598,6 +600,31 @@ static int planset_get(PlanSet *s, int n) {
     *q = np_;
   }
   return (int)(s->plans.n - 1);
+}
+
+/* Offset of line_dft's coefficients of length n (agd_general.h), n > 0: for
+ * q = 1 .. (n - 1) / 2 a row of the pairs cos, sin(2 pi q k / n), k = 1 ..
+ * (n - 1) / 2, padded with zeros to groups of 4. -1 on error. */
+static int dft_get(PlanSet *s, int n) {
+  int const pi = planset_get(s, n);
+  AgdFftPlan *pl;
+  int const h = (n - 1) / 2, row = (h + 3) / 4 * 4;
+  int q, k;
+  if (pi < 0) return -1;
+  pl = (AgdFftPlan *)s->plans.p + pi;
+  if (pl->dft_off >= 0) return pl->dft_off;
+  pl->dft_off = (int)s->dft.n;
+  for (q = 1; q <= h; q++)
+    for (k = 1; k <= row; k++) {
+      double const a = 2.0 * M_PI * (double)((int64_t)q * k % n) / (double)n;
+      float *c = (float *)vec_push(&s->dft), *d;
+      if (c == NULL) return -1;
+      *c = k <= h ? (float)cos(a) : 0.0f;
+      d = (float *)vec_push(&s->dft);
+      if (d == NULL) return -1;
+      *d = k <= h ? (float)sin(a) : 0.0f;
+    }
+  return pl->dft_off;
 }
 
 /* smallest even M >= n whose half has no prime factor above 7 */
@@ -1078,23 +1105,98 @@ static void time_sizes(AgdWin const *W, int *m1, int *m2) {
     }
 }
 
-/* Traces per U / V tile: 16 when both transforms of the window have
- * specialised kernels and the traces form whole tiles, else the whole
- * window (untiled layout of the generic kernels). */
+/* Traces per tile of U / V and per block of the time kernels. The
+ * specialised time kernels serve windows of whole tiles whose spatial
+ * transform is specialised too. */
 #define TIME_TILE 16
-static int window_ug(AgdWin const *W) {
-  int a, b;
-  spatial_key(W, &a, &b);
-  if (!a || W->ntr % TIME_TILE) return W->ntr;
-  time_sizes(W, &a, &b);
-  return a ? TIME_TILE : W->ntr;
+static int tile_traces(AgdWin const *W) {
+  return (W->ntr + TIME_TILE - 1) / TIME_TILE * TIME_TILE;
 }
-
-/* the specialised time kernels serve tiled windows only */
 static void time_key(AgdWin const *W, int *m1, int *m2) {
+  int a, b;
   *m1 = 0;
   *m2 = 0;
-  if (W->ug == TIME_TILE && W->ntr % TIME_TILE == 0) time_sizes(W, m1, m2);
+  spatial_key(W, &a, &b);
+  if (a && W->ntr % TIME_TILE == 0) time_sizes(W, m1, m2);
+}
+
+/* Instances of the run-time sized kernels (agd_general.h): the smallest of
+ * inst (0-terminated) whose lines hold length n, or 0 */
+static int line_instance(int n, int const *inst) {
+  int i;
+  for (i = 0; inst[i]; i++)
+    if (n <= 2 * inst[i] + 1) return inst[i];
+  return 0;
+}
+static int const kSpatialInst[] = {8, 16, 24, 32, 48, 64, 0};
+static int const kTimeInst[] = {8, 16, 32, 64, 0};
+
+/* coefficient pairs of the window's run-time sized spatial kernel: lines up
+ * to 129 and planes within the generic kernel's limit (0: the LDS-resident
+ * generic kernel) */
+static int spatial_lines(AgdWin const *W) {
+  int d, m = 0;
+  if (W->S > AGD_LINES_VALUES || (size_t)2 * W->S * 8 > LDS_BUDGET) return 0;
+  for (d = 0; d < W->nsp; d++)
+    if (W->P[d] > m) m = W->P[d];
+  return line_instance(m, kSpatialInst);
+}
+
+/* dynamic LDS of the run-time sized time kernels (time_g_lds) */
+static size_t time_lines_lds(AgdWin const *W) {
+  size_t const pitch = (size_t)(W->Pt + 3) / 8 * 8 + 4;
+  return 8 * (TIME_TILE / 2 * pitch + (size_t)W->Pt) + 4 * (size_t)W->Wt +
+         4 * (size_t)TIME_TILE * (size_t)W->half + 2 * (size_t)W->Pt + 16;
+}
+
+/* Pt = m1 m2 with the smaller longest factor (an odd one last: the second
+ * phase's lanes are m2 apart in LDS) of the run-time sized time kernels:
+ * even window lengths, factors up to 129, 96 KB of LDS; else 0 0 */
+static void time_lines(AgdWin const *W, int *m1, int *m2) {
+  int a;
+  *m1 = 0;
+  *m2 = 0;
+  if (W->Wt % 2 || time_lines_lds(W) > 96 * 1024) return;
+  for (a = 1; a * a <= W->Pt; a++)
+    if (W->Pt % a == 0) {
+      *m1 = a;
+      *m2 = W->Pt / a;
+    }
+  if (*m2 % 2 == 0 && *m1 % 2 && *m1 > 1) {
+    int const t = *m1;
+    *m1 = *m2;
+    *m2 = t;
+  }
+  if (line_instance(*m1 > *m2 ? *m1 : *m2, kTimeInst) == 0) *m1 = *m2 = 0;
+}
+static int time_instance(AgdWin const *W) {
+  return W->gm2 ? line_instance(W->gm1 > W->gm2 ? W->gm1 : W->gm2, kTimeInst) : 0;
+}
+
+/* Planes per task of the run-time sized spatial kernel: at most
+ * AGD_LINES_VALUES values (a block holds them in registers and LDS, four
+ * blocks to a CU). A stage of l lines costs ceil(l / 64) waves of lines of
+ * P^2 multiply-adds; the task's planes share its barriers and latencies
+ * (counted as 2000 multiply-adds a lane). The cheapest per plane. */
+static int lines_nk(AgdWin const *W) {
+  int nk_max = AGD_LINES_VALUES / W->S, nk, best = 1, d, e;
+  double best_c = -1.0;
+  if (nk_max > W->Ft) nk_max = W->Ft;
+  for (nk = 1; nk <= nk_max; nk++) {
+    double c = 2000.0;
+    for (d = 0; d < W->nsp; d++) {
+      /* lines of dim d: the dims before it cropped, the dims after it padded */
+      int l = nk;
+      for (e = 0; e < W->nsp; e++)
+        if (e != d) l *= e < d ? W->W[e] : W->P[e];
+      c += ((l + 63) / 64) * (double)W->P[d] * W->P[d];
+    }
+    if (best_c < 0.0 || c / nk < best_c) {
+      best_c = c / nk;
+      best = nk;
+    }
+  }
+  return best;
 }
 
 /* Spatial tasks (chunks of time-frequency planes) and time blocks (runs of
@@ -1129,11 +1231,15 @@ static int spatial_tasks(AgdProblem *p, AgdClass *cls, int ncls, int const *nk_r
     cl->begin = (int)tasks->n;
     for (w = 0; w < p->n_win; w++) {
       AgdWin const *W = &p->win[w];
-      int a, b, nk, tw, k0;
+      int a, b, tm, tn, nk, tw, k0;
       wpos[w] = (int)tasks->n - cl->begin;
       spatial_key(W, &a, &b);
-      if (a != cl->p0 || b != cl->p1 || (a && (W->ug != W->ntr) != cl->tb)) continue;
-      if (a) {
+      time_key(W, &tm, &tn);
+      if (a != cl->p0 || b != cl->p1 || (a ? (tm > 0) != cl->tb : spatial_lines(W) != cl->hb))
+        continue;
+      if (cl->hb) {
+        nk = lines_nk(W);
+      } else if (a) {
         nk = (nk_req && nk_req[c] > 0) ? nk_req[c] : default_nk(a, b);
       } else {
         nk = (int)(LDS_BUDGET / (2 * (size_t)W->S * 8));
@@ -1155,6 +1261,10 @@ static int spatial_tasks(AgdProblem *p, AgdClass *cls, int ncls, int const *nk_r
       }
       if (a) {
         size_t const l = (size_t)nk * spec_len(a) * (b + 1) * 8;
+        if (l > cl->lds) cl->lds = l;
+      } else if (cl->hb) {
+        int const last = W->P[W->nsp - 1];
+        size_t const l = (size_t)nk * (W->S / last) * (last | 1) * 8;
         if (l > cl->lds) cl->lds = l;
       } else if ((size_t)2 * nk * W->S * 8 > *lds_sp) {
         *lds_sp = (size_t)2 * nk * W->S * 8;
@@ -1229,31 +1339,36 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
   vec_init(&tc, sizeof(AgdClass));
   for (w = 0; w < p->n_win; w++) {
     AgdWin const *W = &p->win[w];
-    int a, b, found = 0;
+    int a, b, tm, tn, hb, found = 0;
     AgdClass *cl = (AgdClass *)sc.p;
-    int const tiled = (W->ug != W->ntr);
     spatial_key(W, &a, &b);
+    time_key(W, &tm, &tn);
+    hb = a ? 0 : spatial_lines(W);
     for (c = 0; c < (int)sc.n; c++)
-      if (cl[c].p0 == a && cl[c].p1 == b && (!a || cl[c].tb == tiled)) found = 1;
+      if (cl[c].p0 == a && cl[c].p1 == b && (a ? cl[c].tb == (tm > 0) : cl[c].hb == hb)) found = 1;
     if (!found) {
       AgdClass *n = (AgdClass *)vec_push(&sc);
       if (n == NULL) return 1;
       memset(n, 0, sizeof(*n));
       n->p0 = a;
       n->p1 = b;
-      n->tb = a ? tiled : 0; /* spatial classes: U / V tiled by TIME_TILE traces */
+      n->tb = a ? tm > 0 : 0;
+      n->hb = hb;
     }
-    time_key(W, &a, &b);
+    a = tm;
+    b = tn;
+    hb = a ? 0 : time_instance(W);
     found = 0;
     cl = (AgdClass *)tc.p;
     for (c = 0; c < (int)tc.n; c++)
-      if (cl[c].p0 == a && cl[c].p1 == b) found = 1;
+      if (cl[c].p0 == a && cl[c].p1 == b && cl[c].hb == hb) found = 1;
     if (!found) {
       AgdClass *n = (AgdClass *)vec_push(&tc);
       if (n == NULL) return 1;
       memset(n, 0, sizeof(*n));
       n->p0 = a;
       n->p1 = b;
+      n->hb = hb;
     }
   }
   if (spatial_tasks(p, (AgdClass *)sc.p, (int)sc.n, NULL, tasks, &lds_sp)) return 1;
@@ -1274,8 +1389,10 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
         int a, b;
         size_t l;
         time_key(W, &a, &b);
-        if (a != cl->p0 || b != cl->p1) continue;
-        if (a) {
+        if (a != cl->p0 || b != cl->p1 || (!a && time_instance(W) != cl->hb)) continue;
+        if (cl->hb) {
+          l = time_lines_lds(W);
+        } else if (a) {
           /* the forward's tile, work buffer and roots (the larger of the
            * two kernels; the launcher passes each its own size) */
           size_t const M = (size_t)a * b;
@@ -1287,17 +1404,17 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
         if (l > need) need = l;
       }
       cl->lds = need;
-      if (cl->p0 || need <= (size_t)LDS_BUDGET || tb == 1) break;
+      if (cl->p0 || cl->hb || need <= (size_t)LDS_BUDGET || tb == 1) break;
     }
     cl->tb = tb;
-    if (!cl->p0) lds_t = cl->lds > lds_t ? cl->lds : lds_t;
+    if (!cl->p0 && !cl->hb) lds_t = cl->lds > lds_t ? cl->lds : lds_t;
     cl->begin = (int)tblocks->n;
     for (w = 0; w < p->n_win; w++) {
       AgdWin const *W = &p->win[w];
       int a, b, t0, q, parts;
       wpos[w] = (int)tblocks->n - cl->begin;
       time_key(W, &a, &b);
-      if (a != cl->p0 || b != cl->p1) continue;
+      if (a != cl->p0 || b != cl->p1 || (!a && time_instance(W) != cl->hb)) continue;
       /* the specialised kernels' blocks split the window's time windows
        * into nearly equal runs of at most tw_run (0: one run) */
       parts = (a && tw_run > 0) ? (W->ntw + tw_run - 1) / tw_run : 1;
@@ -1344,6 +1461,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
   vec wsrc, wspec;
   vec_init(&ps.plans, sizeof(AgdFftPlan));
   vec_init(&ps.roots, 2 * sizeof(float));
+  vec_init(&ps.dft, sizeof(float));
   vec_init(&wsrc, sizeof(WavSrc));
   vec_init(&wspec, 2 * sizeof(float));
   if (!host_only && agdg_init()) return NULL;
@@ -1478,12 +1596,27 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
       if (W->tplan < 0 || W->tplan_full < 0) goto err;
       W->wplan = -1;
       W->wplan_full = -1;
-      W->ug = window_ug(W);
+      {
+        /* coefficients of the run-time sized kernels */
+        int m1, m2;
+        spatial_key(W, &m1, &m2);
+        for (d = 0; d < nsp; d++) W->sdft[d] = 0;
+        if (m1 == 0 && spatial_lines(W))
+          for (d = 0; d < nsp; d++)
+            if ((W->sdft[d] = dft_get(&ps, W->P[d])) < 0) goto err;
+        time_key(W, &m1, &m2);
+        if (m1 == 0) {
+          time_lines(W, &W->gm1, &W->gm2);
+          if (W->gm2 && ((W->tdft1 = dft_get(&ps, W->gm1)) < 0 ||
+                         (W->tdft2 = dft_get(&ps, W->gm2)) < 0))
+            goto err;
+        }
+      }
       W->x_off = xo;
       W->u_off = uo;
       W->t_off = to;
       xo += (int64_t)W->ntw * W->Ft * W->S;
-      uo += (int64_t)W->ntw * W->Ft * W->ntr;
+      uo += (int64_t)W->ntw * W->Ft * tile_traces(W);
       to += (int64_t)W->ntr * W->nconv;
       /* time taper */
       W->tt_off = (int)tapers.n;
@@ -1610,6 +1743,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
     p->dev.win = (AgdWin const *)dev_upload(p, p->win, (size_t)p->n_win * sizeof(AgdWin));
     p->dev.plans = (AgdFftPlan const *)dev_upload(p, ps.plans.p, ps.plans.n * sizeof(AgdFftPlan));
     p->dev.roots = (float const *)dev_upload(p, ps.roots.p, ps.roots.n * 2 * sizeof(float));
+    p->dev.dft = (float const *)dev_upload(p, ps.dft.p, ps.dft.n * sizeof(float));
     p->dev.tapers = (float const *)dev_upload(p, tapers.p, tapers.n * sizeof(float));
     p->dev.tscale = (float const *)dev_upload(p, tscale, (size_t)p->n_wtr * sizeof(float));
     p->dev.tconst = (float const *)dev_upload(p, tconst, (size_t)p->n_wtr * sizeof(float));
@@ -1641,7 +1775,8 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
       p->n_chunk = 0;
       p->chunk[0] = 0;
       for (w = 0; w < p->n_win; w++) {
-        double const b = 2.0 * 8.0 * (double)p->win[w].ntw * p->win[w].Ft * p->win[w].ntr;
+        double const b =
+            2.0 * 8.0 * (double)p->win[w].ntw * p->win[w].Ft * tile_traces(&p->win[w]);
         if (cap > 0.0 && acc > 0.0 && acc + b > cap) {
           p->chunk[++p->n_chunk] = w;
           acc = 0.0;
@@ -1707,7 +1842,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
     vec_free(&tapers);
     vec_free(&tasks);
     vec_free(&tblocks);
-    if (!p->dev.win || !p->dev.plans || !p->dev.roots || !p->dev.tapers ||
+    if (!p->dev.win || !p->dev.plans || !p->dev.roots || !p->dev.dft || !p->dev.tapers ||
         !p->dev.tscale || !p->dev.tconst || !p->dev.went || !p->dev.trace_win ||
         !p->dev.tasks || !p->dev.tblocks || !p->dev.tadj || !p->dev.wsrc_off || !p->dev.X ||
         !p->dev.U || !p->dev.V || !p->dev.T || !p->dev.T2 || !p->dev.d || !p->dev.r ||
@@ -1861,6 +1996,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
   free(all);
   vec_free(&ps.plans);
   vec_free(&ps.roots);
+  vec_free(&ps.dft);
   vec_free(&wsrc);
   vec_free(&wspec);
   return p;
@@ -1874,6 +2010,7 @@ err:
   free(all);
   vec_free(&ps.plans);
   vec_free(&ps.roots);
+  vec_free(&ps.dft);
   vec_free(&wsrc);
   vec_free(&wspec);
   agdx_destroy(p);

@@ -35,9 +35,9 @@
 #include <vector>
 
 #include "agd_fft.h"
+#include "agd_general.h"
 #include "agd_gpu.h"
-
-#define NTHR 256
+#include "agd_launch.h"
 
 static hipStream_t g_stream = nullptr;
 static int g_timing = 0;
@@ -75,20 +75,21 @@ static void flush_timing() {
   g_pending.clear();
 }
 
-// Launch helper: optional per-kernel event timing on the library stream.
-template <typename K, typename... Args>
-static int launch(char const *name, K kernel, dim3 grid, dim3 block, size_t lds,
-                  Args... args) {
-  hipEvent_t a = nullptr, b = nullptr;
-  if (grid.x == 0 || grid.y == 0 || grid.z == 0) return 0;
+// the library stream's launches (agd_launch.h): optional per-kernel event
+// timing
+hipStream_t agd_launch_begin(hipEvent_t *a) {
+  *a = nullptr;
   if (g_timing) {
-    (void)hipEventCreate(&a);
-    (void)hipEventCreate(&b);
-    (void)hipEventRecord(a, g_stream);
+    (void)hipEventCreate(a);
+    (void)hipEventRecord(*a, g_stream);
   }
-  hipLaunchKernelGGL(kernel, grid, block, lds, g_stream, args...);
+  return g_stream;
+}
+int agd_launch_end(char const *name, hipEvent_t a) {
   if (hip_check(hipGetLastError(), name)) return 1;
-  if (g_timing) {
+  if (a != nullptr) {
+    hipEvent_t b = nullptr;
+    (void)hipEventCreate(&b);
     (void)hipEventRecord(b, g_stream);
     g_pending.push_back({name, a, b});
     if (g_pending.size() > 4096) flush_timing();
@@ -115,13 +116,12 @@ __device__ __forceinline__ float2 rootf(float2 const *roots, int n, int e, int s
   return w;
 }
 
-// Blocks go to the eight XCDs in turn (block b runs on XCD b mod 8, each
-// XCD with its own L2). This bijection of [0, n) gives XCD x a contiguous
-// run of the n work items instead.
-__device__ __forceinline__ int xcd_chunk(int b, int n) {
-  int const q = n >> 3, r = n & 7, x = b & 7, i = b >> 3;
-  return x * q + min(x, r) + i;
+// element of trace tr, plane k of one time window's tiles of U / V
+// ([tile of 16 traces][Ft][16]); ntr16: complex values per plane and window
+__device__ __forceinline__ int64_t tile_at(int tr, int k, int Ft) {
+  return ((int64_t)(tr >> 4) * Ft + k) * 16 + (tr & 15);
 }
+__device__ __forceinline__ int tile_plane(int ntr) { return (ntr + 15) & ~15; }
 
 // ---------------------------------------------------------------------------
 // Line geometries for LDS-resident batched FFTs
@@ -268,7 +268,8 @@ __device__ float2 *fft_lines(float2 *a, float2 *b, AgdFftPlan const &p,
 }
 
 // ---------------------------------------------------------------------------
-// Forward spatial transform: X[w][tw][k][S] -> U[w][tw][k][ntr]
+// Forward spatial transform: X[w][tw][k][S] -> the tiles of U. The generic
+// kernels serve lines too long for the run-time sized ones (agd_general.h).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(NTHR) void k_fwd_spatial(
     AgdWin const *__restrict__ wins, AgdTask const *__restrict__ tasks, int task0,
@@ -318,7 +319,8 @@ __global__ __launch_bounds__(NTHR) void k_fwd_spatial(
       r /= w.W[e];
       off += c * g.str[e];
     }
-    U[w.u_off + ((int64_t)t.tw * w.Ft + t.k0 + k) * ntr + tr] = A[k * S + off];
+    U[w.u_off + (int64_t)t.tw * w.Ft * tile_plane(ntr) + tile_at(tr, t.k0 + k, w.Ft)] =
+        A[k * S + off];
   }
 }
 
@@ -351,11 +353,11 @@ __global__ __launch_bounds__(NTHR) void k_fwd_time(
   for (int i = threadIdx.x; i < tb * Wt; i += blockDim.x) acc[i] = 0.f;
   LinesContig lc{M};
   for (int tw = 0; tw < w.ntw; ++tw) {
-    float2 const *u = U + w.u_off + (int64_t)tw * Ft * w.ntr + t0;
+    float2 const *u = U + w.u_off + (int64_t)tw * Ft * tile_plane(w.ntr);
     for (int i = threadIdx.x; i < Ft * tb; i += blockDim.x) {
       int const k = i / tb;
       int const j = i - k * tb;
-      H[j * Ft + k] = j < nt ? u[(int64_t)k * w.ntr + j] : make_float2(0.f, 0.f);
+      H[j * Ft + k] = j < nt ? u[tile_at(t0 + j, k, Ft)] : make_float2(0.f, 0.f);
     }
     __syncthreads();
     if (even) {
@@ -613,7 +615,7 @@ __global__ __launch_bounds__(NTHR) void k_adj_time(
         X.x *= 2.f;
         X.y *= 2.f;
       }
-      V[w.u_off + ((int64_t)tw * Ft + k) * w.ntr + t0 + j] = X;
+      V[w.u_off + (int64_t)tw * Ft * tile_plane(w.ntr) + tile_at(t0 + j, k, Ft)] = X;
     }
     (void)out;
     __syncthreads();
@@ -663,7 +665,8 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial(
       r /= w.W[e];
       off += c * g.str[e];
     }
-    A[k * S + off] = V[w.u_off + ((int64_t)t.tw * w.Ft + t.k0 + k) * ntr + tr];
+    A[k * S + off] =
+        V[w.u_off + (int64_t)t.tw * w.Ft * tile_plane(ntr) + tile_at(tr, t.k0 + k, w.Ft)];
   }
   __syncthreads();
   for (int e = 0; e < nsp; ++e) g.ext[e] = w.W[e];
@@ -1282,20 +1285,19 @@ __device__ __forceinline__ void rows_fft(float2 *sm, int nk) {
   }
 }
 
-// LDS rows of the nk planes <-> the window traces of the planes in U / V.
-// Per time window U holds [ntr / ug][Ft][ug] (ug = 16: tiles of 16 traces
-// for the specialised time kernels; ug = ntr: [Ft][ntr]); the element
-// order below walks each tile's nk planes contiguously. Utw points at the
-// task's time window, k0 is its first plane.
-template <int P0, int P1, bool TILED, bool TO_LDS>
+// LDS rows of the nk planes <-> the window traces of the planes in U / V
+// ([tile of 16 traces][Ft][16] per time window); the element order below
+// walks each tile's nk planes contiguously. Utw points at the task's time
+// window, k0 is its first plane.
+template <int P0, int P1, bool TO_LDS>
 __device__ __forceinline__ void planes_copy(float2 *sm, float2 *Utw, int k0, int Ft, int nk) {
   constexpr int LD = P1 + 1;
   constexpr int W0 = win_len<P0>();
   constexpr int W1 = win_len<P1>();
-  constexpr int ug = TILED ? TG : W0 * W1;
+  constexpr int NTR = W0 * W1, NTP = (NTR + TG - 1) / TG * TG;  // padded last tile
   constexpr int NB = 8;  // loads issued together per thread
-  int const span = nk * ug;
-  int const total = nk * W0 * W1;
+  int const span = nk * TG;
+  int const total = nk * NTP;
   for (int base = 0; base < total; base += NB * NTHR) {
     float2 v[NB];
     int lp[NB];
@@ -1304,25 +1306,27 @@ __device__ __forceinline__ void planes_copy(float2 *sm, float2 *Utw, int k0, int
       int const i = min(base + (int)threadIdx.x + b * NTHR, total - 1);
       int const g = i / span;
       int const rem = i - g * span;
-      int const k = rem / ug;
-      int const tr = g * ug + (rem - k * ug);
+      int const k = rem / TG;
+      int const tr = g * TG + (rem - k * TG);
       int const row = tr / W1;
       lp[b] = (k * W0 + row) * LD + (tr - row * W1);
-      float2 *u = Utw + ((int64_t)g * Ft + k0) * ug + rem;
+      if (NTR < NTP && tr >= NTR) lp[b] = -1;
+      float2 *u = Utw + ((int64_t)g * Ft + k0) * TG + rem;
       if (TO_LDS)
         v[b] = *u;
-      else if (base + (int)threadIdx.x + b * NTHR < total)
+      else if (base + (int)threadIdx.x + b * NTHR < total && (NTR == NTP || lp[b] >= 0))
         *u = sm[lp[b]];
     }
     if (TO_LDS) {
 #pragma unroll
       for (int b = 0; b < NB; ++b)
-        if (base + (int)threadIdx.x + b * NTHR < total) sm[lp[b]] = v[b];
+        if (base + (int)threadIdx.x + b * NTHR < total && (NTR == NTP || lp[b] >= 0))
+          sm[lp[b]] = v[b];
     }
   }
 }
 
-template <int P0, int P1, bool TILED>
+template <int P0, int P1>
 __global__ __launch_bounds__(NTHR) void k_fwd_spatial_t(
     AgdWin const *__restrict__ wins, AgdTask const *__restrict__ tasks, int task0,
     float2 const *__restrict__ X, float2 *__restrict__ U) {
@@ -1348,8 +1352,8 @@ __global__ __launch_bounds__(NTHR) void k_fwd_spatial_t(
   __syncthreads();
   rows_fft<P0, P1, +1, P1, W1>(sm, nk);
   __syncthreads();
-  planes_copy<P0, P1, TILED, false>(sm, U + w.u_off + (int64_t)t.tw * w.Ft * (W0 * W1), t.k0,
-                                    w.Ft, nk);
+  planes_copy<P0, P1, false>(sm, U + w.u_off + (int64_t)t.tw * w.Ft * tile_plane(W0 * W1),
+                             t.k0, w.Ft, nk);
 }
 
 // Adjoint spatial transform of V and the model update, by MODE:
@@ -1361,7 +1365,7 @@ __global__ __launch_bounds__(NTHR) void k_fwd_spatial_t(
 //      start whose model is written afterwards)
 // With FUSE (modes 0 and 3) the new model's forward spatial transform, the
 // next forward's first stage, is written to U.
-template <int P0, int P1, bool TILED, int MODE, bool FUSE>
+template <int P0, int P1, int MODE, bool FUSE>
 __global__ __launch_bounds__(NTHR) void k_adj_spatial_t(
     AgdWin const *__restrict__ wins, AgdTask const *__restrict__ tasks, int task0,
     float2 const *__restrict__ V, float2 *__restrict__ X, float2 *__restrict__ U,
@@ -1376,8 +1380,8 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial_t(
   AgdTask const t = tasks[task0 + blockIdx.x];
   AgdWin const &w = wins[t.win];
   int const nk = t.nk;
-  int64_t const uoff = w.u_off + (int64_t)t.tw * w.Ft * (W0 * W1);
-  planes_copy<P0, P1, TILED, true>(sm, const_cast<float2 *>(V) + uoff, t.k0, w.Ft, nk);
+  int64_t const uoff = w.u_off + (int64_t)t.tw * w.Ft * tile_plane(W0 * W1);
+  planes_copy<P0, P1, true>(sm, const_cast<float2 *>(V) + uoff, t.k0, w.Ft, nk);
   __syncthreads();
   rows_fft<P0, P1, -1, W1, P1>(sm, nk);
   __syncthreads();
@@ -1437,7 +1441,7 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial_t(
     __syncthreads();
     rows_fft<P0, P1, +1, P1, W1>(sm, nk);
     __syncthreads();
-    planes_copy<P0, P1, TILED, false>(sm, U + uoff, t.k0, w.Ft, nk);
+    planes_copy<P0, P1, false>(sm, U + uoff, t.k0, w.Ft, nk);
   }
 }
 
@@ -2240,48 +2244,17 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial_x3(
   X(5, 8) X(8, 5) X(4, 10) X(10, 8) X(8, 10) X(16, 5) X(10, 16) X(16, 10) X(20, 8) \
   X(8, 20) X(20, 16) X(16, 20) X(32, 10) X(10, 32)
 
-// units of class c within the launch's window range: [*first, *first + n)
-static inline int class_range(AgdDev const *g, AgdClass const &c, int *first) {
-  int const a = c.wpos[g->w0], b = c.wpos[g->w1];
-  *first = c.begin + a;
-  return b - a;
-}
-
-// the specialised kernels may use up to the CU's 160 KB of LDS: set once per
-// kernel instance, on its first launch
-static int allow_lds(void const *f) {
-  (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  (void)hipGetLastError();
-  return 1;
-}
-
-template <int P0, int P1, bool TILED, int MODE, bool FUSE>
+template <int P0, int P1, int MODE, bool FUSE>
 static int launch_adj_spatial(AgdDev const *g, AgdClass const &c, float alpha, float lamb) {
-  static int const lds_ok = allow_lds((void const *)k_adj_spatial_t<P0, P1, TILED, MODE, FUSE>);
+  static int const lds_ok = allow_lds((void const *)k_adj_spatial_t<P0, P1, MODE, FUSE>);
   (void)lds_ok;
   int first;
   int const n = class_range(g, c, &first);
   if (n <= 0) return 0;
-  return launch("adj_spatial", k_adj_spatial_t<P0, P1, TILED, MODE, FUSE>, dim3(n),
+  return launch("adj_spatial", k_adj_spatial_t<P0, P1, MODE, FUSE>, dim3(n),
                 dim3(NTHR), c.lds, g->win, g->tasks, first, (float2 const *)g->V,
                 (float2 *)g->X, (float2 *)g->U, alpha, lamb, (float const *)g->lamb_dev,
                 g->scalar);
-}
-
-template <int P0, int P1, bool TILED>
-static int adj_spatial_layout(AgdDev const *g, AgdClass const &c, float alpha, float lamb,
-                              int mode, int fuse) {
-  switch (mode) {
-    case 0:
-      return fuse ? launch_adj_spatial<P0, P1, TILED, 0, true>(g, c, alpha, lamb)
-                  : launch_adj_spatial<P0, P1, TILED, 0, false>(g, c, alpha, lamb);
-    case 1: return launch_adj_spatial<P0, P1, TILED, 1, false>(g, c, alpha, lamb);
-    case 2: return launch_adj_spatial<P0, P1, TILED, 2, false>(g, c, alpha, lamb);
-    case 4: return launch_adj_spatial<P0, P1, TILED, 4, false>(g, c, alpha, lamb);
-    default:
-      return fuse ? launch_adj_spatial<P0, P1, TILED, 3, true>(g, c, alpha, lamb)
-                  : launch_adj_spatial<P0, P1, TILED, 3, false>(g, c, alpha, lamb);
-  }
 }
 
 template <int P0, int P1>
@@ -2291,25 +2264,28 @@ static int adj_spatial_sized(AgdDev const *g, AgdClass const &c, float alpha, fl
     fprintf(stderr, "ERROR: fused update requested for mode %d\n", mode);
     return 1;
   }
-  return c.tb ? adj_spatial_layout<P0, P1, true>(g, c, alpha, lamb, mode, fuse)
-              : adj_spatial_layout<P0, P1, false>(g, c, alpha, lamb, mode, fuse);
-}
-
-template <int P0, int P1, bool TILED>
-static int launch_fwd_spatial(AgdDev const *g, AgdClass const &c, float const *X) {
-  static int const lds_ok = allow_lds((void const *)k_fwd_spatial_t<P0, P1, TILED>);
-  (void)lds_ok;
-  int first;
-  int const n = class_range(g, c, &first);
-  if (n <= 0) return 0;
-  return launch("fwd_spatial", k_fwd_spatial_t<P0, P1, TILED>, dim3(n), dim3(NTHR), c.lds,
-                g->win, g->tasks, first, (float2 const *)X, (float2 *)g->U);
+  switch (mode) {
+    case 0:
+      return fuse ? launch_adj_spatial<P0, P1, 0, true>(g, c, alpha, lamb)
+                  : launch_adj_spatial<P0, P1, 0, false>(g, c, alpha, lamb);
+    case 1: return launch_adj_spatial<P0, P1, 1, false>(g, c, alpha, lamb);
+    case 2: return launch_adj_spatial<P0, P1, 2, false>(g, c, alpha, lamb);
+    case 4: return launch_adj_spatial<P0, P1, 4, false>(g, c, alpha, lamb);
+    default:
+      return fuse ? launch_adj_spatial<P0, P1, 3, true>(g, c, alpha, lamb)
+                  : launch_adj_spatial<P0, P1, 3, false>(g, c, alpha, lamb);
+  }
 }
 
 template <int P0, int P1>
 static int fwd_spatial_sized(AgdDev const *g, AgdClass const &c, float const *X) {
-  return c.tb ? launch_fwd_spatial<P0, P1, true>(g, c, X)
-              : launch_fwd_spatial<P0, P1, false>(g, c, X);
+  static int const lds_ok = allow_lds((void const *)k_fwd_spatial_t<P0, P1>);
+  (void)lds_ok;
+  int first;
+  int const n = class_range(g, c, &first);
+  if (n <= 0) return 0;
+  return launch("fwd_spatial", k_fwd_spatial_t<P0, P1>, dim3(n), dim3(NTHR), c.lds,
+                g->win, g->tasks, first, (float2 const *)X, (float2 *)g->U);
 }
 
 // ---------------------------------------------------------------------------
@@ -2442,12 +2418,12 @@ void *agdg_stream(void) { return (void *)g_stream; }
 int agdg_can_fuse(AgdDev const *g) {
   if (g->precision != 0) return 0;  // the split-precision transforms are not fused
   for (int c = 0; c < g->n_sclass; ++c)
-    if (g->sclass[c].p0 == 0) return 0;
+    if (g->sclass[c].p0 == 0 && g->sclass[c].hb == 0) return 0;
   return 1;
 }
 
 // classes served by the split-precision transforms: square P in {20, 40},
-// tiled U / V
+// time transform specialised too (c.tb)
 static inline int x3_class(AgdDev const *g, AgdClass const &c) {
   return g->precision == 1 && c.tb && c.p0 == c.p1 && (c.p0 == 20 || c.p0 == 40);
 }
@@ -2485,6 +2461,10 @@ int agdg_fwd_spatial(AgdDev const *g, float const *X) {
     }
     SPATIAL_SIZES(FWD_CASE)
 #undef FWD_CASE
+    if (!done && c.hb) {
+      if (agdgen::spatial_general(g, c, (float2 *)X, 0.f, 0.f, -1, 0)) return 1;
+      done = true;
+    }
     int first;
     int const n = class_range(g, c, &first);
     if (!done && n > 0 &&
@@ -2520,6 +2500,10 @@ int agdg_fwd_time(AgdDev const *g) {
     }
     TIME_SIZES(FT_CASE)
 #undef FT_CASE
+    if (!done && c.hb) {
+      if (n > 0 && agdgen::fwd_time_general(g, c, first, n)) return 1;
+      done = true;
+    }
     if (!done && n > 0 &&
         launch("fwd_time", k_fwd_time, dim3(n), dim3(NTHR), g->lds_time, g->win,
                g->tblocks, first, c.tb, g->plans, (float2 const *)g->roots, g->tapers,
@@ -2568,6 +2552,10 @@ int agdg_adj_time(AgdDev const *g, float const *Tin, int plain) {
     }
     TIME_SIZES(AT_CASE)
 #undef AT_CASE
+    if (!done && c.hb) {
+      if (n > 0 && agdgen::adj_time_general(g, c, first, n, Tin, plain)) return 1;
+      done = true;
+    }
     if (!done && n > 0 &&
         launch("adj_time", k_adj_time, dim3(n), dim3(NTHR), g->lds_time, g->win,
                g->tblocks, first, c.tb, g->plans, (float2 const *)g->roots, g->tapers,
@@ -2625,6 +2613,10 @@ int agdg_adj_spatial(AgdDev const *g, float alpha, float lamb, int mode, int fus
     }
     SPATIAL_SIZES(AS_CASE)
 #undef AS_CASE
+    if (!done && c.hb) {
+      if (agdgen::spatial_general(g, c, (float2 *)g->X, alpha, lamb, mode, fuse)) return 1;
+      done = true;
+    }
     if (!done) {
       if (fuse) {
         fprintf(stderr, "ERROR: fused update requested for a generic window size\n");

@@ -1,0 +1,46 @@
+// Launches on the library stream, shared by the files that hold its kernels.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "agd_gpu.h"
+
+#define NTHR 256
+
+// the library stream; *a: the start event when kernels are timed, else null
+hipStream_t agd_launch_begin(hipEvent_t *a);
+// checks the launch and, when timed, keeps the pair of events under name
+int agd_launch_end(char const *name, hipEvent_t a);
+
+template <typename K, typename... Args>
+static int launch(char const *name, K kernel, dim3 grid, dim3 block, size_t lds,
+                  Args... args) {
+  hipEvent_t a;
+  if (grid.x == 0 || grid.y == 0 || grid.z == 0) return 0;
+  hipStream_t const s = agd_launch_begin(&a);
+  hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
+  return agd_launch_end(name, a);
+}
+
+// Blocks go to the eight XCDs in turn (block b runs on XCD b mod 8, each
+// XCD with its own L2). This bijection of [0, n) gives XCD x a contiguous
+// run of the n work items instead.
+__device__ __forceinline__ int xcd_chunk(int b, int n) {
+  int const q = n >> 3, r = n & 7, x = b & 7, i = b >> 3;
+  return x * q + min(x, r) + i;
+}
+
+// units of class c within the launch's window range: [*first, *first + n)
+static inline int class_range(AgdDev const *g, AgdClass const &c, int *first) {
+  int const a = c.wpos[g->w0], b = c.wpos[g->w1];
+  *first = c.begin + a;
+  return b - a;
+}
+
+// the specialised kernels may use up to the CU's 160 KB of LDS: set once per
+// kernel instance, on its first launch
+static int allow_lds(void const *f) {
+  (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  (void)hipGetLastError();
+  return 1;
+}

@@ -8,12 +8,11 @@
  *             spatial coefficients contiguously, row-major, last space dim
  *             fastest). Mathematically the same coefficients as the
  *             reference's [ntw][P_space...][Ft] (fk.c:256-262), transposed.
- *   inter U   complex float, per window [ntw][ntr/ug][Ft][ug]: spatial
- *             transform of X cropped to the window's traces (forward), or
- *             time transform of the traces (adjoint); ntr = prod(W_space).
- *             ug = 16 (tiles of 16 traces, one contiguous [Ft][16] block per
- *             time window) for windows served by the specialised kernels,
- *             else ug = ntr ([ntw][Ft][ntr]).
+ *   inter U   complex float, per window [ntw][ntr/16][Ft][16] (tiles of 16
+ *             traces, one contiguous block per time window; the last tile of
+ *             a window is padded): spatial transform of X cropped to the
+ *             window's traces (forward), or time transform of the traces
+ *             (adjoint); ntr = prod(W_space).
  *   traces T  float, per window [ntr][nconv] (the reference's temp_1 trace
  *             buffer, fk.c:330-331).
  *   record    float, all (channel, interval) continuous records concatenated
@@ -26,6 +25,8 @@
 
 #define AGD_MAXSP 4      /* AGD_MAX_N_COORDS */
 #define AGD_MAXSTAGE 24  /* FFT stages per plan */
+/* model values of one task of the run-time sized spatial kernel at most */
+#define AGD_LINES_VALUES 4096
 /* half lengths Mr / 2 of the wavelet convolution with a compile-time kernel
  * (k_wavelet_t); the host prefers them to the smallest 7-smooth length when
  * one is at most 25% longer */
@@ -38,7 +39,7 @@ typedef struct {
   int nstage;
   int radix[AGD_MAXSTAGE];
   int roots_off; /* complex offset in the roots pool */
-  int pad;
+  int dft_off;   /* float offset of line_dft's coefficients in the dft pool */
 } AgdFftPlan;
 
 typedef struct {
@@ -57,9 +58,12 @@ typedef struct {
   int wM;                /* wavelet convolution length M */
   int trace0;            /* first global window-trace index */
   int patch;
-  int ug;                /* trace group of the U / V layout (16 or ntr) */
   float scaler;          /* 1 / sqrt(prod P) (fk.c:157-163) */
-  int spare;
+  /* run-time sized kernels (agd_general.h): coefficient offsets per space
+   * dim, Pt = gm1 * gm2 (gm2 0: none) and its two factors' offsets */
+  int sdft[AGD_MAXSP];
+  int gm1, gm2;
+  int tdft1, tdft2;
   int64_t x_off;         /* model offset (complex) */
   int64_t u_off;         /* intermediate offset (complex) */
   int64_t t_off;         /* trace buffer offset (float) */
@@ -75,15 +79,18 @@ typedef struct {
   int n;
 } AgdEntry;
 
-/* A contiguous range of spatial tasks (or time blocks) whose windows share
- * the transform sizes, so one specialised kernel instance serves them.
- * p0 == 0: no specialised kernel, the generic one runs the range. */
+/* A contiguous range of spatial tasks (or time blocks) served by one kernel
+ * instance: p0 > 0 windows of one transform size with a specialised kernel;
+ * p0 == 0 and hb > 0 any sizes whose lines fit the run-time sized kernels'
+ * registers; else the LDS-resident generic kernel. */
 typedef struct {
   int p0, p1;   /* spatial: padded sizes (p0 = 1 when one space dim);
                    time: p0 = M1, p1 = M2 with M1*M2 = Pt/2 */
   int begin, count;
   int tb;       /* time classes: traces per block; specialised spatial
-                   classes: 1 when U / V are tiled by 16 traces */
+                   classes: 1 when the time transform is specialised too */
+  int hb;       /* run-time sized kernels: coefficient pairs held per line
+                   (half the longest line, rounded up to an instance) */
   int var;      /* time classes: forward kernel variant (0 register
                    prefetch, 1 lean tile); spatial classes: unused */
   size_t lds;
