@@ -498,7 +498,9 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
   int const *const bl = blocks + TB_INTS * (block0 + blockIdx.x);
   AgdWin const &w = wins[bl[0]];
   int const t0 = bl[1], nt = min(2 * kPairs, w.ntr - t0);
-  int const tw0 = bl[2], tw1 = bl[3];
+  int const twn = bl[3] - bl[2];
+  int const tw0 = bl[2] + twn * blockIdx.y / gridDim.y;
+  int const tw1 = bl[2] + twn * (blockIdx.y + 1) / gridDim.y;
   int const twa = tw0 > 0 ? tw0 - 1 : 0;
   int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2;
   int const nconv = w.nconv, ntw = w.ntw, pitch = time_pitch(N);
@@ -587,7 +589,9 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
   int const *const bl = blocks + TB_INTS * bid;
   AgdWin const &w = wins[bl[0]];
   int const t0 = bl[1], nt = min(2 * kPairs, w.ntr - t0);
-  int const tw0 = bl[2], tw1 = bl[3];
+  int const twn = bl[3] - bl[2];
+  int const tw0 = bl[2] + twn * blockIdx.y / gridDim.y;
+  int const tw1 = bl[2] + twn * (blockIdx.y + 1) / gridDim.y;
   int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2;
   int const nconv = w.nconv, pitch = time_pitch(N);
   TimeTables t;
@@ -701,7 +705,7 @@ template <int HB>
 static int launch_fwd_time_g(AgdDev const *g, AgdClass const &c, int first, int n) {
   static int const lds_ok = allow_lds((void const *)k_fwd_time_g<HB>);
   (void)lds_ok;
-  return launch("fwd_time", k_fwd_time_g<HB>, dim3(n), dim3(NTHR), c.lds, g->win,
+  return launch("fwd_time", k_fwd_time_g<HB>, dim3(n, time_split(c, n, 2)), dim3(NTHR), c.lds, g->win,
                 g->tblocks, first, g->dft, g->plans, (float2 const *)g->roots, g->tapers,
                 g->tscale, (float2 const *)g->U, g->T);
 }
@@ -718,7 +722,7 @@ static int launch_adj_time_g(AgdDev const *g, AgdClass const &c, int first, int 
                              float const *Tin, int plain) {
   static int const lds_ok = allow_lds((void const *)k_adj_time_g<HB>);
   (void)lds_ok;
-  return launch("adj_time", k_adj_time_g<HB>, dim3(n), dim3(NTHR), c.lds, g->win,
+  return launch("adj_time", k_adj_time_g<HB>, dim3(n, time_split(c, n, 1)), dim3(NTHR), c.lds, g->win,
                 g->tblocks, first, g->dft, g->plans, (float2 const *)g->roots, g->tapers,
                 g->tscale, g->went, (float const *)g->r, Tin, (float2 *)g->V, plain,
                 first == c.begin && n == c.count ? g->tadj : (int const *)nullptr);

@@ -1427,6 +1427,7 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
           b4[1] = t0;
           b4[2] = (int)((int64_t)W->ntw * q / parts);
           b4[3] = (int)((int64_t)W->ntw * (q + 1) / parts);
+          if (b4[3] - b4[2] > cl->ntw) cl->ntw = b4[3] - b4[2];
         }
       }
     }

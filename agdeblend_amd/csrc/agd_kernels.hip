@@ -1526,7 +1526,10 @@ __global__ __launch_bounds__(time_threads<M1 * M2>()) void k_fwd_time_t(
   int const t0 = blocks[TB_INTS * bid + 1];
   // the block's time windows [tw0, tw1); one that starts inside the window
   // first transforms time window tw0 - 1 again, for its overlap carry only
-  int const tw0 = blocks[TB_INTS * bid + 2], tw1 = blocks[TB_INTS * bid + 3];
+  // (the launch may split the block's run over grid y)
+  int const twb = blocks[TB_INTS * bid + 2], twn = blocks[TB_INTS * bid + 3] - twb;
+  int const tw0 = twb + twn * blockIdx.y / gridDim.y;
+  int const tw1 = twb + twn * (blockIdx.y + 1) / gridDim.y;
   int const twa = tw0 > 0 ? tw0 - 1 : 0;
   int const nconv = w.nconv, ntw = w.ntw;
   int const tid = threadIdx.x;
@@ -1710,7 +1713,9 @@ __global__ __launch_bounds__(time_threads<M1 * M2>()) void k_adj_time_t(
   int const bid = order ? order[block0 + xcd_chunk(blockIdx.x, gridDim.x)] : block0 + blockIdx.x;
   AgdWin const &w = wins[blocks[TB_INTS * bid]];
   int const t0 = blocks[TB_INTS * bid + 1];
-  int const tw0 = blocks[TB_INTS * bid + 2], tw1 = blocks[TB_INTS * bid + 3];
+  int const twb = blocks[TB_INTS * bid + 2], twn = blocks[TB_INTS * bid + 3] - twb;
+  int const tw0 = twb + twn * blockIdx.y / gridDim.y;
+  int const tw1 = twb + twn * (blockIdx.y + 1) / gridDim.y;
   int const nconv = w.nconv;
   int const tid = threadIdx.x;
   {
@@ -2485,13 +2490,13 @@ int agdg_fwd_time(AgdDev const *g) {
 #define FT_CASE(a, b)                                                                   \
     if (!done && c.p0 == a && c.p1 == b) {                                              \
       if (n > 0 && c.var == 0 &&                                                        \
-          launch("fwd_time", k_fwd_time_t<a, b, false>, dim3(n),                        \
+          launch("fwd_time", k_fwd_time_t<a, b, false>, dim3(n, time_split(c, n, 2)),                        \
                  dim3(time_threads<a * b>()), fwd_time_lds<a * b, false>(), g->win,     \
                  g->tblocks, first, g->plans, (float2 const *)g->roots, g->tapers,      \
                  g->tscale, (float2 const *)g->U, g->T))                                \
         return 1;                                                                       \
       if (n > 0 && c.var != 0 &&                                                        \
-          launch("fwd_time", k_fwd_time_t<a, b, true>, dim3(n),                         \
+          launch("fwd_time", k_fwd_time_t<a, b, true>, dim3(n, time_split(c, n, 2)),                         \
                  dim3(time_threads<a * b>()), fwd_time_lds<a * b, true>(), g->win,      \
                  g->tblocks, first, g->plans, (float2 const *)g->roots, g->tapers,      \
                  g->tscale, (float2 const *)g->U, g->T))                                \
@@ -2542,7 +2547,7 @@ int agdg_adj_time(AgdDev const *g, float const *Tin, int plain) {
 #define AT_CASE(a, b)                                                                   \
     if (!done && c.p0 == a && c.p1 == b) {                                              \
       if (n > 0 &&                                                                      \
-          launch("adj_time", k_adj_time_t<a, b>, dim3(n),                                 \
+          launch("adj_time", k_adj_time_t<a, b>, dim3(n, time_split(c, n, 1)),                                 \
                  dim3(time_threads<a * b>()), adj_time_lds<a * b>(), g->win, g->tblocks,   \
                  first, g->plans, (float2 const *)g->roots, g->tapers, g->tscale,        \
                  g->went, (float const *)g->r, Tin, (float2 *)g->V, plain,              \

@@ -6,6 +6,7 @@
 #include "agd_gpu.h"
 
 #define NTHR 256
+#define TIME_SPLIT_BLOCKS 1536
 
 // the library stream; *a: the start event when kernels are timed, else null
 hipStream_t agd_launch_begin(hipEvent_t *a);
@@ -43,4 +44,18 @@ static int allow_lds(void const *f) {
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   (void)hipGetLastError();
   return 1;
+}
+
+// Runs that a launch of n time blocks of class c splits each block's time
+// windows into (grid y), at least `least` time windows to a run. A block's
+// time windows are a serial chain, so below TIME_SPLIT_BLOCKS blocks (six
+// per CU) the chip waits on it: 30 blocks of 9 time windows (256 x 1024
+// line, windows 32 x 256) took 27 us forward and 34 adjoint as one run each
+// and take 15 and 11 split, 236 blocks of 14 (1510 x 1251 line) 113 and 132
+// against 67 and 52; above it the runs would only repeat the forward's
+// carry windows.
+static inline unsigned time_split(AgdClass const &c, int n, int least) {
+  int const want = (TIME_SPLIT_BLOCKS + n - 1) / n, most = c.ntw / least;
+  int const r = want < most ? want : most;
+  return r > 1 ? r : 1;
 }

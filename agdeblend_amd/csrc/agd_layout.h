@@ -93,6 +93,7 @@ typedef struct {
                    (half the longest line, rounded up to an instance) */
   int var;      /* time classes: forward kernel variant (0 register
                    prefetch, 1 lean tile); spatial classes: unused */
+  int ntw;      /* time classes: most time windows of a block */
   size_t lds;
   int const *wpos; /* host array [n_win + 1]: first unit of the class that
                       belongs to window w or later (units are in window
