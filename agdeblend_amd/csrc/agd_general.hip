@@ -569,8 +569,6 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
     float *const tj = Tb + (int64_t)j * nconv;
     for (int s = lane; s < half; s += 64)
       if (ntw * half + s < nconv) tj[ntw * half + s] = CA[j * half + s];
-    // zero the capacity beyond the data portion (wavelet input padding)
-    for (int s = (ntw + 1) * half + lane; s < nconv; s += 64) tj[s] = 0.f;
   }
 }
 

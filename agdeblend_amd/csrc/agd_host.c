@@ -2309,8 +2309,8 @@ EXPORT int agdx_operator(AgdProblem *p, int op, int adjoint, float const *in, fl
   if ((op == 1 && !p->use_wavelets) || (op != 0 && ident_entries(p))) return 1;
   set_u_valid(p, 0);
   if (op == 0 && !adjoint) {
-    /* F: model -> traces */
-    if (agdg_h2d(p->dev.X, in, mb) || agdg_fwd_spatial(&p->dev, p->dev.X) ||
+    /* F: model -> traces (zero beyond n_times_fk, which it does not write) */
+    if (agdg_h2d(p->dev.X, in, mb) || (p->use_wavelets && agdg_zero(p->dev.T, tb)) || agdg_fwd_spatial(&p->dev, p->dev.X) ||
         agdg_fwd_time(&p->dev) || agdg_d2h(out, p->dev.T, tb))
       rc = 1;
   } else if (op == 0) {

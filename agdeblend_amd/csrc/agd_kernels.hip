@@ -435,12 +435,6 @@ __global__ __launch_bounds__(NTHR) void k_fwd_time(
     int const t = w.ntw * half + s;
     if (j < nt && t < w.nconv) T[w.t_off + (int64_t)(t0 + j) * w.nconv + t] = acc[j * Wt + s];
   }
-  // zero the capacity beyond the data portion (wavelet input padding)
-  int const tail0 = w.ntw * half + (Wt - half);
-  for (int j = 0; j < nt; ++j) {
-    for (int t = tail0 + threadIdx.x; t < w.nconv; t += blockDim.x)
-      T[w.t_off + (int64_t)(t0 + j) * w.nconv + t] = 0.f;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1672,9 +1666,6 @@ __global__ __launch_bounds__(time_threads<M1 * M2>()) void k_fwd_time_t(
   for (int r = 0; r < NJ; ++r)
     if (tl < nconv)
       Tb[(j0 + JS * r) * nconv + tl] = LT ? ca[LT ? r : 0] : CA[(j0 + JS * r) * half + s];
-  // zero the capacity beyond the data portion (wavelet input padding)
-  for (int j = 0; j < TG; ++j)
-    for (int t = (ntw + 1) * half + tid; t < nconv; t += NT) Tb[(int64_t)j * nconv + t] = 0.f;
 }
 
 // Adjoint time transform: record (or wavelet-adjoint traces) -> windowed,
