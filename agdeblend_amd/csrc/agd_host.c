@@ -1206,15 +1206,19 @@ static int lines_nk(AgdWin const *W) {
  * one column transform per thread of a 256-thread block (b per plane),
  * within a 48 KB LDS tile of spec_len(a) rows of b + 1 per plane;
  * AGD_SPATIAL_NK overrides */
-static int default_nk(int a, int b) {
+static int default_nk(int a, int b, int Ft) {
   size_t const plane = (size_t)spec_len(a) * (b + 1) * 8;
   char const *e = getenv("AGD_SPATIAL_NK");
-  int nk = e ? atoi(e) : 256 / b;
+  int nk = e ? atoi(e) : a == 1 ? 32 : 256 / b;
   if (nk < 1) nk = 1;
   if ((size_t)nk * plane > 48 * 1024) nk = (int)(48 * 1024 / plane);
   return nk;
 }
 
+  if (e == NULL && a == 1) {
+    int const n = (Ft + nk - 1) / nk; /* tasks of a time window */
+    nk = (Ft + n - 1) / n;
+  }
 /* Spatial tasks of the classes cls[0, ncls): per window of the class, per
  * time window, runs of nk time frequencies (nk_req[c] when given and > 0,
  * else the default rule); fills each class's begin, count, wpos and LDS
@@ -1240,7 +1244,7 @@ static int spatial_tasks(AgdProblem *p, AgdClass *cls, int ncls, int const *nk_r
       if (cl->hb) {
         nk = lines_nk(W);
       } else if (a) {
-        nk = (nk_req && nk_req[c] > 0) ? nk_req[c] : default_nk(a, b);
+        nk = (nk_req && nk_req[c] > 0) ? nk_req[c] : default_nk(a, b, W->Ft);
       } else {
         nk = (int)(LDS_BUDGET / (2 * (size_t)W->S * 8));
       }
@@ -1381,7 +1385,10 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
     int *wpos = (int *)malloc(((size_t)p->n_win + 1) * sizeof(int));
     if (wpos == NULL) return 1;
     cl->wpos = wpos;
-    cl->var = 0;
+    /* the lean tile where the register-prefetch kernel's LDS leaves a CU two
+     * blocks (half lengths from 320: 0.75 against 0.92 ms per iteration on
+     * 64 x 256 x 2048 with windows of 512 samples); equal below */
+    cl->var = cl->p0 * cl->p1 >= 320;
     for (tb = tb_max; tb >= 1; tb /= 2) {
       size_t need = 0;
       for (w = 0; w < p->n_win; w++) {
