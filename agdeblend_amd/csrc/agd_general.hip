@@ -311,7 +311,7 @@ __device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr,
   }
 }
 
-// mode -1: forward only (X -> U); 0..4 as k_adj_spatial_t's MODE, followed by
+// mode -1: forward only (X -> U); 0..5 as k_adj_spatial_t's MODE, followed by
 // the forward transform of the new model when fuse is set
 template <int HB>
 __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_spatial_g(
@@ -381,16 +381,11 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
             nv = gv;
           } else if (mode == 1 || mode == 4) {
             nv = make_float2(0.f - alpha * gv.x, 0.f - alpha * gv.y);
-            mx = fmaxf(mx, nv.x * nv.x + nv.y * nv.y);
+            float const q = nv.x * nv.x + nv.y * nv.y;
+            mx = mode == 1 ? fmaxf(mx, q) : max_bits(mx, q);
           } else {
-            nv = make_float2(v[b].x - alpha * gv.x, v[b].y - alpha * gv.y);
-            if (mode == 0) {
-              // x (|x| - lamb) / |x| when |x| > lamb, else 0
-              float const q = nv.x * nv.x + nv.y * nv.y;
-              float const sh = fmaxf(1.f - lamb * __builtin_amdgcn_rsqf(q), 0.f);
-              nv.x *= sh;
-              nv.y *= sh;
-            }
+            nv = step(mode == 5 ? make_float2(0.f, 0.f) : v[b], alpha, gv);
+            if (mode == 0 || mode == 5) nv = soft(nv, lamb);
           }
           if (mode != 4) x[i] = nv;
         }
@@ -406,12 +401,15 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
     }
     if (mode == 1 || mode == 4) {
       __shared__ float red[4];
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      for (int o = 32; o > 0; o >>= 1) {
+        float const q = __shfl_xor(mx, o, 64);
+        mx = mode == 1 ? fmaxf(mx, q) : max_bits(mx, q);
+      }
       if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
       __syncthreads();
       if (threadIdx.x == 0) {
         float m = red[0];
-        for (int q = 1; q < 4; ++q) m = fmaxf(m, red[q]);
+        for (int q = 1; q < 4; ++q) m = mode == 1 ? fmaxf(m, red[q]) : max_bits(m, red[q]);
         atomicMax(maxbits, __float_as_uint(m));
       }
     }

@@ -134,13 +134,17 @@ int agdg_adj_time(AgdDev const *g, float const *Tin, int plain);
 /* mode 0: X = X - alpha*G then shrink by lamb; mode 1: X = -alpha*G and
  * record max |X|^2 bits in scalar[0]; mode 2: X = X - alpha*G (no shrink);
  * mode 3: X = G; mode 4: as mode 1 without writing X where the kernels
- * allow it (X then holds the previous model or -alpha*G). fuse: also write the forward spatial transform of the new X
+ * allow it (X then holds the previous model or -alpha*G; a NaN anywhere may
+ * make the maximum one); mode 5 (fused only): mode 0 from a zero model,
+ * without reading X. fuse: also write the forward spatial transform of the new X
  * into U (the next iteration's first forward stage). */
 int agdg_adj_spatial(AgdDev const *g, float alpha, float lamb, int mode, int fuse);
 /* 1 when every spatial class has a specialised kernel (fusion available) */
 int agdg_can_fuse(AgdDev const *g);
 /* number of spatial classes the split-precision transforms can serve */
 int agdg_x3_classes(AgdDev const *g);
+/* r = the residual record of the zero model, mute(0) - d */
+int agdg_zero_resid(AgdDev const *g);
 int agdg_shrink(AgdDev const *g, int64_t n_complex, float lamb);
 /* fold of spatial tapers for the stepsize; max written to scalar[1] */
 int agdg_stepsize_fold(AgdDev const *g);

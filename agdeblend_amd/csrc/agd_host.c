@@ -1204,7 +1204,10 @@ static int lines_nk(AgdWin const *W) {
  * sizes; a class is served by one kernel launch. */
 /* planes per spatial task of a specialised class of padded sizes (a, b):
  * one column transform per thread of a 256-thread block (b per plane),
- * within a 48 KB LDS tile of spec_len(a) rows of b + 1 per plane;
+ * within a 48 KB LDS tile of spec_len(a) rows of b + 1 per plane. One space
+ * dim (a = 1): a plane is one row transform, a thread's work, so planes are
+ * what fills a wave: up to 32, in tasks of equal size (256 x 1024 line,
+ * windows 32 x 256: 30 us per launch with 6 planes, 12 with 27).
  * AGD_SPATIAL_NK overrides */
 static int default_nk(int a, int b, int Ft) {
   size_t const plane = (size_t)spec_len(a) * (b + 1) * 8;
@@ -1212,13 +1215,13 @@ static int default_nk(int a, int b, int Ft) {
   int nk = e ? atoi(e) : a == 1 ? 32 : 256 / b;
   if (nk < 1) nk = 1;
   if ((size_t)nk * plane > 48 * 1024) nk = (int)(48 * 1024 / plane);
-  return nk;
-}
-
   if (e == NULL && a == 1) {
     int const n = (Ft + nk - 1) / nk; /* tasks of a time window */
     nk = (Ft + n - 1) / n;
   }
+  return nk;
+}
+
 /* Spatial tasks of the classes cls[0, ncls): per window of the class, per
  * time window, runs of nk time frequencies (nk_req[c] when given and > 0,
  * else the default rule); fills each class's begin, count, wpos and LDS
@@ -2245,7 +2248,7 @@ static int forward_record(AgdProblem *p, int resid) {
 
 /* model_adjoint_update of dev.r into dev.X (modes of agdg_adj_spatial) */
 static int adjoint_update(AgdProblem *p, float alpha, float lamb, int mode) {
-  int const fuse = p->fuse && mode == 0;
+  int const fuse = p->fuse && (mode == 0 || mode == 5);
   if (p->use_wavelets) {
     if (agdg_wavelet(&p->dev, 1)) return 1;
     if (agdg_adj_time(&p->dev, p->dev.T2, 0)) return 1;
@@ -2428,16 +2431,16 @@ static int adjoint_update(AgdProblem *p, float alpha, float lamb, int mode);
 
 /* One iteration in window-chunk order, starting from the residual record of
  * the current model: for each chunk of windows, the adjoint update with
- * threshold lamb and then (unless last) the chunk's forward traces for the
+ * threshold lamb (mode as adjoint_update's) and then (unless last) the chunk's forward traces for the
  * next iteration, whose intermediates are still in cache; finally the
  * residual record of the new model. The same kernels over the same
  * elements as forward_record + adjoint_update, in another launch order. */
-static int chunked_iteration(AgdProblem *p, float alpha, float lamb, int last) {
+static int chunked_iteration(AgdProblem *p, float alpha, float lamb, int last, int mode) {
   int k, rc = 0;
   for (k = 0; k < p->n_chunk && rc == 0; k++) {
     p->dev.w0 = p->chunk[k];
     p->dev.w1 = p->chunk[k + 1];
-    if (adjoint_update(p, alpha, lamb, 0)) rc = 1;
+    if (adjoint_update(p, alpha, lamb, mode)) rc = 1;
     if (rc == 0 && !last) {
       if (!p->fuse && agdg_fwd_spatial(&p->dev, p->dev.X)) rc = 1;
       if (rc == 0 && agdg_fwd_time(&p->dev)) rc = 1;
@@ -2464,7 +2467,7 @@ static int run_captured(AgdProblem *p, float alpha, float const *lamb, int n, in
   if (agdg_graph_begin()) return 1;
   p->dev.lamb_dev = p->lamb_cur;
   if (agdg_next_lamb(&p->dev)) rc = 1;
-  else if (chunked) rc = chunked_iteration(p, alpha, 0.0f, 0);
+  else if (chunked) rc = chunked_iteration(p, alpha, 0.0f, 0, 0);
   else if (forward_record(p, 1) || adjoint_update(p, alpha, 0.0f, 0)) rc = 1;
   p->dev.lamb_dev = NULL;
   {
@@ -2483,9 +2486,10 @@ static int run_captured(AgdProblem *p, float alpha, float const *lamb, int n, in
 
 /* Iterations 1 .. n_its - 1 with thresholds sched[it], from the current
  * model; r_ready: dev.r already holds its residual A x - d (otherwise the
- * first iteration computes it). */
+ * first iteration computes it); x_zero: the current model is zero and dev.X
+ * need not hold it (r_ready, fused kernels). */
 static int run_loop(AgdProblem *p, float alpha, float const *sched, int n_its,
-                    int print_freq, int r_ready) {
+                    int print_freq, int r_ready, int x_zero) {
   int it, rc = 0;
   /* from the second iteration on, every iteration launches the same
    * kernels with the same arguments except the threshold: capture one
@@ -2508,7 +2512,8 @@ static int run_loop(AgdProblem *p, float alpha, float const *sched, int n_its,
         if (agdg_norm2(&p->dev, p->dev.r, p->cfg.rec_len, &r2)) rc = 1;
         else printf("Iteration %d Residual %f\n", it, sqrt(r2));
       }
-      if (rc == 0) rc = chunked_iteration(p, alpha, sched[it], it == n_its - 1);
+      if (rc == 0)
+        rc = chunked_iteration(p, alpha, sched[it], it == n_its - 1, it == 1 && x_zero ? 5 : 0);
       continue;
     }
     if (graph && it == 2) {
@@ -2521,7 +2526,7 @@ static int run_loop(AgdProblem *p, float alpha, float const *sched, int n_its,
       if (agdg_norm2(&p->dev, p->dev.r, p->cfg.rec_len, &r2)) rc = 1;
       else printf("Iteration %d Residual %f\n", it, sqrt(r2));
     }
-    if (rc == 0 && adjoint_update(p, alpha, sched[it], 0)) rc = 1;
+    if (rc == 0 && adjoint_update(p, alpha, sched[it], it == 1 && x_zero ? 5 : 0)) rc = 1;
   }
   return rc;
 }
@@ -2549,12 +2554,13 @@ EXPORT int agdx_run_warm_dev(AgdProblem *p, float f, int n_its, int print_freq,
   return run_impl(p, f, n_its, print_freq, NULL, NULL, warm_dev);
 }
 
-/* The zero start's first update x = 0 - alpha A^H d into dev.X and its
- * threshold lambda0 = max |x| (agdeblend.c:584-590, model.c:1202-1227). */
-/* lambda0 = max |alpha A^H d| (the zero start's first update); keep_x: also
- * leave that update -alpha A^H d in dev.X (else dev.X is left to be
- * overwritten: a warm start or a given initial model) */
-static int lambda0_update(AgdProblem *p, float alpha, float *lamb, int keep_x) {
+/* lambda0 = max |alpha A^H d|, the threshold scale of the zero start's first
+ * update x = 0 - alpha A^H d (agdeblend.c:584-590, model.c:1202-1227);
+ * keep_x: also leave that update in dev.X (else dev.X is left to be
+ * overwritten: a warm start, a given initial model, or an update that the
+ * threshold takes to zero). Set when the update is kept after all, because
+ * it is not finite everywhere. */
+static int lambda0_update(AgdProblem *p, float alpha, float *lamb, int *keep_x) {
   unsigned int bits = 0;
   float l2;
   float *tmp;
@@ -2563,9 +2569,14 @@ static int lambda0_update(AgdProblem *p, float alpha, float *lamb, int keep_x) {
   /* the adjoint reads its record through dev.r: point it at d */
   tmp = p->dev.r;
   p->dev.r = p->dev.d;
-  rc = adjoint_update(p, alpha, 0.0f, keep_x ? 1 : 4);
+  rc = adjoint_update(p, alpha, 0.0f, *keep_x ? 1 : 4);
   p->dev.r = tmp;
   if (rc || agdg_d2h(&bits, p->dev.scalar, sizeof(bits))) return 1;
+  if (!*keep_x && bits >= 0x7f800000u) {
+    /* not finite: the update itself, whose maximum passes over NaN */
+    *keep_x = 1;
+    return lambda0_update(p, alpha, lamb, keep_x);
+  }
   memcpy(&l2, &bits, sizeof(l2));
   *lamb = sqrtf(l2);
   return 0;
@@ -2583,7 +2594,13 @@ static int run_impl(AgdProblem *p, float f, int n_its, int print_freq, float con
   int it;
   int const warm_any = x0 == NULL && (warm != NULL || warm_dev != NULL);
   int zero_start = x0 == NULL && !warm_any;
-  int r_ready = 0;
+  int r_ready = 0, x_zero = 0, keep = 0;
+  /* f = 1: no coefficient of the first update exceeds its own maximum, so
+   * the threshold leaves the zero model (agdeblend.c:587-590). Its residual is
+   * -d and the first iteration starts from it without a model in memory: of
+   * 72 ms for ten iterations of the 64 x 1024 x 2048 volume the writes and
+   * reads of that model, its shrink and its forward took 8. */
+  int const to_zero = f == 1.0f && n_its > 1 && p->fuse;
   double r2_start = -1.0;
   if (!p->have_data) {
     fprintf(stderr, "ERROR: no data set\n");
@@ -2598,7 +2615,8 @@ static int run_impl(AgdProblem *p, float f, int n_its, int print_freq, float con
   } else {
     /* x = 0 - alpha * A^H d; lambda0 = max |x| (for a warm start or x0 the
      * schedule keeps the scale of the zero start) */
-    if (lambda0_update(p, alpha, &lamb, zero_start)) return 1;
+    keep = zero_start && !to_zero;
+    if (lambda0_update(p, alpha, &lamb, &keep)) return 1;
     if (x0 != NULL && agdg_h2d(p->dev.X, x0, (size_t)agdx_model_len(p) * 8)) return 1;
   }
   if (warm_any) {
@@ -2622,13 +2640,18 @@ static int run_impl(AgdProblem *p, float f, int n_its, int print_freq, float con
       g_last_warm_fallback = 1;
       r2_start = -1.0;
       zero_start = 1;
-      if (lambda0_update(p, alpha, &lamb, 1)) return 1;
+      keep = !to_zero;
+      if (lambda0_update(p, alpha, &lamb, &keep)) return 1;
     }
   }
   g_last_lambda0 = lamb;
   slope *= lamb;
   lamb *= f;
-  if (zero_start) {
+  if (zero_start && !keep) {
+    if (agdg_zero_resid(&p->dev)) return 1;
+    set_u_valid(p, 0);
+    r_ready = x_zero = 1;
+  } else if (zero_start) {
     if (agdg_shrink(&p->dev, agdx_model_len(p), lamb)) return 1;
     set_u_valid(p, 0);
   } else if (x0 != NULL) {
@@ -2650,7 +2673,7 @@ static int run_impl(AgdProblem *p, float f, int n_its, int print_freq, float con
       else lamb = (float)(n_its - 1 - it) * slope;
       sched[it] = lamb;
     }
-    rc = run_loop(p, alpha, sched, n_its, print_freq, r_ready);
+    rc = run_loop(p, alpha, sched, n_its, print_freq, r_ready, x_zero);
     free(sched);
     if (rc) return 1;
   }
@@ -2908,7 +2931,7 @@ EXPORT int agdx_iterate(AgdProblem *p, int n, float lamb) {
   sched = (float *)malloc(((size_t)n + 1) * sizeof(float));
   if (sched == NULL) return 1;
   for (it = 0; it <= n; it++) sched[it] = lamb;
-  rc = run_loop(p, p->stepsize, sched, n + 1, 0, 0);
+  rc = run_loop(p, p->stepsize, sched, n + 1, 0, 0, 0);
   free(sched);
   if (rc) return 1;
   return agdg_sync();

@@ -721,6 +721,14 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial(
   }
 }
 
+// r = mute(0) - d: the residual record of the zero model
+__global__ void k_zero_resid(unsigned char const *__restrict__ mute, float const *__restrict__ d,
+                             float *__restrict__ r, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    r[i] = mute[i] ? 0.f : 0.f - d[i];
+}
+
 __global__ void k_shrink(float2 *__restrict__ X, int64_t n, float lamb) {
   float const l2 = lamb * lamb;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -1356,8 +1364,10 @@ __global__ __launch_bounds__(NTHR) void k_fwd_spatial_t(
 //   2  x <- x - alpha g
 //   3  x <- g
 //   4  max |alpha g|^2 into maxbits, x untouched (the threshold scale of a
-//      start whose model is written afterwards)
-// With FUSE (modes 0 and 3) the new model's forward spatial transform, the
+//      start whose model is written afterwards); a NaN makes the result one,
+//      where mode 1 passes over it
+//   5  x <- S_lamb(0 - alpha g): mode 0 from the zero model, which is not read
+// With FUSE (modes 0, 3 and 5) the new model's forward spatial transform, the
 // next forward's first stage, is written to U.
 template <int P0, int P1, int MODE, bool FUSE>
 __global__ __launch_bounds__(NTHR) void k_adj_spatial_t(
@@ -1398,18 +1408,11 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial_t(
         nv = gv;
       } else if constexpr (MODE == 1 || MODE == 4) {
         nv = make_float2(0.f - alpha * gv.x, 0.f - alpha * gv.y);
-        mx = fmaxf(mx, nv.x * nv.x + nv.y * nv.y);
+        float const a = nv.x * nv.x + nv.y * nv.y;
+        mx = MODE == 1 ? fmaxf(mx, a) : max_bits(mx, a);
       } else {
-        nv = xc[c0 * P1];
-        nv.x -= alpha * gv.x;
-        nv.y -= alpha * gv.y;
-        if constexpr (MODE == 0) {
-          // x (|x| - lamb) / |x| when |x| > lamb, else 0
-          float const a = nv.x * nv.x + nv.y * nv.y;
-          float const sh = fmaxf(1.f - lamb * __builtin_amdgcn_rsqf(a), 0.f);
-          nv.x *= sh;
-          nv.y *= sh;
-        }
+        nv = step(MODE == 5 ? make_float2(0.f, 0.f) : xc[c0 * P1], alpha, gv);
+        if constexpr (MODE == 0 || MODE == 5) nv = soft(nv, lamb);
       }
       if constexpr (MODE != 4) xc[c0 * P1] = nv;
       v[c0] = nv;
@@ -1422,12 +1425,16 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial_t(
   }
   if constexpr (MODE == 1 || MODE == 4) {
     __shared__ float red[NTHR / 64];
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    for (int o = 32; o > 0; o >>= 1) {
+      float const a = __shfl_xor(mx, o, 64);
+      mx = MODE == 1 ? fmaxf(mx, a) : max_bits(mx, a);
+    }
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
     __syncthreads();
     if (threadIdx.x == 0) {
       float m = red[0];
-      for (int q = 1; q < (int)(blockDim.x >> 6); ++q) m = fmaxf(m, red[q]);
+      for (int q = 1; q < (int)(blockDim.x >> 6); ++q)
+        m = MODE == 1 ? fmaxf(m, red[q]) : max_bits(m, red[q]);
       atomicMax(maxbits, __float_as_uint(m));
     }
   }
@@ -2256,7 +2263,7 @@ static int launch_adj_spatial(AgdDev const *g, AgdClass const &c, float alpha, f
 template <int P0, int P1>
 static int adj_spatial_sized(AgdDev const *g, AgdClass const &c, float alpha, float lamb,
                              int mode, int fuse) {
-  if (fuse && mode != 0 && mode != 3) {
+  if (fuse && mode != 0 && mode != 3 && mode != 5) {
     fprintf(stderr, "ERROR: fused update requested for mode %d\n", mode);
     return 1;
   }
@@ -2267,6 +2274,7 @@ static int adj_spatial_sized(AgdDev const *g, AgdClass const &c, float alpha, fl
     case 1: return launch_adj_spatial<P0, P1, 1, false>(g, c, alpha, lamb);
     case 2: return launch_adj_spatial<P0, P1, 2, false>(g, c, alpha, lamb);
     case 4: return launch_adj_spatial<P0, P1, 4, false>(g, c, alpha, lamb);
+    case 5: return launch_adj_spatial<P0, P1, 5, true>(g, c, alpha, lamb);
     default:
       return fuse ? launch_adj_spatial<P0, P1, 3, true>(g, c, alpha, lamb)
                   : launch_adj_spatial<P0, P1, 3, false>(g, c, alpha, lamb);
@@ -2629,6 +2637,13 @@ int agdg_adj_spatial(AgdDev const *g, float alpha, float lamb, int mode, int fus
     }
   }
   return 0;
+}
+
+int agdg_zero_resid(AgdDev const *g) {
+  int64_t blocks = (g->rec_len + NTHR - 1) / NTHR;
+  if (blocks > 65536) blocks = 65536;
+  return launch("zero_resid", k_zero_resid, dim3((unsigned)blocks), dim3(NTHR), 0, g->mute,
+                (float const *)g->d, g->r, g->rec_len);
 }
 
 int agdg_shrink(AgdDev const *g, int64_t n_complex, float lamb) {

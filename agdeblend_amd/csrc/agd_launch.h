@@ -31,6 +31,24 @@ __device__ __forceinline__ int xcd_chunk(int b, int n) {
   return x * q + min(x, r) + i;
 }
 
+// the larger of two non-negative floats, or a NaN if there is one (their
+// bits order that way)
+__device__ __forceinline__ float max_bits(float a, float b) {
+  return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
+}
+
+// soft threshold x (|x| - lamb) / |x| when |x| > lamb, else 0; one rounding
+// order in every kernel that inlines it
+__device__ __forceinline__ float2 soft(float2 v, float lamb) {
+  float const a = fmaf(v.x, v.x, v.y * v.y);
+  float const s = fmaxf(fmaf(-lamb, __builtin_amdgcn_rsqf(a), 1.f), 0.f);
+  return make_float2(v.x * s, v.y * s);
+}
+// x - alpha g
+__device__ __forceinline__ float2 step(float2 x, float alpha, float2 g) {
+  return make_float2(fmaf(-alpha, g.x, x.x), fmaf(-alpha, g.y, x.y));
+}
+
 // units of class c within the launch's window range: [*first, *first + n)
 static inline int class_range(AgdDev const *g, AgdClass const &c, int *first) {
   int const a = c.wpos[g->w0], b = c.wpos[g->w1];

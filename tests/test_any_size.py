@@ -65,12 +65,17 @@ def test_any_window_length_matches_fp64_oracle(shape, windows):
         pm.close()
 
 
+@pytest.mark.parametrize("nan", [False, True])
 @pytest.mark.parametrize("shape,windows", [((61, 300), (24, 106)), ((17, 34, 160), (16, 33, 64))])
-def test_fused_iterations_match_separate_transforms(shape, windows, monkeypatch):
-    """The update fused with the next forward against the same kernel run
-    as two launches (AGD_NO_FUSE): the same operations, bit for bit."""
+def test_fused_iterations_match_separate_transforms(shape, windows, nan, monkeypatch):
+    """The update fused with the next forward, from a zero model that is
+    never in memory, against a written zero model and the same transforms as
+    two launches (AGD_NO_FUSE): the same operations, bit for bit; a NaN in
+    the data reaches the same samples."""
     kw = _kw(_spec_geometry(shape, windows, 5))
     data = [np.random.default_rng(6).standard_normal(shape).astype(np.float32)]
+    if nan:
+        data[0][..., -1, 40] = np.nan
     outs = []
     for fused in (True, False):
         monkeypatch.delenv("AGD_NO_FUSE", raising=False)
@@ -79,8 +84,30 @@ def test_fused_iterations_match_separate_transforms(shape, windows, monkeypatch)
         pm = L.Problem(**kw)
         try:
             pm.set_data(data)
-            pm.run(1.0, 7)
+            pm.run(1.0, 2 if nan else 7)
             outs.append(pm.output()[0])
         finally:
             pm.close()
-    assert np.array_equal(outs[0], outs[1])
+    assert np.array_equal(outs[0], outs[1], equal_nan=True)
+    assert np.isnan(outs[0]).any() == nan
+
+
+@pytest.mark.parametrize("n_its", [2, 7])
+@pytest.mark.parametrize("shape,windows", [((61, 300), (24, 106)), ((17, 34, 160), (16, 33, 64)),
+                                           ((64, 512), (32, 128)), ((16, 64, 512), (16, 32, 256))])
+def test_zero_start_matches_a_zero_model(shape, windows, n_its):
+    """The zero start keeps no model in memory before its first update; an
+    initial model of zeros given by the caller is read: the same numbers,
+    bit for bit."""
+    kw = _kw(_spec_geometry(shape, windows, 5))
+    data = [np.random.default_rng(6).standard_normal(shape).astype(np.float32)]
+    pm = L.Problem(**kw)
+    try:
+        pm.set_data(data)
+        pm.run(1.0, n_its)
+        out = pm.output()[0]
+        pm.set_data(data)
+        pm.run(1.0, n_its, x0=np.zeros(pm.model_len, np.complex64))
+        assert np.array_equal(out, pm.output()[0])
+    finally:
+        pm.close()
