@@ -58,7 +58,7 @@ static inline int class_range(AgdDev const *g, AgdClass const &c, int *first) {
 
 // the specialised kernels may use up to the CU's 160 KB of LDS: set once per
 // kernel instance, on its first launch
-static int allow_lds(void const *f) {
+static inline int allow_lds(void const *f) {
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   (void)hipGetLastError();
   return 1;

@@ -19,6 +19,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include "agd_launch.h"
 #include "agdeblend_unet.h"
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
@@ -1138,181 +1139,186 @@ __global__ void k_flip_weights(uint16_t const *__restrict__ wt, uint16_t *__rest
 // Weight and bias gradients: dW[tap][co][ci] = sum_v dy[v][co] x[v + tap][ci],
 // db[co] = sum_v dy[v][co]
 // ---------------------------------------------------------------------------
-// A GEMM over voxels (K) on the matrix cores: for one tap, A[co][v] = dy and
-// B[v][ci] = the shifted input. A block owns one 64-voxel w chunk of RB
-// consecutive (n, d, h) rows and a group of taps (NKH = 3: the nine taps of
-// one kd, grid.y = kd; NKH = 1: the three taps of one (kd, kh)). Per row it
-// stages dy transposed (dys[co][v]) and the input rows transposed once per
-// kw shift (xs[r][kw][ci][v]), so both operands are aligned 16-byte LDS
-// reads (K = 32 voxels per matrix-core step); waves split the (tap, co
-// tile, ci tile) products and the two 32-voxel chunks of the row. The block's partial sums (fixed-order
-// reduction over its waves) go to part[block][27][CO][CI] (taps of its
-// group only) and, for grid.y == 0, the bias partials to bpart[block][CO].
-template <int CI, int CO, int NKH>
-struct WgradShape {
-  static constexpr int NTAP = NKH * 3;
-  static constexpr int NTILE = NTAP * (CO / 16) * (CI / 16);
-  static constexpr int TG = NTILE <= 64 ? 2 : 4;  // waves over tiles
-  static constexpr int NCS = 4 / TG;               // chunk groups (of the two 32-voxel chunks)
-  static constexpr int CPW = 2 / NCS;              // chunks per wave
-  static constexpr int NPW = (NTILE + TG - 1) / TG;  // tiles per wave
-  // LDS row: 64 voxels + 8: 16-byte aligned reads, and the eight rows of a
-  // read cycle in distinct bank groups
-  static constexpr int LR = 72;
-  static constexpr int XS = NKH * 3 * CI * LR;                          // bf16 elements
-  static constexpr int DS = CO * LR;
-  static constexpr int RED = (NCS > 1 ? TG * NPW * 256 : 0) > 256       // floats
-                                 ? (NCS > 1 ? TG * NPW * 256 : 0)
-                                 : 256;
-  static constexpr int LDS_BYTES =
-      (2 * (XS + DS) > 4 * RED ? 2 * (XS + DS) : 4 * RED);
-  static constexpr int NPART = 256 / CO;  // bias: voxel parts per channel
-  static constexpr int VPP = 64 / NPART;
-};
+// A GEMM over voxels (K) on the matrix cores, one 16 x 16 tile pair of
+// (output, input) channels per block (grid.y): per tap A[co][v] = dy and
+// B[v][ci] = the shifted input, K = 32 voxels along w per instruction. Rows
+// sit in LDS as in memory, [voxel][16 channels], and both operands come
+// through the transposing LDS read, so a kw shift is a row offset and
+// nothing is transposed when staged. A block owns a 64-voxel w chunk of RB
+// consecutive (n, d, h) rows and one kd; its two waves take a 32-voxel half
+// each and walk the input rows with the three dy rows (kh) that meet one in
+// registers: one new row of each per step, so a step's nine matrix-core
+// instructions need four operand reads. The rows of the next two steps are in flight during the current one
+// (two register sets, two LDS stages, one barrier per step). A row chunk's
+// three kd are neighbours on one XCD (they read the same dy rows). The sums
+// keep one fixed order: a half's rows in turn, the two halves, then the
+// blocks (k_reduce_parts). The partial sums go to part[block][27][CO][CI],
+// the bias's to bpart[block][CO].
+//
+// Bound by its loads (dy and x three times). 11 launches of a training step
+// on 16 x 32 x 32 x 256: 4.65 ms when rows were staged transposed, once per
+// (kh, kw), for 18 instructions a row; 2.64 with the rows as they are and six
+// waves a block (all kd), 2.06 so. Input rows against nine dy rows, four d to
+// a block, read less and took 1.1 ms, but sum in another order: enough to
+// change the second step of Adam in the fifth digit.
+#define WG_T 128
+// LDS row of voxel v: 32 bytes, 128 more per 8 voxels (the four row groups of
+// an operand read then fall in distinct banks)
+#define WG_ROW(v) ((v) * 32 + ((v) >> 3) * 128)
+#define WG_DY WG_ROW(64)                     // bytes of a stage's dy row
+#define WG_X (WG_ROW(65) + 32)               // and of one input row (w0 - 1 .. w0 + 64)
+#define WG_STAGE (WG_DY + (WG_X + 127) / 128 * 128)
 
-template <int CI, int CO, int NKH>
-__global__ __launch_bounds__(UT) void k_conv3_wgrad(
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// 8 voxels of one channel (lane: channel l % 16, voxels 8 (l / 16) + e): two
+// transposing reads of 4 rows of 16 channels, at lo and hi
+__device__ __forceinline__ u32x4 ld_tr(unsigned char *lo, unsigned char *hi) {
+  typedef s16x4 __attribute__((address_space(3))) * lds4;
+  s16x4 const a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(s16x4 *)lo);
+  s16x4 const b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(s16x4 *)hi);
+  uint2 const l = __builtin_bit_cast(uint2, a), h = __builtin_bit_cast(uint2, b);
+  return u32x4{l.x, l.y, h.x, h.y};
+}
+
+__global__ __launch_bounds__(WG_T, 4) void k_conv3_wgrad(
     uint16_t const *__restrict__ x, uint16_t const *__restrict__ dy, float *__restrict__ part,
-    float *__restrict__ bpart, int D, int H, int W, int64_t rows, int RB) {
-  using S = WgradShape<CI, CO, NKH>;
-  static_assert(CI % 16 == 0 && (CO == 16 || CO == 32 || CO == 64), "channel counts");
-  constexpr int LR = S::LR;
-  __shared__ __align__(16) unsigned char lds[S::LDS_BYTES];
-  uint16_t *const xs = (uint16_t *)lds;         // [NKH][3][CI][LR]
-  uint16_t *const dys = xs + S::XS;             // [CO][LR]
-  int const tid = threadIdx.x;
-  int const lane = tid & 63, wave = tid >> 6;
+    float *__restrict__ bpart, int D, int H, int W, int CI, int CO, int64_t rows, int RB) {
+  constexpr int RED = 9 * 256 * 4;
+  __shared__ __align__(16) unsigned char lds[2 * WG_STAGE > RED ? 2 * WG_STAGE : RED];
+  int const tid = threadIdx.x, lane = tid & 63;
   int const i = lane & 15, kq = lane >> 4;
-  int const tg = wave % S::TG, cs = wave / S::TG;
+  int const cs = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int const id = xcd_chunk(blockIdx.x, gridDim.x);
+  int const blk = id / 3, kd = id - 3 * blk;
+  int const ct = blockIdx.y % (CO / 16), it = blockIdx.y / (CO / 16);
   int const nwc = (W + 63) / 64;
-  int const wc = blockIdx.x % nwc;
-  int64_t const rb = blockIdx.x / nwc;
-  int const w0 = wc * 64;
-  int const g = blockIdx.y;
-  int const kd = NKH == 3 ? g : g / 3;
-  int const kh0 = NKH == 3 ? 0 : g % 3;
-  bool const do_bias = bpart != nullptr && g == 0;
-  f32x4 acc[S::NPW];
-#pragma unroll
-  for (int t = 0; t < S::NPW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.f;
-  int64_t const r0 = rb * RB;
+  int const w0 = (blk % nwc) * 64;
+  int64_t const r0 = (int64_t)(blk / nwc) * RB;
   int64_t const r1 = r0 + RB < rows ? r0 + RB : rows;
-  for (int64_t row = r0; row < r1; ++row) {
-    int const h = (int)(row % H);
-    int64_t const nd = row / H;
-    int const d = (int)(nd % D);
-    int64_t const n = nd / D;
-    __syncthreads();
-    // dy row, transposed: item = (voxel pair, 8-channel group)
-    for (int e = tid; e < 32 * (CO / 8); e += UT) {
-      int const v2 = e & 31, c8 = e >> 5;
-      int const wv = w0 + 2 * v2;
-      uint4 p0 = make_uint4(0, 0, 0, 0), p1 = p0;
-      int64_t const base = (row * W + wv) * CO + c8 * 8;
-      if (wv < W) p0 = *(uint4 const *)(dy + base);
-      if (wv + 1 < W) p1 = *(uint4 const *)(dy + base + CO);
-      uint32_t const a0[4] = {p0.x, p0.y, p0.z, p0.w}, a1[4] = {p1.x, p1.y, p1.z, p1.w};
+  // bias sums: channel tid % 16, voxels [vpp p, vpp (p + 1)), p = tid / 16 (+ 8)
+  int const npart = 256 / CO, vpp = 64 / npart, pt = tid >> 4;
+  bool const do_bias = bpart != nullptr && it == 0 && kd == 1;
+  float bsum[2] = {0.f, 0.f};
+  f32x4 acc[9];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        uint32_t const lo = (a0[k] & 0xffffu) | (a1[k] << 16);
-        uint32_t const hi = (a0[k] >> 16) | (a1[k] & 0xffff0000u);
-        *(uint32_t *)(dys + (c8 * 8 + 2 * k) * LR + 2 * v2) = lo;
-        *(uint32_t *)(dys + (c8 * 8 + 2 * k + 1) * LR + 2 * v2) = hi;
+  for (int t = 0; t < 9; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // the thread's 16-byte items of a stage (voxel, half of its 16 channels):
+  // one of the dy row and one of the input row per 64 threads and half, and
+  // the input row's two last voxels
+  int const v = tid >> 1, half = (tid & 1) * 16;
+  int const c8 = (tid & 1) * 8;
+  bool const dylive = w0 + v < W, more = tid < 4 && w0 + 63 + v < W;
+  bool const xlive = w0 - 1 + v >= 0 && w0 - 1 + v < W;
+  int const dyat = WG_ROW(v) + half, xat = WG_DY + dyat, mat = WG_DY + WG_ROW(64 + v) + half;
+  // the lane's operand rows: of dy, and of the input row by kw
+  int const rl = cs * 32 + 8 * kq + (i >> 2), col = (i & 3) * 8;
+  int const alo = col + WG_ROW(rl), ahi = col + WG_ROW(rl + 4);
+  int blo[3], bhi[3];
+#pragma unroll
+  for (int kw = 0; kw < 3; ++kw) {
+    blo[kw] = col + WG_DY + WG_ROW(rl + kw);
+    bhi[kw] = col + WG_DY + WG_ROW(rl + 4 + kw);
+  }
+  int buf = 0;
+  // runs of rows of one (n, d)
+  for (int64_t ra = r0; ra < r1;) {
+    int const h0 = (int)(ra % H);
+    int64_t const nd = ra / H;
+    int const d = (int)(nd % D), dd = d + kd - 1;
+    int const h1 = (int)(r1 - ra < H - h0 ? h0 + (r1 - ra) : H);
+    ra += h1 - h0;
+    bool const plane = dd >= 0 && dd < D;
+    // step h = h0 - 1 .. h1: the input row h and the dy row h + 1. Loads are
+    // unconditional (a row outside the run or the volume reads the tensor's
+    // first voxel and is zeroed).
+    uint16_t const *const py = dy + (nd * H * W + w0 + v) * CO + ct * 16 + c8;
+    uint16_t const *const px =
+        x + ((nd + (kd - 1)) * H * W + (w0 - 1 + v)) * (int64_t)CI + it * 16 + c8;
+    struct Rows {
+      uint4 y, x, m;
+    };
+    auto fetch = [&](int h) {
+      Rows r;
+      bool const oy = dylive && h + 1 < h1, ox = plane && h >= 0 && h < H;
+      r.y = *(uint4 const *)(oy ? py + (int64_t)(h + 1) * W * CO : dy);
+      r.x = *(uint4 const *)(ox && xlive ? px + (int64_t)h * W * CI : x);
+      r.m = make_uint4(0, 0, 0, 0);
+      if (tid < 4) r.m = *(uint4 const *)(ox && more ? px + ((int64_t)h * W + 64) * CI : x);
+      if (!oy) r.y = make_uint4(0, 0, 0, 0);
+      if (!(ox && xlive)) r.x = make_uint4(0, 0, 0, 0);
+      if (!(ox && more)) r.m = make_uint4(0, 0, 0, 0);
+      return r;
+    };
+    u32x4 a[3] = {};  // dy rows h + 1 - kh
+    auto step = [&](int h, Rows &r) {
+      unsigned char *const st = lds + buf * WG_STAGE;
+      buf ^= 1;
+      *(uint4 *)(st + dyat) = r.y;
+      *(uint4 *)(st + xat) = r.x;
+      if (tid < 4) *(uint4 *)(st + mat) = r.m;
+      __syncthreads();
+      if (h + 2 <= h1) r = fetch(h + 2);
+      a[2] = a[1];
+      a[1] = a[0];
+      a[0] = ld_tr(st + alo, st + ahi);
+      u32x4 b[3];
+#pragma unroll
+      for (int kw = 0; kw < 3; ++kw) b[kw] = ld_tr(st + blo[kw], st + bhi[kw]);
+      if (do_bias && h + 1 < h1) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          int const p = pt + 8 * u;
+          if (p >= npart) continue;
+          uint16_t const *const q = (uint16_t const *)st + (tid & 15);
+          for (int k = p * vpp; k < (p + 1) * vpp; k += 4) {
+            uint16_t const *const z = q + WG_ROW(k) / 2;  // 4 voxels of one group of 8
+            bsum[u] += (bf2f(z[0]) + bf2f(z[16])) + (bf2f(z[32]) + bf2f(z[48]));
+          }
+        }
       }
-    }
-    // input rows (dd, hh) for the group's kh, once per kw shift
-    int const dd = d + kd - 1;
-    for (int e = tid; e < NKH * 3 * 32 * (CI / 8); e += UT) {
-      int const v2 = e & 31;
-      int const c8 = (e >> 5) % (CI / 8);
-      int const rk = (e >> 5) / (CI / 8);  // r * 3 + kw
-      int const r = rk / 3, kw = rk - r * 3;
-      int const hh = h + kh0 + r - 1;
-      int const wv = w0 + 2 * v2 + kw - 1;
-      bool const okrow = dd >= 0 && dd < D && hh >= 0 && hh < H;
-      uint4 p0 = make_uint4(0, 0, 0, 0), p1 = p0;
-      int64_t const base = (((n * D + dd) * H + hh) * (int64_t)W + wv) * CI + c8 * 8;
-      if (okrow && wv >= 0 && wv < W) p0 = *(uint4 const *)(x + base);
-      if (okrow && wv + 1 >= 0 && wv + 1 < W) p1 = *(uint4 const *)(x + base + CI);
-      uint32_t const a0[4] = {p0.x, p0.y, p0.z, p0.w}, a1[4] = {p1.x, p1.y, p1.z, p1.w};
-      uint16_t *const dst = xs + (rk * CI + c8 * 8) * LR + 2 * v2;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        *(uint32_t *)(dst + (2 * k) * LR) = (a0[k] & 0xffffu) | (a1[k] << 16);
-        *(uint32_t *)(dst + (2 * k + 1) * LR) = (a0[k] >> 16) | (a1[k] & 0xffff0000u);
+      for (int kh = 0; kh < 3; ++kh) {
+        if (h + 1 - kh < h0 || h + 1 - kh >= h1) continue;
+#pragma unroll
+        for (int kw = 0; kw < 3; ++kw) acc[kh * 3 + kw] = mfma32(a[kh], b[kw], acc[kh * 3 + kw]);
       }
-    }
-    __syncthreads();
-    if (do_bias) {
-      int const co = tid % CO, pt = tid / CO;
-#pragma unroll
-      for (int v = 0; v < S::VPP; v += 4) {
-        bf16x4 const q = *(bf16x4 const *)(dys + co * LR + pt * S::VPP + v);
-        bsum += (bf2f((uint16_t)q[0]) + bf2f((uint16_t)q[1])) +
-                (bf2f((uint16_t)q[2]) + bf2f((uint16_t)q[3]));
-      }
-    }
-#pragma unroll
-    for (int cc = 0; cc < S::CPW; ++cc) {
-      int const c = cs + cc * S::NCS;  // 32-voxel chunk
-#pragma unroll
-      for (int j = 0; j < S::NPW; ++j) {
-        int const t = tg + j * S::TG;
-        if (S::NTILE % S::TG != 0 && t >= S::NTILE) break;
-        int const ct = t % (CO / 16);
-        int const it = (t / (CO / 16)) % (CI / 16);
-        int const tap = t / ((CO / 16) * (CI / 16));  // r * 3 + kw
-        u32x4 const a = *(u32x4 const *)(dys + (ct * 16 + i) * LR + c * 32 + 8 * kq);
-        u32x4 const b = *(u32x4 const *)(xs + (tap * CI + it * 16 + i) * LR + c * 32 + 8 * kq);
-        acc[j] = mfma32(a, b, acc[j]);
-      }
+    };
+    Rows p0 = fetch(h0 - 1), p1 = fetch(h0);
+    for (int h = h0 - 1; h <= h1; h += 2) {
+      step(h, p0);
+      if (h + 1 <= h1) step(h + 1, p1);
     }
   }
-  // bias: fixed-order sum over the voxel parts
   float *const red = (float *)lds;
   if (do_bias) {
     __syncthreads();
-    red[tid] = bsum;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (pt + 8 * u < npart) red[tid + 128 * u] = bsum[u];
     __syncthreads();
-    if (tid < CO) {
-      float b = 0.f;
-      for (int pt = 0; pt < S::NPART; ++pt) b += red[pt * CO + tid];
-      bpart[(int64_t)blockIdx.x * CO + tid] = b;
+    if (tid < 16) {
+      float s = 0.f;
+      for (int q = 0; q < npart; ++q) s += red[q * 16 + tid];
+      bpart[(int64_t)blk * CO + ct * 16 + tid] = s;
     }
   }
-  // fixed-order sum over the chunk groups, then one partial per block
-  for (int sgrp = 1; sgrp < S::NCS; ++sgrp) {
-    __syncthreads();
-    if (cs == sgrp) {
+  // the two halves, then one partial per block
+  __syncthreads();
+  if (cs == 1) {
 #pragma unroll
-      for (int j = 0; j < S::NPW; ++j)
+    for (int t = 0; t < 9; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red[(tg * S::NPW + j) * 256 + r * 64 + lane] = acc[j][r];
-    }
-    __syncthreads();
-    if (cs == 0) {
-#pragma unroll
-      for (int j = 0; j < S::NPW; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[j][r] += red[(tg * S::NPW + j) * 256 + r * 64 + lane];
-    }
+      for (int q = 0; q < 4; ++q) red[t * 256 + q * 64 + lane] = acc[t][q];
   }
+  __syncthreads();
   if (cs == 0) {
-    float *const out = part + (int64_t)blockIdx.x * 27 * CO * CI;
+    float *const out = part + (int64_t)blk * 27 * CO * CI;
 #pragma unroll
-    for (int j = 0; j < S::NPW; ++j) {
-      int const t = tg + j * S::TG;
-      if (S::NTILE % S::TG != 0 && t >= S::NTILE) break;
-      int const ct = t % (CO / 16);
-      int const it = (t / (CO / 16)) % (CI / 16);
-      int const tl = t / ((CO / 16) * (CI / 16));
-      int const kh = kh0 + tl / 3, kw = tl % 3;
-      int const tap = (kd * 3 + kh) * 3 + kw;
+    for (int t = 0; t < 9; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        out[((int64_t)tap * CO + ct * 16 + 4 * kq + r) * CI + it * 16 + i] = acc[j][r];
-    }
+      for (int q = 0; q < 4; ++q)
+        out[((int64_t)(kd * 9 + t) * CO + ct * 16 + 4 * kq + q) * CI + it * 16 + i] =
+            acc[t][q] + red[t * 256 + q * 64 + lane];
   }
 }
 
@@ -1761,24 +1767,26 @@ int agdu_flip_weights(void const *wt, void *wtt, int CI, int CO, void *stream) {
                  dim3(UT), stream, (uint16_t const *)wt, (uint16_t *)wtt, CI, CO);
 }
 
+// the channel pairs of the network's layers (and their input gradients), and
+// the share of 2048 blocks that cuts a pair's rows into blocks
 #define WGRAD_CASES(X) \
-  X(16, 16, 3) X(16, 32, 3) X(32, 32, 3) X(48, 16, 3) X(32, 16, 3) X(32, 64, 1) X(64, 64, 1) \
-  X(96, 32, 1) X(64, 32, 1) X(16, 64, 3)
+  X(16, 16, 3) X(16, 32, 3) X(32, 32, 3) X(48, 16, 3) X(32, 16, 3) X(32, 64, 9) X(64, 64, 9) \
+  X(96, 32, 9) X(64, 32, 9) X(16, 64, 3)
 
-// launch shape of the weight gradient: tap groups (grid.y), rows per block
+// launch shape of the weight gradient: tile pairs (grid.y), rows per block
 // and blocks (grid.x); 0 when the channel pair has no kernel
-static int wgrad_plan(int N, int D, int H, int W, int CI, int CO, int *groups, int *rb,
+static int wgrad_plan(int N, int D, int H, int W, int CI, int CO, int *pairs, int *rb,
                       int64_t *nblk) {
-  int nkh = 0;
+  int share = 0;
 #define WC(a, b, k) \
-  if (CI == a && CO == b) nkh = k;
+  if (CI == a && CO == b) share = k;
   WGRAD_CASES(WC)
 #undef WC
-  if (nkh == 0) return 0;
-  *groups = nkh == 3 ? 3 : 9;
+  if (share == 0) return 0;
+  *pairs = (CI / 16) * (CO / 16);
   int64_t const rows = (int64_t)N * D * H;
   int64_t const nwc = (W + 63) / 64;
-  int64_t const target = 2048 / *groups;
+  int64_t const target = 2048 / share;
   int64_t r = (rows * nwc + target - 1) / target;
   if (r < 1) r = 1;
   *rb = (int)r;
@@ -1789,19 +1797,19 @@ static int wgrad_plan(int N, int D, int H, int W, int CI, int CO, int *groups, i
 #define RED_PER 32
 
 int64_t agdu_wgrad_part_len(int N, int D, int H, int W, int CI, int CO) {
-  int groups, rb;
+  int pairs, rb;
   int64_t nblk;
-  if (!wgrad_plan(N, D, H, W, CI, CO, &groups, &rb, &nblk)) return -1;
+  if (!wgrad_plan(N, D, H, W, CI, CO, &pairs, &rb, &nblk)) return -1;
   int64_t const ng = (nblk + RED_PER - 1) / RED_PER;
   return nblk * (27 * CI * CO + CO) + ng * (27 * CI * CO + CO);
 }
 
 int agdu_conv3_wgrad(void const *x, void const *dy, float *part, float *dw, float *db, int N,
                      int D, int H, int W, int CI, int CO, void *stream) {
-  int groups, rb;
+  int pairs, rb;
   int64_t nblk;
   if (N < 1 || D < 1 || H < 1 || W < 1 ||
-      !wgrad_plan(N, D, H, W, CI, CO, &groups, &rb, &nblk) || nblk > 0x7fffffff) {
+      !wgrad_plan(N, D, H, W, CI, CO, &pairs, &rb, &nblk) || 3 * nblk > 0x7fffffff) {
     fprintf(stderr, "ERROR: weight gradient for %d -> %d channels, %d x %d x %d x %d "
                     "unsupported\n", CI, CO, N, D, H, W);
     return 1;
@@ -1811,17 +1819,10 @@ int agdu_conv3_wgrad(void const *x, void const *dy, float *part, float *dw, floa
   float *const gw = bpart + nblk * CO;
   int64_t const ng = (nblk + RED_PER - 1) / RED_PER;
   float *const gb = gw + ng * len;
-  int64_t const rows = (int64_t)N * D * H;
-  dim3 const grid((unsigned)nblk, (unsigned)groups);
-  int rc = 1;
-#define WC(a, b, k)                                                                        \
-  if (CI == a && CO == b)                                                                  \
-    rc = ulaunch("conv3_wgrad", k_conv3_wgrad<a, b, k>, grid, dim3(UT), stream,            \
-                 (uint16_t const *)x, (uint16_t const *)dy, part, db ? bpart : (float *)0, \
-                 D, H, W, rows, rb);
-  WGRAD_CASES(WC)
-#undef WC
-  if (rc) return 1;
+  if (ulaunch("conv3_wgrad", k_conv3_wgrad, dim3(3 * (unsigned)nblk, (unsigned)pairs), dim3(WG_T),
+              stream, (uint16_t const *)x, (uint16_t const *)dy, part, db ? bpart : (float *)0, D,
+              H, W, CI, CO, (int64_t)N * D * H, rb))
+    return 1;
   // two-level fixed-order sums over the blocks
   if (ulaunch("reduce_parts", k_reduce_parts, dim3((unsigned)blocks_for(len, UT), (unsigned)ng),
               dim3(UT), stream, (float const *)part, gw, (int)nblk, len, RED_PER) ||
