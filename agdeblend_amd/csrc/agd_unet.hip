@@ -1140,7 +1140,7 @@ __global__ void k_flip_weights(uint16_t const *__restrict__ wt, uint16_t *__rest
 // db[co] = sum_v dy[v][co]
 // ---------------------------------------------------------------------------
 // A GEMM over voxels (K) on the matrix cores, one 16 x 16 tile pair of
-// (output, input) channels per block (grid.y): per tap A[co][v] = dy and
+// (output, input) channels per block: per tap A[co][v] = dy and
 // B[v][ci] = the shifted input, K = 32 voxels along w per instruction. Rows
 // sit in LDS as in memory, [voxel][16 channels], and both operands come
 // through the transposing LDS read, so a kw shift is a row offset and
@@ -1150,7 +1150,9 @@ __global__ void k_flip_weights(uint16_t const *__restrict__ wt, uint16_t *__rest
 // registers: one new row of each per step, so a step's nine matrix-core
 // instructions need four operand reads. The rows of the next two steps are in flight during the current one
 // (two register sets, two LDS stages, one barrier per step). A row chunk's
-// three kd are neighbours on one XCD (they read the same dy rows). The sums
+// tile pairs and kd are neighbours on one XCD: they read the same rows, and
+// 32 of the 2 CI bytes of a voxel each (pairs apart: 715 us for 48 -> 16
+// channels). The sums
 // keep one fixed order: a half's rows in turn, the two halves, then the
 // blocks (k_reduce_parts). The partial sums go to part[block][27][CO][CI],
 // the bias's to bpart[block][CO].
@@ -1188,9 +1190,11 @@ __global__ __launch_bounds__(WG_T, 4) void k_conv3_wgrad(
   int const tid = threadIdx.x, lane = tid & 63;
   int const i = lane & 15, kq = lane >> 4;
   int const cs = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (row chunk, input tile, output tile, kd), kd fastest
+  int const nct = CO / 16, nsub = 3 * nct * (CI / 16);
   int const id = xcd_chunk(blockIdx.x, gridDim.x);
-  int const blk = id / 3, kd = id - 3 * blk;
-  int const ct = blockIdx.y % (CO / 16), it = blockIdx.y / (CO / 16);
+  int const blk = id / nsub, sub = id - blk * nsub;
+  int const kd = sub % 3, ct = sub / 3 % nct, it = sub / 3 / nct;
   int const nwc = (W + 63) / 64;
   int const w0 = (blk % nwc) * 64;
   int64_t const r0 = (int64_t)(blk / nwc) * RB;
@@ -1809,7 +1813,8 @@ int agdu_conv3_wgrad(void const *x, void const *dy, float *part, float *dw, floa
   int pairs, rb;
   int64_t nblk;
   if (N < 1 || D < 1 || H < 1 || W < 1 ||
-      !wgrad_plan(N, D, H, W, CI, CO, &pairs, &rb, &nblk) || 3 * nblk > 0x7fffffff) {
+      !wgrad_plan(N, D, H, W, CI, CO, &pairs, &rb, &nblk) ||
+      3 * pairs * nblk > 0x7fffffff) {
     fprintf(stderr, "ERROR: weight gradient for %d -> %d channels, %d x %d x %d x %d "
                     "unsupported\n", CI, CO, N, D, H, W);
     return 1;
@@ -1819,7 +1824,7 @@ int agdu_conv3_wgrad(void const *x, void const *dy, float *part, float *dw, floa
   float *const gw = bpart + nblk * CO;
   int64_t const ng = (nblk + RED_PER - 1) / RED_PER;
   float *const gb = gw + ng * len;
-  if (ulaunch("conv3_wgrad", k_conv3_wgrad, dim3(3 * (unsigned)nblk, (unsigned)pairs), dim3(WG_T),
+  if (ulaunch("conv3_wgrad", k_conv3_wgrad, dim3((unsigned)(3 * pairs * nblk)), dim3(WG_T),
               stream, (uint16_t const *)x, (uint16_t const *)dy, part, db ? bpart : (float *)0, D,
               H, W, CI, CO, (int64_t)N * D * H, rb))
     return 1;
