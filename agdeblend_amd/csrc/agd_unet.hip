@@ -1326,18 +1326,36 @@ __global__ __launch_bounds__(WG_T, 4) void k_conv3_wgrad(
   }
 }
 
-// out[i] = sum_s part[s][i] for s < nslab, in order; grid.y splits the
-// slabs into groups of `per` whose sums go to out[group][i] (a second pass
-// with grid.y = 1 then sums the groups in order)
-__global__ void k_reduce_parts(float const *__restrict__ part, float *__restrict__ out,
-                               int nslab, int len, int per) {
-  int const i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= len) return;
-  int const s0 = blockIdx.y * per;
-  int const s1 = s0 + per < nslab ? s0 + per : nslab;
-  float s = 0.f;
-  for (int k = s0; k < s1; ++k) s += part[(int64_t)k * len + i];
-  out[(int64_t)blockIdx.y * len + i] = s;
+// The blocks' partial sums in a fixed order: groups of RED_PER blocks, each in
+// turn, then the groups in turn. dw: [len] from part [nslab][len]; blocks
+// beyond it: db [co] from bpart [nslab][co]. A block takes 16 outputs, 16
+// groups at a time: one launch per layer instead of four (11 layers of a step:
+// 0.35 ms -> 0.19).
+#define RED_PER 32
+__global__ __launch_bounds__(UT) void k_reduce_parts(float const *__restrict__ part,
+                                                     float *__restrict__ dw, int nslab, int len,
+                                                     float const *__restrict__ bpart,
+                                                     float *__restrict__ db, int co) {
+  __shared__ float sum[16][17];
+  int const wblk = (len + 15) / 16;
+  bool const bias = (int)blockIdx.x >= wblk;
+  int const o = ((int)blockIdx.x - (bias ? wblk : 0)) * 16 + (threadIdx.x & 15);
+  int const n = bias ? co : len, slot = threadIdx.x >> 4;
+  float const *const src = (bias ? bpart : part) + min(o, n - 1);
+  int const ng = (nslab + RED_PER - 1) / RED_PER;
+  float total = 0.f;
+  for (int g0 = 0; g0 < ng; g0 += 16) {
+    int const s0 = (g0 + slot) * RED_PER, s1 = min(s0 + RED_PER, nslab);
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = s0; k < s1; ++k) s += src[(int64_t)k * n];
+    sum[slot][threadIdx.x & 15] = s;
+    __syncthreads();
+    if (slot == 0)
+      for (int g = 0; g < min(16, ng - g0); ++g) total += sum[g][threadIdx.x];
+    __syncthreads();
+  }
+  if (slot == 0 && o < n) (bias ? db : dw)[o] = total;
 }
 
 // ---------------------------------------------------------------------------
@@ -1351,22 +1369,27 @@ typedef uint8_t u8x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ u16x8 ld8(uint16_t const *p) { return *(u16x8 const *)p; }
 __device__ __forceinline__ void st8(uint16_t *p, u16x8 v) { *(u16x8 *)p = v; }
 
+// The training pass's resampling kernels take one (n, d, h) row of their
+// output per block: the row's indices are divided out once, a thread only
+// splits its (w, 8 channels), in 32 bits (64-bit divisions per 16 bytes had
+// these kernels at 1.5 TB/s).
+struct Row {
+  int n, d, h;
+};
+__device__ __forceinline__ Row out_row(int D, int H) {
+  int const r = blockIdx.x, nd = r / H;
+  return Row{nd / D, nd % D, r - nd * H};
+}
+
 // 2x2x2 max pool: y[n][d][h][w][c] over x[n][2d..][2h..][2w..][c]; arg holds
-// the winning offset (first maximum in (a, b, e) order)
+// the winning offset (first maximum in (a, b, e) order). D, H, W: of y
 __global__ void k_maxpool(uint16_t const *__restrict__ x, uint16_t *__restrict__ y,
-                          uint8_t *__restrict__ arg, int N, int D, int H, int W, int C) {
-  int const Do = D / 2, Ho = H / 2, Wo = W / 2, C8 = C / 8;
-  int64_t const total = (int64_t)N * Do * Ho * Wo * C8;
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    int const c = (int)(idx % C8) * 8;
-    int64_t r = idx / C8;
-    int const w = (int)(r % Wo);
-    r /= Wo;
-    int const h = (int)(r % Ho);
-    r /= Ho;
-    int const d = (int)(r % Do);
-    int const n = (int)(r / Do);
+                          uint8_t *__restrict__ arg, int D, int H, int W, int C) {
+  Row const r = out_row(D, H);
+  int const C8 = C / 8;
+  int64_t const out0 = (int64_t)blockIdx.x * W * C;
+  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
+    int const w = idx / C8, c = (idx - w * C8) * 8;
     float best[8];
     int barg[8];
 #pragma unroll
@@ -1377,8 +1400,8 @@ __global__ void k_maxpool(uint16_t const *__restrict__ x, uint16_t *__restrict__
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
       int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
-      u16x8 const v =
-          ld8(x + ((((int64_t)n * D + 2 * d + a) * H + 2 * h + b) * W + 2 * w + e) * C + c);
+      int64_t const row = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
+      u16x8 const v = ld8(x + (row * 2 * W + 2 * w + e) * C + c);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         float const f = bf2f(v[k]);
@@ -1395,35 +1418,51 @@ __global__ void k_maxpool(uint16_t const *__restrict__ x, uint16_t *__restrict__
       out[k] = f2bf(best[k]);
       ar[k] = (uint8_t)barg[k];
     }
-    st8(y + idx * 8, out);
-    *(u8x8 *)(arg + idx * 8) = ar;
+    st8(y + out0 + (int64_t)idx * 8, out);
+    *(u8x8 *)(arg + out0 + (int64_t)idx * 8) = ar;
   }
 }
 
-// one thread per 8 channels of an input voxel
+// gradient of the pooling, D, H, W: of dx. add (or NULL): a second gradient of
+// the pooled tensor's input, its channels [c0, c0 + C) of Ca, added in fp32 and
+// rounded once (as k_copy_channels mode 1 on the written dx)
 __global__ void k_maxpool_bwd(uint16_t const *__restrict__ dy, uint8_t const *__restrict__ arg,
-                              uint16_t *__restrict__ dx, int N, int D, int H, int W, int C) {
+                              uint16_t *__restrict__ dx, int D, int H, int W, int C,
+                              uint16_t const *__restrict__ add, int Ca, int c0) {
+  Row const r = out_row(D, H);
   int const C8 = C / 8;
-  int64_t const total = (int64_t)N * D * H * W * C8;
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    int const c = (int)(idx % C8) * 8;
-    int64_t r = idx / C8;
-    int const w = (int)(r % W);
-    r /= W;
-    int const h = (int)(r % H);
-    r /= H;
-    int const d = (int)(r % D);
-    int const n = (int)(r / D);
-    int const Do = D / 2, Ho = H / 2, Wo = W / 2;
-    int64_t const o = ((((int64_t)n * Do + d / 2) * Ho + h / 2) * Wo + w / 2) * C + c;
-    int const mine = ((d & 1) << 2) | ((h & 1) << 1) | (w & 1);
+  int64_t const prow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
+  int const mine = ((r.d & 1) << 2) | ((r.h & 1) << 1);
+  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
+    int const w = idx / C8, c = (idx - w * C8) * 8;
+    int64_t const o = (prow * (W / 2) + w / 2) * C + c;
     u16x8 const g = ld8(dy + o);
     u8x8 const a = *(u8x8 const *)(arg + o);
     u16x8 out;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) out[k] = a[k] == mine ? g[k] : (uint16_t)0;
-    st8(dx + idx * 8, out);
+    for (int k = 0; k < 8; ++k) out[k] = a[k] == (mine | (w & 1)) ? g[k] : (uint16_t)0;
+    if (add != nullptr) {
+      u16x8 const s = ld8(add + ((int64_t)blockIdx.x * W + w) * Ca + c0 + c);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) out[k] = f2bf(bf2f(s[k]) + bf2f(out[k]));
+    }
+    st8(dx + ((int64_t)blockIdx.x * W + w) * C + c, out);
+  }
+}
+
+// y = [upsample(xu), xs]: the nearest x2 upsampling of xu (CU channels) and xs
+// (CS channels) side by side, whole voxels of y [n][D][H][W][CU + CS] at a time
+__global__ void k_concat_up(uint16_t const *__restrict__ xu, uint16_t const *__restrict__ xs,
+                            uint16_t *__restrict__ y, int D, int H, int W, int CU, int CS) {
+  Row const r = out_row(D, H);
+  int const C8 = (CU + CS) / 8;
+  int64_t const urow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
+  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
+    int const w = idx / C8, c = (idx - w * C8) * 8;
+    uint16_t const *const q = c < CU
+                                  ? xu + (urow * (W / 2) + w / 2) * CU + c
+                                  : xs + ((int64_t)blockIdx.x * W + w) * CS + (c - CU);
+    st8(y + (int64_t)blockIdx.x * W * (CU + CS) + (int64_t)idx * 8, ld8(q));
   }
 }
 
@@ -1449,36 +1488,28 @@ __global__ void k_upsample(uint16_t const *__restrict__ x, uint16_t *__restrict_
 }
 
 // gradient of the upsampling: dx[v][c] = sum of the 8 children's
-// dy[..][c0 + c], in a fixed order; accumulated in fp32
-__global__ void k_upsample_bwd(uint16_t const *__restrict__ dy, uint16_t *__restrict__ dx,
-                               int N, int D, int H, int W, int C, int Cy, int c0) {
+// dy[..][c0 + c], in a fixed order; accumulated in fp32. D, H, W: of dx
+__global__ void k_upsample_bwd(uint16_t const *__restrict__ dy, uint16_t *__restrict__ dx, int D,
+                               int H, int W, int C, int Cy, int c0) {
+  Row const r = out_row(D, H);
   int const C8 = C / 8;
-  int64_t const total = (int64_t)N * D * H * W * C8;
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    int const c = (int)(idx % C8) * 8;
-    int64_t r = idx / C8;
-    int const w = (int)(r % W);
-    r /= W;
-    int const h = (int)(r % H);
-    r /= H;
-    int const d = (int)(r % D);
-    int const n = (int)(r / D);
+  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
+    int const w = idx / C8, c = (idx - w * C8) * 8;
     float s[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) s[k] = 0.f;
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
       int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
-      u16x8 const g = ld8(dy + ((((int64_t)n * 2 * D + 2 * d + a) * 2 * H + 2 * h + b) * 2 * W +
-                                2 * w + e) * Cy + c0 + c);
+      int64_t const row = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
+      u16x8 const g = ld8(dy + (row * 2 * W + 2 * w + e) * Cy + c0 + c);
 #pragma unroll
       for (int k = 0; k < 8; ++k) s[k] += bf2f(g[k]);
     }
     u16x8 out;
 #pragma unroll
     for (int k = 0; k < 8; ++k) out[k] = f2bf(s[k]);
-    st8(dx + idx * 8, out);
+    st8(dx + (int64_t)blockIdx.x * W * C + (int64_t)idx * 8, out);
   }
 }
 
@@ -1546,8 +1577,17 @@ __global__ __launch_bounds__(UT) void k_l2_loss(uint16_t const *__restrict__ y,
   if (v < nvox) {
     float const e = bf2f(y[v * C]) - t[v] * tscale;
     e2 = e * e;
-    dy[v * C] = f2bf(2.f * e / (float)nvox);
-    for (int c = 1; c < C; ++c) dy[v * C + c] = 0;
+    uint16_t const g = f2bf(2.f * e / (float)nvox);
+    if (C % 8 == 0) {
+      u16x8 o = {g, 0, 0, 0, 0, 0, 0, 0};
+      for (int c = 0; c < C; c += 8) {
+        st8(dy + v * C + c, o);
+        o[0] = 0;
+      }
+    } else {
+      dy[v * C] = g;
+      for (int c = 1; c < C; ++c) dy[v * C + c] = 0;
+    }
   }
   red[threadIdx.x] = e2;
   __syncthreads();
@@ -1598,6 +1638,20 @@ static inline int64_t blocks_for(int64_t n, int t) { return (n + t - 1) / t; }
 static inline int64_t blocks_capped(int64_t n, int t) {
   int64_t const b = blocks_for(n, t);
   return b < (1 << 20) ? b : (1 << 20);
+}
+
+// a kernel with one block per (n, d, h) row of `items` 16-byte items
+template <typename K, typename... A>
+static int row_launch(char const *name, K kernel, int N, int D, int H, int64_t items,
+                      void *stream, A... args) {
+  int64_t const rows = (int64_t)N * D * H;
+  if (rows > 0x7fffffff || items > 0x7fffffff / 2) {
+    fprintf(stderr, "ERROR: %s of %lld rows of %lld items unsupported\n", name, (long long)rows,
+            (long long)items);
+    return 1;
+  }
+  int const t = items >= UT ? UT : (int)((items + 63) / 64 * 64);
+  return ulaunch(name, kernel, dim3((unsigned)rows), dim3(t > 0 ? t : 64), stream, args...);
 }
 
 extern "C" {
@@ -1798,8 +1852,6 @@ static int wgrad_plan(int N, int D, int H, int W, int CI, int CO, int *pairs, in
   return 1;
 }
 
-#define RED_PER 32
-
 int64_t agdu_wgrad_part_len(int N, int D, int H, int W, int CI, int CO) {
   int pairs, rb;
   int64_t nblk;
@@ -1821,26 +1873,13 @@ int agdu_conv3_wgrad(void const *x, void const *dy, float *part, float *dw, floa
   }
   int const len = 27 * CI * CO;
   float *const bpart = part + nblk * len;
-  float *const gw = bpart + nblk * CO;
-  int64_t const ng = (nblk + RED_PER - 1) / RED_PER;
-  float *const gb = gw + ng * len;
   if (ulaunch("conv3_wgrad", k_conv3_wgrad, dim3((unsigned)(3 * pairs * nblk)), dim3(WG_T),
               stream, (uint16_t const *)x, (uint16_t const *)dy, part, db ? bpart : (float *)0, D,
               H, W, CI, CO, (int64_t)N * D * H, rb))
     return 1;
-  // two-level fixed-order sums over the blocks
-  if (ulaunch("reduce_parts", k_reduce_parts, dim3((unsigned)blocks_for(len, UT), (unsigned)ng),
-              dim3(UT), stream, (float const *)part, gw, (int)nblk, len, RED_PER) ||
-      ulaunch("reduce_parts", k_reduce_parts, dim3((unsigned)blocks_for(len, UT), 1), dim3(UT),
-              stream, (float const *)gw, dw, (int)ng, len, (int)ng))
-    return 1;
-  if (db == NULL) return 0;
-  if (ulaunch("reduce_parts", k_reduce_parts, dim3((unsigned)blocks_for(CO, UT), (unsigned)ng),
-              dim3(UT), stream, (float const *)bpart, gb, (int)nblk, CO, RED_PER) ||
-      ulaunch("reduce_parts", k_reduce_parts, dim3((unsigned)blocks_for(CO, UT), 1), dim3(UT),
-              stream, (float const *)gb, db, (int)ng, CO, (int)ng))
-    return 1;
-  return 0;
+  return ulaunch("reduce_parts", k_reduce_parts,
+                 dim3((unsigned)((len + 15) / 16 + (db ? CO / 16 : 0))), dim3(UT), stream,
+                 (float const *)part, dw, (int)nblk, len, (float const *)bpart, db, CO);
 }
 
 int agdu_maxpool(void const *x, void *y, void *arg, int N, int D, int H, int W, int C,
@@ -1853,13 +1892,12 @@ int agdu_maxpool(void const *x, void *y, void *arg, int N, int D, int H, int W, 
     fprintf(stderr, "ERROR: channel count %d is not a multiple of 8\n", C);
     return 1;
   }
-  int64_t const total = (int64_t)N * (D / 2) * (H / 2) * (W / 2) * (C / 8);
-  return ulaunch("maxpool", k_maxpool, dim3((unsigned)blocks_capped(total, UT)), dim3(UT),
-                 stream, (uint16_t const *)x, (uint16_t *)y, (uint8_t *)arg, N, D, H, W, C);
+  return row_launch("maxpool", k_maxpool, N, D / 2, H / 2, (W / 2) * (int64_t)(C / 8), stream,
+                    (uint16_t const *)x, (uint16_t *)y, (uint8_t *)arg, D / 2, H / 2, W / 2, C);
 }
 
-int agdu_maxpool_bwd(void const *dy, void const *arg, void *dx, int N, int D, int H, int W,
-                     int C, void *stream) {
+int agdu_maxpool_bwd_add(void const *dy, void const *arg, void const *add, int Ca, int c0,
+                         void *dx, int N, int D, int H, int W, int C, void *stream) {
   if ((D | H | W) & 1) {
     fprintf(stderr, "ERROR: max pooling needs even sizes, got %d x %d x %d\n", D, H, W);
     return 1;
@@ -1868,10 +1906,32 @@ int agdu_maxpool_bwd(void const *dy, void const *arg, void *dx, int N, int D, in
     fprintf(stderr, "ERROR: channel count %d is not a multiple of 8\n", C);
     return 1;
   }
-  int64_t const total = (int64_t)N * D * H * W * (C / 8);
-  return ulaunch("maxpool_bwd", k_maxpool_bwd, dim3((unsigned)blocks_capped(total, UT)),
-                 dim3(UT), stream, (uint16_t const *)dy, (uint8_t const *)arg,
-                 (uint16_t *)dx, N, D, H, W, C);
+  if (add != NULL && ((Ca | c0) % 8 || c0 < 0 || c0 + C > Ca)) {
+    fprintf(stderr, "ERROR: added channels %d at %d of %d unsupported\n", C, c0, Ca);
+    return 1;
+  }
+  return row_launch("maxpool_bwd", k_maxpool_bwd, N, D, H, W * (int64_t)(C / 8), stream,
+                    (uint16_t const *)dy, (uint8_t const *)arg, (uint16_t *)dx, D, H, W, C,
+                    (uint16_t const *)add, Ca, c0);
+}
+
+int agdu_maxpool_bwd(void const *dy, void const *arg, void *dx, int N, int D, int H, int W,
+                     int C, void *stream) {
+  return agdu_maxpool_bwd_add(dy, arg, NULL, 0, 0, dx, N, D, H, W, C, stream);
+}
+
+int agdu_concat_up(void const *xu, void const *xs, void *y, int N, int D, int H, int W, int CU,
+                   int CS, void *stream) {
+  if ((D | H | W) & 1) {
+    fprintf(stderr, "ERROR: upsampling needs even sizes, got %d x %d x %d\n", D, H, W);
+    return 1;
+  }
+  if ((CU | CS) % 8) {
+    fprintf(stderr, "ERROR: concatenating %d and %d channels unsupported\n", CU, CS);
+    return 1;
+  }
+  return row_launch("concat_up", k_concat_up, N, D, H, W * (int64_t)((CU + CS) / 8), stream,
+                    (uint16_t const *)xu, (uint16_t const *)xs, (uint16_t *)y, D, H, W, CU, CS);
 }
 
 int agdu_upsample(void const *x, void *y, int N, int D, int H, int W, int C, int Cy, int c0,
@@ -1892,9 +1952,8 @@ int agdu_upsample_bwd(void const *dy, void *dx, int N, int D, int H, int W, int 
     return 1;
   }
   int64_t const total = (int64_t)N * D * H * W * (C / 8);
-  return ulaunch("upsample_bwd", k_upsample_bwd, dim3((unsigned)blocks_capped(total, UT)),
-                 dim3(UT), stream, (uint16_t const *)dy, (uint16_t *)dx, N, D, H, W, C, Cy,
-                 c0);
+  return row_launch("upsample_bwd", k_upsample_bwd, N, D, H, W * (int64_t)(C / 8), stream,
+                    (uint16_t const *)dy, (uint16_t *)dx, D, H, W, C, Cy, c0);
 }
 
 int agdu_copy_channels(void const *x, void *y, int64_t nvox, int Cx, int cx0, int Cy,

@@ -107,6 +107,8 @@ def load():
     fn("agdu_conv3_wgrad", ci, vp, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci, vp)
     fn("agdu_maxpool", ci, vp, vp, vp, ci, ci, ci, ci, ci, vp)
     fn("agdu_maxpool_bwd", ci, vp, vp, vp, ci, ci, ci, ci, ci, vp)
+    fn("agdu_maxpool_bwd_add", ci, vp, vp, vp, ci, ci, vp, ci, ci, ci, ci, ci, vp)
+    fn("agdu_concat_up", ci, vp, vp, vp, ci, ci, ci, ci, ci, ci, vp)
     fn("agdu_upsample", ci, vp, vp, ci, ci, ci, ci, ci, ci, ci, vp)
     fn("agdu_upsample_bwd", ci, vp, vp, ci, ci, ci, ci, ci, ci, ci, vp)
     fn("agdu_copy_channels", ci, vp, vp, i64, ci, ci, ci, ci, ci, ci, vp, vp)
@@ -138,7 +140,8 @@ EXPORTS = ["agd_deblend", "agd_blend", "agdeblend_deblend", "agdeblend_blend", "
            "agdx_timing_get", "agdx_bytes",
            "agdu_conv3", "agdu_conv3_pool", "agdu_conv3_cat", "agdu_up_weights", "agdu_conv3_up", "agdu_conv_in", "agdu_conv_out",
            "agdu_flip_weights", "agdu_wgrad_part_len", "agdu_conv3_wgrad",
-           "agdu_maxpool", "agdu_maxpool_bwd", "agdu_upsample",
+           "agdu_maxpool", "agdu_maxpool_bwd", "agdu_maxpool_bwd_add", "agdu_concat_up",
+           "agdu_upsample",
            "agdu_upsample_bwd", "agdu_copy_channels", "agdu_pack_input",
            "agdu_unpack_output", "agdu_l2_loss", "agdu_loss_parts", "agdu_adam",
            "agdu_to_bf16", "agdu_from_bf16"]

@@ -206,17 +206,12 @@ class UNet:
                "agdu_maxpool")
         self._conv("b1", B["p2"], B["b1"], d2, 3)
         self._conv("b2", B["b1"], B["b2"], d2, 3)
-        _check(self.L.agdu_upsample(_vp(B["b2"]), _vp(B["c2"]), *d2, 64, 96, 0, s),
-               "agdu_upsample")
-        nv1 = nvox // 8
-        _check(self.L.agdu_copy_channels(_vp(B["e2b"]), _vp(B["c2"]), nv1, 32, 0, 96, 64, 32, 0,
-                                         None, s), "agdu_copy_channels")
+        _check(self.L.agdu_concat_up(_vp(B["b2"]), _vp(B["e2b"]), _vp(B["c2"]), *d1, 64, 32, s),
+               "agdu_concat_up")
         self._conv("d2a", B["c2"], B["d2a"], d1, 3)
         self._conv("d2b", B["d2a"], B["d2b"], d1, 3)
-        _check(self.L.agdu_upsample(_vp(B["d2b"]), _vp(B["c1"]), *d1, 32, 48, 0, s),
-               "agdu_upsample")
-        _check(self.L.agdu_copy_channels(_vp(B["e1b"]), _vp(B["c1"]), nvox, 16, 0, 48, 32, 16,
-                                         0, None, s), "agdu_copy_channels")
+        _check(self.L.agdu_concat_up(_vp(B["d2b"]), _vp(B["e1b"]), _vp(B["c1"]), *d0, 32, 16, s),
+               "agdu_concat_up")
         self._conv("d1a", B["c1"], B["d1a"], d0, 3)
         self._conv("d1b", B["d1a"], B["d1b"], d0, 3)
         self._conv("head", B["d1b"], B["head"], d0, 1)
@@ -351,16 +346,12 @@ class UNet:
         self._layer_bwd("b2", B["b1"], B["gq64a"], d2, B["gq64b"], B["b1"])
         self._layer_bwd("b1", B["p2"], B["gq64b"], d2, B["gq32"], B["p2"])
         # e2b's output gradient: pooled path plus the skip connection
-        _check(self.L.agdu_maxpool_bwd(_vp(B["gq32"]), _vp(B["a2"]), _vp(B["gh32a"]), *d1, 32, s),
-               "agdu_maxpool_bwd")
-        _check(self.L.agdu_copy_channels(_vp(B["gh96"]), _vp(B["gh32a"]), nvox // 8, 96, 64, 32,
-                                         0, 32, 1, None, s), "agdu_copy_channels")
+        _check(self.L.agdu_maxpool_bwd_add(_vp(B["gq32"]), _vp(B["a2"]), _vp(B["gh96"]), 96, 64,
+                                           _vp(B["gh32a"]), *d1, 32, s), "agdu_maxpool_bwd_add")
         self._layer_bwd("e2b", B["e2a"], B["gh32a"], d1, B["gh32b"], B["e2a"])
         self._layer_bwd("e2a", B["p1"], B["gh32b"], d1, B["gh16"], B["p1"])
-        _check(self.L.agdu_maxpool_bwd(_vp(B["gh16"]), _vp(B["a1"]), _vp(g16b), *d0, 16, s),
-               "agdu_maxpool_bwd")
-        _check(self.L.agdu_copy_channels(_vp(g48), _vp(g16b), nvox, 48, 32, 16, 0, 16, 1, None,
-                                         s), "agdu_copy_channels")
+        _check(self.L.agdu_maxpool_bwd_add(_vp(B["gh16"]), _vp(B["a1"]), _vp(g48), 48, 32,
+                                           _vp(g16b), *d0, 16, s), "agdu_maxpool_bwd_add")
         self._layer_bwd("e1b", B["e1a"], g16b, d0, g16a, B["e1a"])
         self._layer_bwd("e1a", B["x"], g16a, d0)
         self.step_count += 1

@@ -74,6 +74,14 @@ int agdu_maxpool(void const *x, void *y, void *arg, int N, int D, int H, int W, 
                  void *stream);
 int agdu_maxpool_bwd(void const *dy, void const *arg, void *dx, int N, int D, int H, int W,
                      int C, void *stream);
+/* agdu_maxpool_bwd plus a second gradient of the same tensor: channels
+ * [c0, c0 + C) of the Ca-channel add, summed in fp32 and rounded once */
+int agdu_maxpool_bwd_add(void const *dy, void const *arg, void const *add, int Ca, int c0,
+                         void *dx, int N, int D, int H, int W, int C, void *stream);
+/* y = [upsample(xu), xs]: xu [N][D/2][H/2][W/2][CU] (nearest x2 upsampling;
+ * D, H, W even), xs [N][D][H][W][CS], y [N][D][H][W][CU + CS] */
+int agdu_concat_up(void const *xu, void const *xs, void *y, int N, int D, int H, int W, int CU,
+                   int CS, void *stream);
 /* nearest x2 upsampling into channels [c0, c0 + C) of a Cy-channel tensor */
 int agdu_upsample(void const *x, void *y, int N, int D, int H, int W, int C, int Cy, int c0,
                   void *stream);
