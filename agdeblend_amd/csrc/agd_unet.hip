@@ -19,6 +19,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <type_traits>
+
 #include "agd_launch.h"
 #include "agdeblend_unet.h"
 
@@ -115,6 +117,27 @@ __device__ __forceinline__ void st_h(uint16_t *base, int row, int half, uint4 v)
   *(uint4 *)(base + swz_h(row, half)) = v;
 }
 
+// byte offset of half `half` of row `row` (swz_h); adding a multiple of 8
+// rows moves it by 32 bytes a row
+__device__ __forceinline__ int off_h(int row, int half) {
+  return row * 32 + ((half ^ ((row >> 2) & 1)) << 4);
+}
+__device__ __forceinline__ u32x4 ld_b(uint16_t const *base, int bytes) {
+  return *(u32x4 const *)((char const *)base + bytes);
+}
+// four output channels of a voxel as bf16 (bias added; ReLU)
+template <bool RELU>
+__device__ __forceinline__ uint2 out4(f32x4 a, f32x4 b) {
+  float v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    v[r] = a[r] + b[r];
+    if (RELU) v[r] = fmaxf(v[r], 0.f);
+  }
+  return make_uint2((uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
+                    (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+}
+
 template <int CO, int CU, bool UPC = false>
 struct ConvDepth {
   // depth planes per block: the ring saves input reads, the accumulators
@@ -166,7 +189,7 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
   constexpr int NPI = PH * PW * 2;     // staging items (8 channels) per plane
   constexpr int NWI = 27 * CO * 2;
   constexpr int NWU = 48 * CO * 2;     // staging items of the combined taps
-  constexpr int NTW = UPC ? 48 : 27;   // taps the weight region holds
+  constexpr int NTW = UPC ? 48 : 28;   // taps the weight region holds (the 28th zero)
   constexpr int OBS = CO + 4;  // output staging row: CO channels + 4 (bank spread)
   // output staging: 4 x 64 rows of OBS, then the pooling partials [2][32][CO]
   constexpr int OSM = 4 * 64 * OBS + 2 * 32 * CO;
@@ -182,8 +205,36 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
   int const d0 = (blockIdx.z - n * ndb) * DB;
   int const h0 = blockIdx.y * CT_H;
   int const w0 = blockIdx.x * CT_W;
-  int const i = lane & 15;   // A row: voxel; B / D column: channel in the tile
+  // The weights are the matrix-core instruction's A operand and the voxels its
+  // B, so that a lane ends with four neighbouring output channels of one
+  // voxel: one 8-byte LDS write in the epilogue instead of four of 2.
+  int const i = lane & 15;   // channel in the tile (weights), voxel (input, output)
   int const kq = lane >> 4;  // k group: channels 8 (kq & 1) .. + 7 of the step's tap kq >> 1
+  // LDS byte offsets of the lane's operands, built once: the loop over the
+  // taps then adds constants only. (Built at each step they were most of the
+  // 6.4 vector instructions per matrix-core one, whose issue bounds these
+  // layers: 96 -> 32 at 32 x 128 x 1024 960 us, now 846; the network on
+  // 64 x 256 x 2048 5.04 ms, now 4.51; a step on 16 patches of 32 x 32 x 256
+  // 4.19 ms, now 3.96.) Input: step st's tap 2 st + (kq >> 1) (the
+  // 28th reads the 27th's voxels, with zero weights) within a plane of the
+  // ring; weights: bof + 32 CO tap.
+  constexpr int PLANEB = PH * PW * 32;
+  constexpr bool STREAM = UPC && DB >= 4;
+  constexpr int NST = STREAM ? 5 : 14;  // steps: positions of a plane, or taps
+  int const hi = kq >> 1;
+  int aof[NST];
+#pragma unroll
+  for (int st = 0; st < NST; ++st) {
+    int const tl = 2 * st + hi, last = STREAM ? 8 : 26;
+    int const t = (tl < last ? tl : last) % 9;
+    aof[st] = off_h((wave + t / 3) * PW + i + t % 3, kq & 1);
+  }
+  int const bof = off_h(i, kq & 1) + hi * CO * 32;
+  // ring slots (bytes) of the planes d0, d0 + 1, d0 + 2 modulo 3
+  int const slot[3] = {d0 % 3 * PLANEB, (d0 + 1) % 3 * PLANEB, (d0 + 2) % 3 * PLANEB};
+  if constexpr (!STREAM)  // the 28th tap (the combined taps come after it)
+    for (int e = tid; e < CO * 2; e += UT)
+      *(uint4 *)(sw + 27 * CO * 16 + e * 8) = make_uint4(0, 0, 0, 0);
   f32x4 acc[DB][4][NT];
 #pragma unroll
   for (int j = 0; j < DB; ++j)
@@ -335,7 +386,14 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
         __syncthreads();
         if (c + 1 < CU / 16) load_coarse(c + 1);
         __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the compute
-        int const ph = (h0 + wave) & 1;
+        int const bofu = bof + ((h0 + wave) & 1) * 12 * CO * 32;
+        static_assert(CPH * CPW % 8 == 0, "planes at whole swizzle periods");
+        int cof[3];
+#pragma unroll
+        for (int sp = 0; sp < 3; ++sp) {
+          int const u = 2 * sp + hi, b = u / 3, kw = u - 3 * b;
+          cof[sp] = off_h(((wave + 1) / 2 + b) * CPW + 1 + ((i + kw - 1) >> 1), kq & 1);
+        }
         // Streamed over the staged coarse planes: fine plane j (parity j & 1,
         // d0 even) reads coarse plane (j + 1) / 2 + a with its d-combination
         // a, so coarse plane cp feeds fine planes 2 (cp - a) - 1 and
@@ -349,12 +407,12 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
         for (int cp = 0; cp < CPD; ++cp) {
 #pragma unroll
           for (int sp = 0; sp < 3; ++sp) {
-            int const u = 2 * sp + (kq >> 1);  // (b, kw) position of this lane
-            int const b = u / 3, kw = u - 3 * b;
-            int const v0 = (cp * CPH + (wave + 1) / 2 + b) * CPW + 1;
+            // (b, kw) position 2 sp + hi of this lane: combined tap
+            // (pd 2 + ph) 12 + a 6 + position
             u32x4 a4[4];
 #pragma unroll
-            for (int m = 0; m < 4; ++m) a4[m] = ld_h(sx, v0 + ((16 * m + i + kw - 1) >> 1), kq & 1);
+            for (int m = 0; m < 4; ++m)
+              a4[m] = ld_b(sx, cof[sp] + cp * CPH * CPW * 32 + m * 8 * 32);
 #pragma unroll
             for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -364,9 +422,10 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
                   int const pd = j & 1;
 #pragma unroll
                   for (int t = 0; t < NT; ++t) {
-                    u32x4 const bt = ld_h(sw, up_tap(pd, ph, a, b, kw) * CO + t * 16 + i, kq & 1);
+                    u32x4 const bt =
+                        ld_b(sw, bofu + (pd * 24 + a * 6 + 2 * sp) * CO * 32 + t * 512);
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) acc[j][m][t] = mfma32(a4[m], bt, acc[j][m][t]);
+                    for (int m = 0; m < 4; ++m) acc[j][m][t] = mfma32(bt, a4[m], acc[j][m][t]);
                   }
                 }
               }
@@ -386,7 +445,7 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
     // done (in the last plane steps), so that waiting for a plane never
     // waits for them
     bool const pre = PRE && c + 1 < CI / 16;
-    if constexpr (UPC && DB >= 4) {
+    if constexpr (STREAM) {
       // The x channels of d1a streamed over the input planes p = d0 - 1 ..
       // d0 + DB (in ring slot (p + 3) % 3): each A fragment (plane p, two
       // (kh, kw) positions of step s) is read once and used for the output
@@ -396,7 +455,6 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
 #pragma unroll
       for (int jp = 0; jp < DB + 2; ++jp) {
         int const p = d0 - 1 + jp;
-        uint16_t const *const pl = sx + ((p + 3) % 3) * PLANE;
         uint4 nxt[NPK];
         bool const more = jp + 3 < DB + 2;  // plane p + 3 still an input
         if (more)
@@ -408,23 +466,22 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
         __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the compute
 #pragma unroll
         for (int st = 0; st < 5; ++st) {
-          int const q = 2 * st + (kq >> 1);
-          int const qq = q < 9 ? q : 8;
-          int const kh = qq / 3, kw = qq - 3 * kh;
-          unsigned const keep = q < 9 ? ~0u : 0u;
-          int const v0 = (wave + kh) * PW + i + kw;
+          // position 2 st + hi; past the ninth: its voxels, zero weights
+          unsigned const keep = st < 4 || hi == 0 ? ~0u : 0u;
           u32x4 a4[4];
 #pragma unroll
-          for (int m = 0; m < 4; ++m) a4[m] = ld_h(pl, v0 + 16 * m, kq & 1);
+          for (int m = 0; m < 4; ++m)
+            a4[m] = ld_b(sx, slot[(jp + 2) % 3] + aof[st] + m * 512);
 #pragma unroll
           for (int kd = 0; kd < 3; ++kd) {
             int const oi = jp - kd;  // output plane d0 + oi = p + 1 - kd
             if (oi >= 0 && oi < DB) {
 #pragma unroll
               for (int tt = 0; tt < NT; ++tt) {
-                u32x4 const bt = ld_h(sw, (kd * 9 + qq) * CO + tt * 16 + i, kq & 1) & keep;
+                u32x4 bt = ld_b(sw, bof + (kd * 9 + 2 * st) * CO * 32 + tt * 512);
+                if (st == 4) bt = bt & keep;
 #pragma unroll
-                for (int m = 0; m < 4; ++m) acc[oi][m][tt] = mfma32(a4[m], bt, acc[oi][m][tt]);
+                for (int m = 0; m < 4; ++m) acc[oi][m][tt] = mfma32(bt, a4[m], acc[oi][m][tt]);
               }
             }
           }
@@ -450,30 +507,31 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
       else if (UPC && c + 1 == CI / 16)
         load_coarse(0);
       __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the compute
-      // operands of step st: this lane's tap 2 st + (kq >> 1) (the 28th,
-      // past the last, reads tap 26 with zero weights), double-buffered so
-      // the LDS reads of the next step overlap this step's MFMAs
+      // operands of step st (taps 2 st, 2 st + 1), double-buffered so the
+      // LDS reads of the next step overlap this step's MFMAs
+      // (the slots pass through an empty asm: their sums with aof, 42 of them,
+      // must not be kept over the planes and chunks, which spilled)
+      int sl[3] = {slot[(j + 2) % 3], slot[j % 3], slot[(j + 1) % 3]};
+#pragma unroll
+      for (int q = 0; q < 3; ++q) asm volatile("" : "+s"(sl[q]));
       auto load_ops = [&](int st, Ops &o) {
-        int const tl = 2 * st + (kq >> 1);
-        int const t = tl < 27 ? tl : 26;
-        int const kd = t / 9, kh = t / 3 - 3 * kd, kw = t - 3 * (t / 3);
-        uint16_t const *const pl = sx + ((d + kd - 1 + 3) % 3) * PLANE;
-        int const v0 = (wave + kh) * PW + i + kw;
-        unsigned const keep = tl < 27 ? ~0u : 0u;
+        int const kd0 = 2 * st / 9, kd1 = 2 * st + 1 < 27 ? (2 * st + 1) / 9 : 2;
+        int const s0 = sl[kd0], s1 = sl[kd1];
+        int const ab = aof[st] + (kd0 == kd1 ? s0 : hi ? s1 : s0);
 #pragma unroll
-        for (int m = 0; m < 4; ++m) o.a[m] = ld_h(pl, v0 + 16 * m, kq & 1);
+        for (int m = 0; m < 4; ++m) o.a[m] = ld_b(sx, ab + m * 512);
 #pragma unroll
-        for (int tt = 0; tt < NT; ++tt) o.b[tt] = ld_h(sw, t * CO + tt * 16 + i, kq & 1) & keep;
+        for (int tt = 0; tt < NT; ++tt) o.b[tt] = ld_b(sw, bof + 2 * st * CO * 32 + tt * 512);
       };
       auto mma_ops = [&](Ops const &o) {
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-          for (int m = 0; m < 4; ++m) acc[j][m][tt] = mfma32(o.a[m], o.b[tt], acc[j][m][tt]);
+          for (int m = 0; m < 4; ++m) acc[j][m][tt] = mfma32(o.b[tt], o.a[m], acc[j][m][tt]);
       };
       Ops opa, opb;
       load_ops(0, opa);
-#pragma unroll 1
+#pragma unroll
       for (int st = 1; st < 14; st += 2) {
         load_ops(st, opb);
         mma_ops(opa);
@@ -489,28 +547,30 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
   }
   coarse_part();
   // Epilogue per plane: each wave writes its row (bias, ReLU applied) into
-  // its own LDS rows [voxel][OBS] (lane (i, kq) holds voxels 4 kq + r of
-  // channel t * 16 + i; the row padding puts the four kq groups in distinct
-  // banks), then stores 16-byte pieces of 8 channels, coalesced.
+  // its own LDS rows [voxel][OBS] (lane (i, kq) holds channels t * 16 + 4 kq
+  // + r of voxel 16 m + i; padded rows spread the banks), then stores 16-byte
+  // pieces of 8 channels, coalesced.
   int const h = h0 + wave;
   uint16_t *const ob = smem + wave * 64 * OBS;
 #pragma unroll
   for (int j = 0; j < DB; ++j) {
     int const d = d0 + j;
     __syncthreads();  // the LDS is free (j = 0: done with the operands)
+    auto rows = [&](auto relu) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      int const co = t * 16 + i;
-      float const b = (mode & 1) ? bias[co] : 0.f;
+      for (int t = 0; t < NT; ++t) {
+        f32x4 const b = (mode & 1) ? *(f32x4 const *)(bias + t * 16 + 4 * kq)
+                                   : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float v = acc[j][m][t][r] + b;
-          if (mode & 2) v = fmaxf(v, 0.f);
-          ob[(16 * m + 4 * kq + r) * OBS + co] = f2bf(v);
-        }
-    }
+        for (int m = 0; m < 4; ++m)
+          *(uint2 *)(ob + (16 * m + i) * OBS + t * 16 + 4 * kq) =
+              out4<decltype(relu)::value>(acc[j][m][t], b);
+      }
+    };
+    if (mode & 2)
+      rows(std::true_type{});
+    else
+      rows(std::false_type{});
     __syncthreads();
     if (h < H && d < D) {
       int64_t const orow = (((int64_t)n * D + d) * H + h) * W;
@@ -638,7 +698,9 @@ __global__ __launch_bounds__(UT, 2) void k_conv3s(uint16_t const *__restrict__ x
   int const d0 = (blockIdx.z - n * ndb) * DB;
   int const h0 = blockIdx.y * CT_H;
   int const w0 = blockIdx.x * CT_W;
-  int const i = lane & 15;   // A row: voxel; B / D column: output channel
+  // weights as the A operand, voxels as the B (k_conv3): a lane ends with the
+  // output channels 4 kq .. + 3 of voxel i of each tile
+  int const i = lane & 15;   // output channel (weights), voxel (input, output)
   int const kq = lane >> 4;  // channels 8 (kq & 1) .. + 7 of position 2 s + (kq >> 1)
   uint16_t const *const xn = x + (int64_t)n * D * H * W * 16;
   int64_t const plane = (int64_t)H * W * 16;
@@ -696,26 +758,38 @@ __global__ __launch_bounds__(UT, 2) void k_conv3s(uint16_t const *__restrict__ x
   auto tcol = [&](int m) { return POOL ? 32 * (wave & 1) + 16 * (m & 1) : 16 * m; };
   // loaded once: a load in the loop would be issued after the next plane's
   // prefetch, and waiting for it would wait for the prefetch too
-  float const b = (mode & 1) ? bias[i] : 0.f;
-  // POOL: the even plane's pooling partials of this lane, per (tile column
-  // mc, voxel pair rp) (one of the bf16 values, so exact)
-  float pp[2][2] = {{-INFINITY, -INFINITY}, {-INFINITY, -INFINITY}};
+  f32x4 const b =
+      (mode & 1) ? *(f32x4 const *)(bias + 4 * kq) : f32x4{0.f, 0.f, 0.f, 0.f};
+  // LDS byte offsets of the lane's voxels in a plane, per step and (POOL)
+  // tile row: the loop adds constants only
+  int aof[POOL ? 2 : 1][5];
+#pragma unroll
+  for (int q = 0; q < (POOL ? 2 : 1); ++q)
+#pragma unroll
+    for (int s = 0; s < 5; ++s) {
+      int const u = 2 * s + (kq >> 1), t = u < 9 ? u : 8;
+      aof[q][s] = off_h((trow(2 * q) + t / 3) * PW + tcol(0) + i + t % 3, kq & 1);
+    }
+  // POOL: the even plane's pooling partials of this lane's two voxel rows'
+  // channels, per tile column mc (bf16 values, so exact)
+  float pp[2][4];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) pp[q >> 2][q & 3] = -INFINITY;
   // output plane oi (d0 + oi): bias, ReLU, into the wave's rows of buffer
   // oi & 1, then stored by the wave itself; POOL: its pooling
   auto epilogue = [&](int oi) {
     int const d = d0 + oi;
     uint16_t *const ob = so + (oi & 1) * ROWS + wave * 64 * OBS;
-    float fv[4][4];
+    uint2 pk[4];
+    if (mode & 2) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+      for (int m = 0; m < 4; ++m) pk[m] = out4<true>(acc[oi][m], b);
+    } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v = acc[oi][m][r] + b;
-        if (mode & 2) v = fmaxf(v, 0.f);
-        uint16_t const q = f2bf(v);
-        fv[m][r] = bf2f(q);
-        ob[(16 * m + 4 * kq + r) * OBS + i] = q;
-      }
+      for (int m = 0; m < 4; ++m) pk[m] = out4<false>(acc[oi][m], b);
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) *(uint2 *)(ob + (16 * m + i) * OBS + 4 * kq) = pk[m];
     __builtin_amdgcn_wave_barrier();
     if (d < D) {
 #pragma unroll
@@ -732,29 +806,41 @@ __global__ __launch_bounds__(UT, 2) void k_conv3s(uint16_t const *__restrict__ x
       }
     }
     if constexpr (POOL) {
-      // pooling window (tile column mc, voxel pair rp): rows m = mc, mc + 2
-      // (h order), voxels 2 rp, 2 rp + 1 (w order), after the even plane's
+      // pooling window of tile column mc: voxel i (and lane i + 1's, for even
+      // i) of tiles mc, mc + 2, scanned in (h, w) order with a strict >, after
+      // the even plane's
       bool const odd = oi & 1;
 #pragma unroll
-      for (int mc = 0; mc < 2; ++mc)
+      for (int mc = 0; mc < 2; ++mc) {
+        uint2 const own[2] = {pk[mc], pk[mc + 2]};
+        uint2 nb[2];
 #pragma unroll
-        for (int rp = 0; rp < 2; ++rp) {
-          float best = odd ? pp[mc][rp] : -INFINITY;
+        for (int q = 0; q < 2; ++q)
+          nb[q] = make_uint2(__shfl_xor(own[q].x, 1, 64), __shfl_xor(own[q].y, 1, 64));
+        uint32_t pq[2] = {0, 0};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          auto ch = [&](uint2 v) {
+            uint32_t const u = r < 2 ? v.x : v.y;
+            return __uint_as_float(r & 1 ? u & 0xffff0000u : u << 16);
+          };
+          float best = odd ? pp[mc][r] : -INFINITY;
 #pragma unroll
           for (int o = 0; o < 4; ++o) {
-            float const f = fv[2 * (o >> 1) + mc][2 * rp + (o & 1)];
+            float const f = ch(o & 1 ? nb[o >> 1] : own[o >> 1]);
             if (f > best) best = f;
           }
-          if (!odd) {
-            pp[mc][rp] = best;
-          } else {
-            int const dp = d / 2, hp = h0 / 2 + (wave >> 1);
-            int const wp = w0 / 2 + 16 * (wave & 1) + 8 * mc + 2 * kq + rp;
-            if (d < D && 2 * hp < H && 2 * wp < W)
-              pool[((((int64_t)n * (D / 2) + dp) * (H / 2) + hp) * (W / 2) + wp) * 16 + i] =
-                  f2bf(best);
-          }
+          pp[mc][r] = best;
+          pq[r >> 1] |= (__float_as_uint(best) >> 16) << (16 * (r & 1));  // a bf16 value
         }
+        if (odd && !(i & 1)) {
+          int const dp = d / 2, hp = h0 / 2 + (wave >> 1);
+          int const wp = w0 / 2 + 16 * (wave & 1) + 8 * mc + i / 2;
+          if (d < D && 2 * hp < H && 2 * wp < W)
+            *(uint2 *)(pool + ((((int64_t)n * (D / 2) + dp) * (H / 2) + hp) * (W / 2) + wp) * 16 +
+                       4 * kq) = make_uint2(pq[0], pq[1]);
+        }
+      }
     }
   };
   // AH2: two planes in flight per block (nxt, nx2), since the loads a CU
@@ -790,19 +876,16 @@ __global__ __launch_bounds__(UT, 2) void k_conv3s(uint16_t const *__restrict__ x
     }
 #pragma unroll
     for (int s = 0; s < 5; ++s) {
-      int const q = 2 * s + (kq >> 1);
-      int const qq = q < 9 ? q : 8;
-      int const kh = qq / 3, kw = qq - 3 * (qq / 3);
       u32x4 a[4];
 #pragma unroll
       for (int m = 0; m < 4; ++m)
-        a[m] = ld_h(cur, (trow(m) + kh) * PW + tcol(m) + i + kw, kq & 1);
+        a[m] = ld_b(cur, (POOL ? aof[m >> 1][s] + (m & 1) * 512 : aof[0][s] + m * 512));
 #pragma unroll
       for (int kd = 0; kd < 3; ++kd) {
         int const oi = j - kd;  // output plane d0 + oi = p + 1 - kd
         if (oi >= 0 && oi < DB) {
 #pragma unroll
-          for (int m = 0; m < 4; ++m) acc[oi][m] = mfma32(a[m], bw[kd][s], acc[oi][m]);
+          for (int m = 0; m < 4; ++m) acc[oi][m] = mfma32(bw[kd][s], a[m], acc[oi][m]);
         }
       }
     }
