@@ -21,7 +21,7 @@
 // (radix passes through LDS with table roots, forward and adjoint apart) ->
 // 1640 lines as above -> 1620 with the codelets -> 990 with reciprocals for
 // integer divisions; it moves 3.9 GB, 820 us at this card's copy rate. Time
-// transforms 1460 and 1670 -> 480 and 500. Prefetching the model's values
+// transforms 1460 and 1670 -> 480 and 500 -> 291 and 278. Prefetching the model's values
 // ahead of the transforms changed nothing (the lines' registers are worth
 // more as waves).
 #include <hip/hip_runtime.h>
@@ -425,69 +425,136 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
 }
 
 // ---------------------------------------------------------------------------
-// Time transforms of any even window length. Pt = M1 M2 (host: gtime), as the
-// complex transform of pairs of neighbouring traces, z = x_a + i x_b: no
-// unpack twiddles, and odd Pt costs the same as even. A block takes a tile of
-// 16 traces (8 pairs) and its time windows [tw0, tw1) as the specialised
-// kernels do; per time window the M1 phase, twiddle and M2 phase run in place
-// on one LDS tile [8][pitch], pitch = 4 mod 8 (the pairs of a load or store
-// fall in distinct banks). Output n = n1 + M1 n2 sits at n1 M2 + n2 (pos).
-// Short lines, so the loads and barriers bound these kernels, and blocks per
-// CU hide them: a register prefetch of the next tile in the forward, which
-// takes a wave per SIMD, ran 656 against 484 us on the volume above.
+// Time transforms of any even window length, as the complex transform of
+// pairs of neighbouring traces, z = x_a + i x_b: no unpack twiddles, and odd
+// Pt costs the same as even. A block takes a tile of 16 traces (8 pairs) and
+// its time windows [tw0, tw1) as the specialised kernels do; per time window
+// the phases run in place on one LDS tile [8][pitch], pitch = 4 mod 8 (lanes
+// are (pair, line): the eight pairs start 4 values apart modulo 32, so that a
+// phase's reads are free of bank conflicts at an odd line stride).
+//
+// HB = 0: Pt = M1 M2 M3 with factors up to 16 (M3 = 1: two phases), each
+// phase a register FFT. HB > 0: Pt = M1 M2, lines of up to 2 HB + 1 values,
+// for the lengths with other primes. Output n = n1 + M1 (n2 + M2 n3) sits at
+// n1 M2 M3 + n2 M3 + n3 (pos).
+//
+// Latency bounds these kernels (loads, barriers, a phase's few lines), and
+// waves hide it, so short factors pay twice: fewer instructions, and
+// registers for more waves. Measured on the volume above (Pt = 250 = 10 x 5 x
+// 5, 1.0 GB a launch), forward and adjoint: lines of 10 x 25 484 and 500 us
+// (four waves to a SIMD, 220 million vector instructions), now 291 and 278
+// (six, 129 million). A register prefetch of the next tile in the forward,
+// which takes waves, ran 656 against 484 us.
 // ---------------------------------------------------------------------------
 constexpr int kPairs = 8;
 __host__ __device__ constexpr int time_pitch(int Pt) { return (Pt + 3) / 8 * 8 + 4; }
 
 struct TimeTables {
-  float2 *Z, *TW;
+  float2 *Z, *TW, *TW2;
   unsigned short *pos;
 };
 
 template <int S>
 __device__ __forceinline__ void time_tables(TimeTables const &t, float2 const *roots, int N,
-                                            int M1, int M2) {
-  float const i1 = 1.f / (float)M1;
+                                            int M1, int M2, int M3) {
+  float const i1 = 1.f / (float)M1, i2 = 1.f / (float)M2;
   for (int m = threadIdx.x; m < N; m += 256) {
-    // TW[k2 M1 + n1] = exp(S 2 pi i n1 k2 / N)
-    int const k2 = quot(m, i1), n1 = m - k2 * M1;
-    float2 const r = roots[n1 * k2];  // n1 k2 < N
-    t.TW[m] = make_float2(r.x, S > 0 ? -r.y : r.y);
-    t.pos[m] = (unsigned short)(n1 * M2 + k2);  // of output m = n1 + M1 n2, n2 = k2
+    // TW[r M1 + n1] = exp(S 2 pi i n1 r / N)
+    int const r = quot(m, i1), n1 = m - r * M1, n3 = quot(r, i2), n2 = r - n3 * M2;
+    float2 const z = roots[n1 * r];  // n1 r < N
+    t.TW[m] = make_float2(z.x, S > 0 ? -z.y : z.y);
+    t.pos[m] = (unsigned short)((n1 * M2 + n2) * M3 + n3);
+    // TW2[k3 M2 + n2] = exp(S 2 pi i n2 k3 / (M2 M3))
+    if (M3 > 1 && n1 == 0) {
+      float2 const y = roots[n2 * n3 * M1];
+      t.TW2[r] = make_float2(y.x, S > 0 ? -y.y : y.y);
+    }
+  }
+}
+
+// a phase's lines as register FFTs of a length in Ps: line l of at(l), stride
+// st, output q through put(line, q, st, value). (st passes through an empty
+// asm, so that the sums of the addresses are not kept, in registers that then
+// spilled, beyond their use.)
+template <int S, class At, class Put>
+__device__ __forceinline__ void phase(int, int, int, At const &, Put const &) {}
+template <int S, int N, int... Ps, class At, class Put>
+__device__ __forceinline__ void phase(int P, int total, int st, At const &at, Put const &put) {
+  if (P != N) {
+    phase<S, Ps...>(P, total, st, at, put);
+    return;
+  }
+  int l = threadIdx.x;
+  asm volatile("" : "+v"(l), "+s"(st));
+  for (; l < total; l += 256) {
+    auto const z = at(l);
+    float2 v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = z.p[k * st];
+    agdfft::fft<N, S>(v);
+    asm volatile("" : "+s"(st) : : "memory");
+#pragma unroll
+    for (int k = 0; k < N; ++k) put(z, k, st, v[k]);
   }
 }
 
 template <int HB, int S>
-__device__ __forceinline__ void time_fft(TimeTables const &t, int pitch, int M1, int M2,
+__device__ __forceinline__ void time_fft(TimeTables const &t, int pitch, int M1, int M2, int M3,
                                          float const *dft, int d1, int d2) {
   struct At {
     float2 *p;
     float2 const *tw;
   };
-  if (M1 > 1) {
-    float const i2 = 1.f / (float)M2;
-    block_lines<HB, S>(
-        kPairs * M2, M2, M1, M1, M1, uniform(dft, d1),
-        [&](int l) {
-          int const p = quot(l, i2), k2 = l - p * M2;
-          return At{t.Z + p * pitch + k2, t.TW + k2 * M1};
-        },
-        [&](At const &z, int q, float2 v) {
-          z.p[q * M2] = q == 0 ? v : agdfft::c_mul(v, z.tw[q]);
-        });
+  int const M23 = M2 * M3;
+  auto const twiddled = [](At const &z, int q, int st, float2 v) {
+    z.p[q * st] = q == 0 ? v : agdfft::c_mul(v, z.tw[q]);
+  };
+  auto const plain = [](At const &z, int q, int st, float2 v) { z.p[q * st] = v; };
+  auto const at1 = [&](int l) {
+    int const p = l % kPairs, r = l / kPairs;
+    return At{t.Z + p * pitch + r, t.TW + r * M1};
+  };
+  auto const at2 = [&](int l) {  // M3 = 1
+    int const p = l % kPairs, n1 = l / kPairs;
+    return At{t.Z + p * pitch + n1 * M2, nullptr};
+  };
+  auto const run = [&](int P, int total, int st, auto const &at, auto const &put) {
+    phase<S, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>(P, total, st, at, put);
+    __syncthreads();
+  };
+  if constexpr (HB == 0) {
+    run(M1, kPairs * M23, M23, at1, twiddled);
+    if (M3 == 1) {
+      run(M2, kPairs * M1, 1, at2, plain);
+    } else {
+      float const i3 = 1.f / (float)M3;
+      run(M2, kPairs * M1 * M3, M3,
+          [&](int l) {
+            int const p = l % kPairs, r = l / kPairs, n1 = quot(r, i3), k3 = r - n1 * M3;
+            return At{t.Z + p * pitch + n1 * M23 + k3, t.TW2 + k3 * M2};
+          },
+          twiddled);
+      run(M3, kPairs * M1 * M2, 1,
+          [&](int l) {
+            int const p = l % kPairs, r = l / kPairs;
+            return At{t.Z + p * pitch + r * M3, nullptr};
+          },
+          plain);
+    }
+  } else {
+    if (M1 > 1)
+      block_lines<HB, S>(kPairs * M2, M2, M1, M1, M1, uniform(dft, d1), at1,
+                         [&](At const &z, int q, float2 v) { twiddled(z, q, M2, v); });
+    block_lines<HB, S>(kPairs * M1, 1, M2, M2, M2, uniform(dft, d2), at2,
+                       [&](At const &z, int q, float2 v) { plain(z, q, 1, v); });
   }
-  float const i1 = 1.f / (float)M1;
-  block_lines<HB, S>(
-      kPairs * M1, 1, M2, M2, M2, uniform(dft, d2),
-      [&](int l) {
-        int const p = quot(l, i1), n1 = l - p * M1;
-        return At{t.Z + p * pitch + n1 * M2, nullptr};
-      },
-      [&](At const &z, int q, float2 v) { z.p[q] = v; });
 }
 
+// waves per SIMD that the registers are bounded for
+constexpr int time_waves(int HB) { return HB == 0 ? 6 : HB <= 16 ? 4 : HB <= 32 ? 2 : 1; }
+
 template <int HB>
-__global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_fwd_time_g(
+__global__ __launch_bounds__(256, time_waves(HB)) void k_fwd_time_g(
     AgdWin const *__restrict__ wins, int const *__restrict__ blocks, int block0,
     float const *__restrict__ dft, AgdFftPlan const *__restrict__ plans,
     float2 const *__restrict__ roots, float const *__restrict__ tapers,
@@ -500,16 +567,17 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
   int const tw0 = bl[2] + twn * blockIdx.y / gridDim.y;
   int const tw1 = bl[2] + twn * (blockIdx.y + 1) / gridDim.y;
   int const twa = tw0 > 0 ? tw0 - 1 : 0;
-  int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2;
+  int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2, M3 = max(w.gm3, 1);
   int const nconv = w.nconv, ntw = w.ntw, pitch = time_pitch(N);
   TimeTables t;
   t.Z = sm;
   t.TW = t.Z + kPairs * pitch;
-  float *const TP = (float *)(t.TW + N);    // [Wt] time taper
+  t.TW2 = t.TW + N;  // [M2 M3], unless M3 = 1
+  float *const TP = (float *)(t.TW2 + (M3 > 1 ? M2 * M3 : 0));    // [Wt] time taper
   float *const CA = TP + Wt;                // [16][half] overlap carry
   t.pos = (unsigned short *)(CA + 2 * kPairs * half);
   int const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = 4;
-  time_tables<+1>(t, roots + plans[w.tplan_full].roots_off, N, M1, M2);
+  time_tables<+1>(t, roots + plans[w.tplan_full].roots_off, N, M1, M2, M3);
   for (int i = tid; i < Wt; i += 256) TP[i] = tapers[w.tt_off + i];
   for (int i = tid; i < 2 * kPairs * half; i += 256) CA[i] = 0.f;
   float *const Tb = T + w.t_off + (int64_t)t0 * nconv;
@@ -540,7 +608,7 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
       }
     }
     __syncthreads();
-    time_fft<HB, +1>(t, pitch, M1, M2, dft, w.tdft1, w.tdft2);
+    time_fft<HB, +1>(t, pitch, M1, M2, M3, dft, w.tdft1, w.tdft2);
     // overlap-add: samples [0, half) complete this window's first half
     for (int p = wave; p < kPairs; p += nw) {
       if (2 * p >= nt) break;
@@ -571,7 +639,7 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
 }
 
 template <int HB>
-__global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_adj_time_g(
+__global__ __launch_bounds__(256, time_waves(HB)) void k_adj_time_g(
     AgdWin const *__restrict__ wins, int const *__restrict__ blocks, int block0,
     float const *__restrict__ dft, AgdFftPlan const *__restrict__ plans,
     float2 const *__restrict__ roots, float const *__restrict__ tapers,
@@ -588,15 +656,16 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
   int const twn = bl[3] - bl[2];
   int const tw0 = bl[2] + twn * blockIdx.y / gridDim.y;
   int const tw1 = bl[2] + twn * (blockIdx.y + 1) / gridDim.y;
-  int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2;
+  int const N = w.Pt, Ft = w.Ft, Wt = w.Wt, half = w.half, M1 = w.gm1, M2 = w.gm2, M3 = max(w.gm3, 1);
   int const nconv = w.nconv, pitch = time_pitch(N);
   TimeTables t;
   t.Z = sm;
   t.TW = t.Z + kPairs * pitch;
-  float *const TP = (float *)(t.TW + N);
+  t.TW2 = t.TW + N;  // [M2 M3], unless M3 = 1
+  float *const TP = (float *)(t.TW2 + (M3 > 1 ? M2 * M3 : 0));
   t.pos = (unsigned short *)(TP + Wt);
-  int const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = 4;
-  time_tables<-1>(t, roots + plans[w.tplan_full].roots_off, N, M1, M2);
+  int const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  time_tables<-1>(t, roots + plans[w.tplan_full].roots_off, N, M1, M2, M3);
   for (int i = tid; i < Wt; i += 256) TP[i] = plain ? 1.f : tapers[w.tt_off + i];
   __syncthreads();
   // one source: the record through the blend entries, or a trace buffer; a
@@ -656,7 +725,7 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
       }
     }
     __syncthreads();
-    time_fft<HB, -1>(t, pitch, M1, M2, dft, w.tdft1, w.tdft2);
+    time_fft<HB, -1>(t, pitch, M1, M2, M3, dft, w.tdft1, w.tdft2);
     // half spectra of the two real traces of a pair, x2 on the interior bins
     float4 *const vo = vt + tw * tw_step;
     for (int i = tid; i < Ft * kPairs; i += 256) {
@@ -707,6 +776,7 @@ static int launch_fwd_time_g(AgdDev const *g, AgdClass const &c, int first, int 
 }
 int fwd_time_general(AgdDev const *g, AgdClass const &c, int first, int n) {
   switch (c.hb) {
+    case AGD_TIME_FACTORED: return launch_fwd_time_g<0>(g, c, first, n);
     case 8: return launch_fwd_time_g<8>(g, c, first, n);
     case 16: return launch_fwd_time_g<16>(g, c, first, n);
     case 32: return launch_fwd_time_g<32>(g, c, first, n);
@@ -726,6 +796,7 @@ static int launch_adj_time_g(AgdDev const *g, AgdClass const &c, int first, int 
 int adj_time_general(AgdDev const *g, AgdClass const &c, int first, int n,
                             float const *Tin, int plain) {
   switch (c.hb) {
+    case AGD_TIME_FACTORED: return launch_adj_time_g<0>(g, c, first, n, Tin, plain);
     case 8: return launch_adj_time_g<8>(g, c, first, n, Tin, plain);
     case 16: return launch_adj_time_g<16>(g, c, first, n, Tin, plain);
     case 32: return launch_adj_time_g<32>(g, c, first, n, Tin, plain);

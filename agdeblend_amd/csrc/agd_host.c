@@ -1142,34 +1142,57 @@ static int spatial_lines(AgdWin const *W) {
   return line_instance(m, kSpatialInst);
 }
 
-/* dynamic LDS of the run-time sized time kernels (time_g_lds) */
+/* dynamic LDS of the run-time sized time kernels: the tile, the twiddles,
+ * the time taper, the overlap carry and the output positions */
 static size_t time_lines_lds(AgdWin const *W) {
   size_t const pitch = (size_t)(W->Pt + 3) / 8 * 8 + 4;
-  return 8 * (TIME_TILE / 2 * pitch + (size_t)W->Pt) + 4 * (size_t)W->Wt +
+  size_t const tw2 = W->gm3 > 1 ? (size_t)W->gm2 * (size_t)W->gm3 : 0;
+  return 8 * (TIME_TILE / 2 * pitch + (size_t)W->Pt + tw2) + 4 * (size_t)W->Wt +
          4 * (size_t)TIME_TILE * (size_t)W->half + 2 * (size_t)W->Pt + 16;
 }
 
-/* Pt = m1 m2 with the smaller longest factor (an odd one last: the second
- * phase's lanes are m2 apart in LDS) of the run-time sized time kernels:
- * even window lengths, factors up to 129, 96 KB of LDS; else 0 0 */
-static void time_lines(AgdWin const *W, int *m1, int *m2) {
-  int a;
-  *m1 = 0;
-  *m2 = 0;
-  if (W->Wt % 2 || time_lines_lds(W) > 96 * 1024) return;
-  for (a = 1; a * a <= W->Pt; a++)
-    if (W->Pt % a == 0) {
-      *m1 = a;
-      *m2 = W->Pt / a;
+/* Phases of the run-time sized time kernels: even window lengths, 96 KB of
+ * LDS; else 0 0 0. Pt = m1 m2 m3 with factors up to 16 where there are such
+ * (fewest phases, then the smallest longest factor; the last phase's lanes
+ * are a factor apart in LDS, so one with the fewest factors 2 last), else
+ * lines Pt = m1 m2 with the smaller longest factor, up to 129 (m3 = 0). */
+#define TIME_LIMIT (96 * 1024)
+static void time_lines(AgdWin *W) {
+  int const N = W->Pt;
+  int a, b, best = 0;
+  W->gm1 = W->gm2 = W->gm3 = 0;
+  if (W->Wt % 2) return;
+  for (a = 2; a <= 16 && a < N; a++)
+    for (b = 2; N % a == 0 && b <= 16; b++) {
+      int const c = N / a / b, last = c > 1 ? c : b;
+      int longest = a > b ? a : b, cost;
+      if (N / a % b || c > 16) continue;
+      if (c > longest) longest = c;
+      cost = (c > 1) * 1024 + longest * 32 + (last & -last);
+      if (best == 0 || cost < best) {
+        best = cost;
+        W->gm1 = a;
+        W->gm2 = b;
+        W->gm3 = c;
+      }
     }
-  if (*m2 % 2 == 0 && *m1 % 2 && *m1 > 1) {
-    int const t = *m1;
-    *m1 = *m2;
-    *m2 = t;
+  if (best && time_lines_lds(W) <= TIME_LIMIT) return;
+  W->gm1 = W->gm2 = W->gm3 = 0;
+  if (time_lines_lds(W) > TIME_LIMIT) return;
+  for (a = 1; a * a <= N; a++)
+    if (N % a == 0) {
+      W->gm1 = a;
+      W->gm2 = N / a;
+    }
+  if (W->gm2 % 2 == 0 && W->gm1 % 2 && W->gm1 > 1) {
+    int const t = W->gm1;
+    W->gm1 = W->gm2;
+    W->gm2 = t;
   }
-  if (line_instance(*m1 > *m2 ? *m1 : *m2, kTimeInst) == 0) *m1 = *m2 = 0;
+  if (line_instance(W->gm1 > W->gm2 ? W->gm1 : W->gm2, kTimeInst) == 0) W->gm1 = W->gm2 = 0;
 }
 static int time_instance(AgdWin const *W) {
+  if (W->gm3) return AGD_TIME_FACTORED;
   return W->gm2 ? line_instance(W->gm1 > W->gm2 ? W->gm1 : W->gm2, kTimeInst) : 0;
 }
 
@@ -1617,9 +1640,10 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
             if ((W->sdft[d] = dft_get(&ps, W->P[d])) < 0) goto err;
         time_key(W, &m1, &m2);
         if (m1 == 0) {
-          time_lines(W, &W->gm1, &W->gm2);
-          if (W->gm2 && ((W->tdft1 = dft_get(&ps, W->gm1)) < 0 ||
-                         (W->tdft2 = dft_get(&ps, W->gm2)) < 0))
+          time_lines(W);
+          if (W->gm2 && W->gm3 == 0 &&
+              ((W->tdft1 = dft_get(&ps, W->gm1)) < 0 ||
+               (W->tdft2 = dft_get(&ps, W->gm2)) < 0))
             goto err;
         }
       }

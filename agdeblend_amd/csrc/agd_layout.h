@@ -27,6 +27,8 @@
 #define AGD_MAXSTAGE 24  /* FFT stages per plan */
 /* model values of one task of the run-time sized spatial kernel at most */
 #define AGD_LINES_VALUES 4096
+/* AgdClass.hb of the run-time sized time kernels on register FFTs */
+#define AGD_TIME_FACTORED 4
 /* half lengths Mr / 2 of the wavelet convolution with a compile-time kernel
  * (k_wavelet_t); the host prefers them to the smallest 7-smooth length when
  * one is at most 25% longer */
@@ -60,9 +62,10 @@ typedef struct {
   int patch;
   float scaler;          /* 1 / sqrt(prod P) (fk.c:157-163) */
   /* run-time sized kernels (agd_general.h): coefficient offsets per space
-   * dim, Pt = gm1 * gm2 (gm2 0: none) and its two factors' offsets */
+   * dim; Pt = gm1 * gm2 * gm3 in register FFTs, or (gm3 0) gm1 * gm2 in
+   * lines with their coefficients' offsets (gm2 0: none) */
   int sdft[AGD_MAXSP];
-  int gm1, gm2;
+  int gm1, gm2, gm3;
   int tdft1, tdft2;
   int64_t x_off;         /* model offset (complex) */
   int64_t u_off;         /* intermediate offset (complex) */
@@ -90,7 +93,8 @@ typedef struct {
   int tb;       /* time classes: traces per block; specialised spatial
                    classes: 1 when the time transform is specialised too */
   int hb;       /* run-time sized kernels: coefficient pairs held per line
-                   (half the longest line, rounded up to an instance) */
+                   (half the longest line, rounded up to an instance), or
+                   AGD_TIME_FACTORED */
   int var;      /* time classes: forward kernel variant (0 register
                    prefetch, 1 lean tile); spatial classes: unused */
   int ntw;      /* time classes: most time windows of a block */

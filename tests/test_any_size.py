@@ -3,9 +3,9 @@
 A line of P padded values is held by one thread in registers: P up to 33,
 49, 65, 97 and 129 by kernel instance (the windows below sit on both sides
 of each edge, at lengths with a register codelet and at primes), longer ones
-go to the LDS-resident kernels; the time transform takes Pt = M1 M2 in two
-phases, with M1 = 1 for a prime Pt, and hands Pt = 313 to the LDS-resident
-kernels. Window traces that do not fill their last tile of 16, batches of
+go to the LDS-resident kernels; the time transform takes Pt in two or three
+register FFTs of up to 16 values, else in lines M1 M2, with M1 = 1 for a
+prime Pt, and hands Pt = 313 to the LDS-resident kernels. Window traces that do not fill their last tile of 16, batches of
 lines shared by several waves, one to four space dims, patches that a window
 covers whole (odd lengths) or with windows of two lengths.
 
@@ -63,6 +63,18 @@ def test_any_window_length_matches_fp64_oracle(shape, windows):
         assert abs(lhs - rhs) <= 1e-6 * np.linalg.norm(got) * np.linalg.norm(y)
     finally:
         pm.close()
+
+
+# time transforms in register FFTs: two phases (15 x 16, 11 x 13), three (equal
+# odd factors, a last factor with a power of two, the longest within the LDS
+# limit), tiles of odd trace counts, several windows of a run
+PHASES = [((19, 384), (18, 192)), ((7, 227), (6, 114)), ((22, 547), (22, 274)),
+          ((21, 1024), (18, 512)), ((18, 1440), (18, 720)), ((35, 60), (34, 16))]
+
+
+@pytest.mark.parametrize("shape,windows", PHASES, ids=[str(w[1]) for _, w in PHASES])
+def test_time_phases_match_fp64_oracle(shape, windows):
+    test_any_window_length_matches_fp64_oracle(shape, windows)
 
 
 @pytest.mark.parametrize("nan", [False, True])
