@@ -13,7 +13,9 @@
 // with coefficients that are the same for every thread and come through
 // the scalar cache as instruction operands. No roots, divisions or LDS
 // traffic inside a line, and no dependence on how P factors. Lengths without
-// a prime factor above 13 take a register FFT instead (codelets).
+// a prime factor above 13 take a register FFT instead (codelets). Where that
+// FFT's registers would leave few waves (above 33), P = A B folds into two
+// short ones in place (HB = 0).
 //
 // Measured (MI355X) on a 45 x 333 x 1500 volume in two patches, windows of
 // 17-18 x 24-25 x 200 (P = 22, 23 x 30, 32, Pt = 250; model 1.15 GB), us per
@@ -180,7 +182,7 @@ __device__ __forceinline__ int quot(int a, float inv) {
 typedef int i4 __attribute__((ext_vector_type(AGD_MAXSP)));
 struct Planes {
   int nsp, rows, pitch, rp;  // rows of a plane, row pitch, values of a plane
-  i4 ext, str, P, W;         // per space dim
+  i4 ext, str, P, W, A;      // per space dim (A: lines' first factor, HB = 0)
 };
 
 // a[i], uniform, without indexed registers
@@ -218,11 +220,81 @@ __device__ __forceinline__ bool codelets(int P, int total, int st, At const &at)
   return codelets<S, Ps...>(P, total, st, at);
 }
 
+// The two phases of a folded line (lines, HB = 0): `total` lines at(i), each
+// B (A) short lines, threads over (short line, line). rt[m] = exp(-2 pi i m /
+// P).
+template <int S, class At>
+__device__ __forceinline__ void fold_a(int, int, int, float, int, int, At const &, float2 const *) {}
+template <int S, int N, int... Ns, class At>
+__device__ __forceinline__ void fold_a(int A, int B, int total, float it, int st, int nin,
+                                       At const &at, float2 const *rt) {
+  if (A != N) {
+    fold_a<S, Ns...>(A, B, total, it, st, nin, at, rt);
+    return;
+  }
+  int l = threadIdx.x, sb = B * st;
+  asm volatile("" : "+v"(l), "+s"(sb));
+  for (; l < total * B; l += 256) {
+    int const r = quot(l, it);
+    float2 *const z = at(l - r * total).p + r * st;
+    float2 v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = r + k * B < nin ? z[k * sb] : make_float2(0.f, 0.f);
+    agdfft::fft<N, S>(v);
+    asm volatile("" : "+s"(sb) : : "memory");
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      float2 w = rt[q * r];
+      if (S > 0) w.y = -w.y;
+      z[q * sb] = q == 0 ? v[q] : agdfft::c_mul(v[q], w);
+    }
+  }
+}
+template <int S, class At>
+__device__ __forceinline__ void fold_b(int, int, int, float, int, int, At const &) {}
+template <int S, int N, int... Ns, class At>
+__device__ __forceinline__ void fold_b(int A, int B, int total, float it, int st, int nout,
+                                       At const &at) {
+  if (B != N) {
+    fold_b<S, Ns...>(A, B, total, it, st, nout, at);
+    return;
+  }
+  // at most AGD_LINES_VALUES / N short lines
+  constexpr int R = (AGD_LINES_VALUES / N + 255) / 256;
+  int l0 = threadIdx.x, sa = A * st;
+  asm volatile("" : "+v"(l0), "+s"(st));
+  float2 v[R][N];
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    int const l = l0 + 256 * c;
+    if (l < total * A) {
+      int const n1 = quot(l, it);
+      float2 const *const z = at(l - n1 * total).p + n1 * N * st;
+#pragma unroll
+      for (int k = 0; k < N; ++k) v[c][k] = z[k * st];
+      agdfft::fft<N, S>(v[c]);
+    }
+  }
+  __syncthreads();
+  asm volatile("" : "+v"(l0), "+s"(sa));
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    int const l = l0 + 256 * c;
+    if (l < total * A) {
+      int const n1 = quot(l, it);
+      float2 *const z = at(l - n1 * total).p + n1 * st;
+#pragma unroll
+      for (int k = 0; k < N; ++k)
+        if (n1 + k * A < nout) z[k * sa] = v[c][k];
+    }
+  }
+}
+
 // transforms every line along dim d of the nk planes in place; the other
 // dims run over their current extents g.ext
 template <int HB, int S>
 __device__ __forceinline__ void lines(float2 *sm, Planes &g, int nk, int d, int nin, int nout,
-                                      cfloat const *tab) {
+                                      cfloat const *tab, float2 const *rt) {
   int cnt = 1;
 #pragma unroll
   for (int e = 0; e < AGD_MAXSP; ++e)
@@ -245,16 +317,33 @@ __device__ __forceinline__ void lines(float2 *sm, Planes &g, int nk, int d, int 
     }
     return At{sm + off};
   };
-  bool done = codelets<S, 8, 9, 10, 12, 13, 14, 15>(P, total, st, at);
-  if constexpr (HB >= 16)
-    if (!done) done = codelets<S, 18, 20, 22, 24, 25, 27, 28, 30, 32, 33>(P, total, st, at);
-  if constexpr (HB >= 24)
-    if (!done) done = codelets<S, 35, 39, 40, 42, 44, 45, 48, 49>(P, total, st, at);
-  if constexpr (HB >= 32)
-    if (!done) done = codelets<S, 50, 52, 54, 55, 60, 63, 64, 65>(P, total, st, at);
-  if (!done)
-    block_lines<HB, S>(total, st, P, nin, nout, tab, at,
-                       [&](At const &z, int q, float2 v) { z.p[q * st] = v; });
+  if constexpr (HB == 0) {
+    if (!codelets<S, 2, 3, 4, 5, 7, 8, 9, 10, 12, 13, 14, 15>(P, total, st, at)) {
+      // P = A B in place: A-point lines over k1 (k = k1 B + k2), twiddle,
+      // then B-point lines over k2, whose outputs n = n1 + A n2 go to their
+      // natural places once every thread has read its inputs
+      // (1-D lines of 64 on 59 windows of 51 x 126: one FFT in 228 registers
+      // left 8 waves to a CU, three of four idle, 88 us; now 58, for 27 at
+      // the cached copy rate; the block's four barriers bound it)
+      int const A = pick(g.A, d), B = quot(P, 1.f / (float)A);
+      float const it = 1.f / (float)total;
+      fold_a<S, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>(A, B, total, it, st, nin, at, rt);
+      __syncthreads();
+      fold_b<S, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>(A, B, total, it, st, nout, at);
+      __syncthreads();
+    }
+  } else {
+    bool done = codelets<S, 8, 9, 10, 12, 13, 14, 15>(P, total, st, at);
+    if constexpr (HB >= 16)
+      if (!done) done = codelets<S, 18, 20, 22, 24, 25, 27, 28, 30, 32, 33>(P, total, st, at);
+    if constexpr (HB >= 24)
+      if (!done) done = codelets<S, 35, 39, 40, 42, 44, 45, 48, 49>(P, total, st, at);
+    if constexpr (HB >= 32)
+      if (!done) done = codelets<S, 50, 52, 54, 55, 60, 63, 64, 65>(P, total, st, at);
+    if (!done)
+      block_lines<HB, S>(total, st, P, nin, nout, tab, at,
+                         [&](At const &z, int q, float2 v) { z.p[q * st] = v; });
+  }
 #pragma unroll
   for (int e = 0; e < AGD_MAXSP; ++e)
     if (e == d) g.ext[e] = nout;
@@ -314,9 +403,11 @@ __device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr,
 // mode -1: forward only (X -> U); 0..5 as k_adj_spatial_t's MODE, followed by
 // the forward transform of the new model when fuse is set
 template <int HB>
-__global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_spatial_g(
+__global__ __launch_bounds__(
+    256, HB == 0 ? 5 : HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_spatial_g(
     AgdWin const *__restrict__ wins, AgdTask const *__restrict__ tasks, int task0,
-    float const *__restrict__ dft, float2 const *__restrict__ V, float2 *__restrict__ X,
+    float const *__restrict__ dft, AgdFftPlan const *__restrict__ plans,
+    float2 const *__restrict__ roots, float2 const *__restrict__ V, float2 *__restrict__ X,
     float2 *__restrict__ U, float alpha, float lamb, float const *__restrict__ lamb_dev, int mode,
     int fuse, unsigned int *__restrict__ maxbits) {
   extern __shared__ float2 sm[];
@@ -336,16 +427,36 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
       if (e < nsp) {
         g.P[e] = w.P[e];
         g.W[e] = w.W[e];
+        g.A[e] = w.sfac[e];
         g.str[e] = st;
         st *= e == nsp - 1 ? g.pitch : w.P[e];
       } else {
-        g.P[e] = g.W[e] = g.str[e] = 1;
+        g.P[e] = g.W[e] = g.str[e] = g.A[e] = 1;
       }
     }
   }
   int64_t const uoff = w.u_off + (int64_t)t.tw * ((w.ntr + 15) / 16) * w.Ft * 16;
   float2 *const x = X + w.x_off + ((int64_t)t.tw * w.Ft + t.k0) * w.S;
   int const total = nk * w.S;
+  // HB = 0: the dims' roots [P_0] .. [P_{n-1}] after the planes (the longest
+  // task's: a class's LDS is its largest)
+  float2 *const rts = sm + nk * g.rp;
+  if constexpr (HB == 0) {
+    int o = 0;
+    for (int d = 0; d < nsp; ++d) {
+      int const P = w.P[d];
+      for (int m = threadIdx.x; m < P; m += 256) rts[o + m] = roots[plans[w.splan[d]].roots_off + m];
+      o += P;
+    }
+    __syncthreads();
+  }
+  auto const rt = [&](int d) {
+    int o = 0;
+#pragma unroll
+    for (int e = 0; e < AGD_MAXSP; ++e)
+      if (e < d) o += g.P[e];
+    return rts + o;
+  };
   bool const has_x = mode == -1 || mode == 0 || mode == 2;
   if (mode >= 0) {
 #pragma unroll
@@ -353,7 +464,7 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
     tiles_copy<true>(sm, g, w.ntr, w.Ft, const_cast<float2 *>(V) + uoff, t.k0, nk);
     __syncthreads();
     for (int d = nsp - 1; d >= 0; --d)
-      lines<HB, -1>(sm, g, nk, d, pick(g.W, d), pick(g.P, d), uniform(dft, w.sdft[d]));
+      lines<HB, -1>(sm, g, nk, d, pick(g.W, d), pick(g.P, d), uniform(dft, w.sdft[d]), rt(d));
   }
   // value i sits at LDS offset i + (row of i) (pitch - last)
   {
@@ -419,7 +530,7 @@ __global__ __launch_bounds__(256, HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1
 #pragma unroll
     for (int e = 0; e < AGD_MAXSP; ++e) g.ext[e] = g.P[e];
     for (int d = 0; d < nsp; ++d)
-      lines<HB, +1>(sm, g, nk, d, pick(g.P, d), pick(g.W, d), uniform(dft, w.sdft[d]));
+      lines<HB, +1>(sm, g, nk, d, pick(g.P, d), pick(g.W, d), uniform(dft, w.sdft[d]), rt(d));
     tiles_copy<false>(sm, g, w.ntr, w.Ft, U + uoff, t.k0, nk);
   }
 }
@@ -752,12 +863,14 @@ static int launch_spatial_g(AgdDev const *g, AgdClass const &c, float2 *X, float
   int const n = class_range(g, c, &first);
   if (n <= 0) return 0;
   return launch(mode < 0 ? "fwd_spatial" : "adj_spatial", k_spatial_g<HB>, dim3(n),
-                dim3(NTHR), c.lds, g->win, g->tasks, first, g->dft, (float2 const *)g->V, X,
+                dim3(NTHR), c.lds, g->win, g->tasks, first, g->dft, g->plans,
+                (float2 const *)g->roots, (float2 const *)g->V, X,
                 (float2 *)g->U, alpha, lamb, (float const *)g->lamb_dev, mode, fuse, g->scalar);
 }
 int spatial_general(AgdDev const *g, AgdClass const &c, float2 *X, float alpha,
                            float lamb, int mode, int fuse) {
   switch (c.hb) {
+    case AGD_FACTORED: return launch_spatial_g<0>(g, c, X, alpha, lamb, mode, fuse);
     case 8: return launch_spatial_g<8>(g, c, X, alpha, lamb, mode, fuse);
     case 16: return launch_spatial_g<16>(g, c, X, alpha, lamb, mode, fuse);
     case 24: return launch_spatial_g<24>(g, c, X, alpha, lamb, mode, fuse);
@@ -776,7 +889,7 @@ static int launch_fwd_time_g(AgdDev const *g, AgdClass const &c, int first, int 
 }
 int fwd_time_general(AgdDev const *g, AgdClass const &c, int first, int n) {
   switch (c.hb) {
-    case AGD_TIME_FACTORED: return launch_fwd_time_g<0>(g, c, first, n);
+    case AGD_FACTORED: return launch_fwd_time_g<0>(g, c, first, n);
     case 8: return launch_fwd_time_g<8>(g, c, first, n);
     case 16: return launch_fwd_time_g<16>(g, c, first, n);
     case 32: return launch_fwd_time_g<32>(g, c, first, n);
@@ -796,7 +909,7 @@ static int launch_adj_time_g(AgdDev const *g, AgdClass const &c, int first, int 
 int adj_time_general(AgdDev const *g, AgdClass const &c, int first, int n,
                             float const *Tin, int plain) {
   switch (c.hb) {
-    case AGD_TIME_FACTORED: return launch_adj_time_g<0>(g, c, first, n, Tin, plain);
+    case AGD_FACTORED: return launch_adj_time_g<0>(g, c, first, n, Tin, plain);
     case 8: return launch_adj_time_g<8>(g, c, first, n, Tin, plain);
     case 16: return launch_adj_time_g<16>(g, c, first, n, Tin, plain);
     case 32: return launch_adj_time_g<32>(g, c, first, n, Tin, plain);

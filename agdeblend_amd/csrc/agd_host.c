@@ -1131,14 +1131,36 @@ static int line_instance(int n, int const *inst) {
 static int const kSpatialInst[] = {8, 16, 24, 32, 48, 64, 0};
 static int const kTimeInst[] = {8, 16, 32, 64, 0};
 
+/* The first factor of the padded length P in two register FFTs of 4 to 16
+ * values, the smaller longest one first; 1 where one FFT holds it (the list
+ * of lines<0>), 0 where none does */
+static int line_factor(int P) {
+  int a;
+  if (P <= 5 || P == 7 || P == 8 || P == 9 || P == 10 || (P >= 12 && P <= 15)) return P > 1;
+  for (a = 16; a >= 4; a--)
+    if (P % a == 0 && a * a >= P && P / a >= 4) {
+      int b = a, c;
+      for (c = a; c >= 4; c--)
+        if (P % c == 0 && c * c >= P) b = c;
+      return b;
+    }
+  return 0;
+}
+
 /* coefficient pairs of the window's run-time sized spatial kernel: lines up
  * to 129 and planes within the generic kernel's limit (0: the LDS-resident
- * generic kernel) */
+ * generic kernel). Above 33 values the folded lines, where every dim has
+ * them: the registers of one FFT leave two or three waves to a SIMD there
+ * (P = 64: 88 us a launch, folded 58; 15 x 60: 2200, 1109; 15 x 35: 1031,
+ * 819); up to 33 one FFT is as fast or faster (30 x 30: 498, folded 579). */
 static int spatial_lines(AgdWin const *W) {
-  int d, m = 0;
+  int d, m = 0, folded = 1;
   if (W->S > AGD_LINES_VALUES || (size_t)2 * W->S * 8 > LDS_BUDGET) return 0;
-  for (d = 0; d < W->nsp; d++)
+  for (d = 0; d < W->nsp; d++) {
     if (W->P[d] > m) m = W->P[d];
+    if (line_factor(W->P[d]) == 0) folded = 0;
+  }
+  if (folded && m > 33) return AGD_FACTORED;
   return line_instance(m, kSpatialInst);
 }
 
@@ -1192,7 +1214,7 @@ static void time_lines(AgdWin *W) {
   if (line_instance(W->gm1 > W->gm2 ? W->gm1 : W->gm2, kTimeInst) == 0) W->gm1 = W->gm2 = 0;
 }
 static int time_instance(AgdWin const *W) {
-  if (W->gm3) return AGD_TIME_FACTORED;
+  if (W->gm3) return AGD_FACTORED;
   return W->gm2 ? line_instance(W->gm1 > W->gm2 ? W->gm1 : W->gm2, kTimeInst) : 0;
 }
 
@@ -1251,7 +1273,7 @@ static int default_nk(int a, int b, int Ft) {
  * size, and the generic kernels' LDS size in *lds_sp. */
 static int spatial_tasks(AgdProblem *p, AgdClass *cls, int ncls, int const *nk_req,
                          vec *tasks, size_t *lds_sp) {
-  int c, w;
+  int c, w, d;
   for (c = 0; c < ncls; c++) {
     AgdClass *cl = cls + c;
     int *wpos = (int *)malloc(((size_t)p->n_win + 1) * sizeof(int));
@@ -1294,7 +1316,8 @@ static int spatial_tasks(AgdProblem *p, AgdClass *cls, int ncls, int const *nk_r
         if (l > cl->lds) cl->lds = l;
       } else if (cl->hb) {
         int const last = W->P[W->nsp - 1];
-        size_t const l = (size_t)nk * (W->S / last) * (last | 1) * 8;
+        size_t l = (size_t)nk * (W->S / last) * (last | 1) * 8;
+        for (d = 0; cl->hb == AGD_FACTORED && d < W->nsp; d++) l += (size_t)W->P[d] * 8;
         if (l > cl->lds) cl->lds = l;
       } else if ((size_t)2 * nk * W->S * 8 > *lds_sp) {
         *lds_sp = (size_t)2 * nk * W->S * 8;
@@ -1634,7 +1657,10 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
         /* coefficients of the run-time sized kernels */
         int m1, m2;
         spatial_key(W, &m1, &m2);
-        for (d = 0; d < nsp; d++) W->sdft[d] = 0;
+        for (d = 0; d < nsp; d++) {
+          W->sdft[d] = 0;
+          W->sfac[d] = line_factor(W->P[d]);
+        }
         if (m1 == 0 && spatial_lines(W))
           for (d = 0; d < nsp; d++)
             if ((W->sdft[d] = dft_get(&ps, W->P[d])) < 0) goto err;

@@ -27,8 +27,8 @@
 #define AGD_MAXSTAGE 24  /* FFT stages per plan */
 /* model values of one task of the run-time sized spatial kernel at most */
 #define AGD_LINES_VALUES 4096
-/* AgdClass.hb of the run-time sized time kernels on register FFTs */
-#define AGD_TIME_FACTORED 4
+/* AgdClass.hb of the run-time sized kernels on short register FFTs */
+#define AGD_FACTORED 4
 /* half lengths Mr / 2 of the wavelet convolution with a compile-time kernel
  * (k_wavelet_t); the host prefers them to the smallest 7-smooth length when
  * one is at most 25% longer */
@@ -65,6 +65,7 @@ typedef struct {
    * dim; Pt = gm1 * gm2 * gm3 in register FFTs, or (gm3 0) gm1 * gm2 in
    * lines with their coefficients' offsets (gm2 0: none) */
   int sdft[AGD_MAXSP];
+  int sfac[AGD_MAXSP]; /* first factor of P, both up to 16 (1: P up to 16) */
   int gm1, gm2, gm3;
   int tdft1, tdft2;
   int64_t x_off;         /* model offset (complex) */
@@ -94,7 +95,7 @@ typedef struct {
                    classes: 1 when the time transform is specialised too */
   int hb;       /* run-time sized kernels: coefficient pairs held per line
                    (half the longest line, rounded up to an instance), or
-                   AGD_TIME_FACTORED */
+                   AGD_FACTORED */
   int var;      /* time classes: forward kernel variant (0 register
                    prefetch, 1 lean tile); spatial classes: unused */
   int ntw;      /* time classes: most time windows of a block */

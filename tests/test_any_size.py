@@ -1,7 +1,7 @@
 """The run-time sized transforms (agd_general.hip): windows of any length.
 
 A line of P padded values is held by one thread in registers: P up to 33,
-49, 65, 97 and 129 by kernel instance (the windows below sit on both sides
+49, 65, 97 and 129 by kernel instance, or folded into two short transforms (the windows below sit on both sides
 of each edge, at lengths with a register codelet and at primes), longer ones
 go to the LDS-resident kernels; the time transform takes Pt in two or three
 register FFTs of up to 16 values, else in lines M1 M2, with M1 = 1 for a
@@ -74,6 +74,18 @@ PHASES = [((19, 384), (18, 192)), ((7, 227), (6, 114)), ((22, 547), (22, 274)),
 
 @pytest.mark.parametrize("shape,windows", PHASES, ids=[str(w[1]) for _, w in PHASES])
 def test_time_phases_match_fp64_oracle(shape, windows):
+    test_any_window_length_matches_fp64_oracle(shape, windows)
+
+
+# spatial lines in two register FFTs: lengths 35, 64, 225 and 240, along a
+# strided dim, along both, and beside a dim that one FFT holds
+FOLDED = [((42, 64), (28, 20)), ((51, 80), (51, 20)), ((180, 40), (180, 10)), ((288, 40), (192, 10)),
+          ((54, 18, 40), (36, 12, 10)), ((60, 48, 40), (40, 32, 10)), ((8, 64, 40), (8, 64, 10)),
+          ((3, 4, 42, 40), (2, 4, 28, 10))]
+
+
+@pytest.mark.parametrize("shape,windows", FOLDED, ids=["x".join(map(str, w)) for _, w in FOLDED])
+def test_folded_lines_match_fp64_oracle(shape, windows):
     test_any_window_length_matches_fp64_oracle(shape, windows)
 
 
