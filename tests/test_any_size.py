@@ -89,6 +89,17 @@ def test_folded_lines_match_fp64_oracle(shape, windows):
     test_any_window_length_matches_fp64_oracle(shape, windows)
 
 
+# the specialised time kernels (whole tiles of 16 traces, Wt 64 to 512) beside
+# run-time sized spatial ones: folded, one FFT a line, 3-D, LDS-resident
+MIXED = [((96, 192), (48, 64)), ((18, 18, 320), (12, 12, 128)), ((4, 12, 4, 256), (4, 8, 4, 256)),
+         ((16, 768), (16, 512)), ((272, 160), (272, 64)), ((6, 12, 96), (4, 8, 64))]
+
+
+@pytest.mark.parametrize("shape,windows", MIXED, ids=["x".join(map(str, w)) for _, w in MIXED])
+def test_specialised_time_with_any_spatial_size(shape, windows):
+    test_any_window_length_matches_fp64_oracle(shape, windows)
+
+
 @pytest.mark.parametrize("nan", [False, True])
 @pytest.mark.parametrize("shape,windows", [((61, 300), (24, 106)), ((17, 34, 160), (16, 33, 64))])
 def test_fused_iterations_match_separate_transforms(shape, windows, nan, monkeypatch):
