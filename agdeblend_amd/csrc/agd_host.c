@@ -1218,6 +1218,18 @@ static int time_instance(AgdWin const *W) {
   return W->gm2 ? line_instance(W->gm1 > W->gm2 ? W->gm1 : W->gm2, kTimeInst) : 0;
 }
 
+/* whether W is served by time class cl (own: a specialised time length
+ * beside a spatial size without a specialised kernel; the interface treats
+ * such a class as generic: no factors to set, one run per block) */
+static int time_match(AgdWin const *W, AgdClass const *cl) {
+  int a, b, s0, s1;
+  time_key(W, &a, &b);
+  if (a != cl->p0 || b != cl->p1) return 0;
+  if (!a) return time_instance(W) == cl->hb;
+  spatial_key(W, &s0, &s1);
+  return (s0 == 0) == cl->own;
+}
+
 /* Planes per task of the run-time sized spatial kernel: at most
  * AGD_LINES_VALUES values (a block holds them in registers and LDS, four
  * blocks to a CU). A stage of l lines costs ceil(l / 64) waves of lines of
@@ -1392,7 +1404,7 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
   vec_init(&tc, sizeof(AgdClass));
   for (w = 0; w < p->n_win; w++) {
     AgdWin const *W = &p->win[w];
-    int a, b, tm, tn, hb, found = 0;
+    int a, b, tm, tn, hb, own, found = 0;
     AgdClass *cl = (AgdClass *)sc.p;
     spatial_key(W, &a, &b);
     time_key(W, &tm, &tn);
@@ -1408,13 +1420,14 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
       n->tb = a ? tm > 0 : 0;
       n->hb = hb;
     }
+    own = tm > 0 && a == 0;
     a = tm;
     b = tn;
     hb = a ? 0 : time_instance(W);
     found = 0;
     cl = (AgdClass *)tc.p;
     for (c = 0; c < (int)tc.n; c++)
-      if (cl[c].p0 == a && cl[c].p1 == b && cl[c].hb == hb) found = 1;
+      if (cl[c].p0 == a && cl[c].p1 == b && cl[c].hb == hb && cl[c].own == own) found = 1;
     if (!found) {
       AgdClass *n = (AgdClass *)vec_push(&tc);
       if (n == NULL) return 1;
@@ -1422,6 +1435,7 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
       n->p0 = a;
       n->p1 = b;
       n->hb = hb;
+      n->own = own;
     }
   }
   if (spatial_tasks(p, (AgdClass *)sc.p, (int)sc.n, NULL, tasks, &lds_sp)) return 1;
@@ -1442,16 +1456,14 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
       size_t need = 0;
       for (w = 0; w < p->n_win; w++) {
         AgdWin const *W = &p->win[w];
-        int a, b;
         size_t l;
-        time_key(W, &a, &b);
-        if (a != cl->p0 || b != cl->p1 || (!a && time_instance(W) != cl->hb)) continue;
+        if (!time_match(W, cl)) continue;
         if (cl->hb) {
           l = time_lines_lds(W);
-        } else if (a) {
+        } else if (cl->p0) {
           /* the forward's tile, work buffer and roots (the larger of the
            * two kernels; the launcher passes each its own size) */
-          size_t const M = (size_t)a * b;
+          size_t const M = (size_t)cl->p0 * cl->p1;
           l = 8 * (2 * TIME_TILE * (M + 1) + 2 * M + 1);
         } else {
           int const M = (W->Pt % 2 == 0 && W->Pt >= 4) ? W->Pt / 2 : W->Pt;
@@ -1467,13 +1479,12 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
     cl->begin = (int)tblocks->n;
     for (w = 0; w < p->n_win; w++) {
       AgdWin const *W = &p->win[w];
-      int a, b, t0, q, parts;
+      int t0, q, parts;
       wpos[w] = (int)tblocks->n - cl->begin;
-      time_key(W, &a, &b);
-      if (a != cl->p0 || b != cl->p1 || (!a && time_instance(W) != cl->hb)) continue;
+      if (!time_match(W, cl)) continue;
       /* the specialised kernels' blocks split the window's time windows
        * into nearly equal runs of at most tw_run (0: one run) */
-      parts = (a && tw_run > 0) ? (W->ntw + tw_run - 1) / tw_run : 1;
+      parts = (cl->p0 && !cl->own && tw_run > 0) ? (W->ntw + tw_run - 1) / tw_run : 1;
       if (parts < 1) parts = 1;
       for (t0 = 0; t0 < W->ntr; t0 += tb) {
         for (q = 0; q < parts; q++) {
@@ -2832,7 +2843,7 @@ static int autotune_time(AgdProblem *p, int reps) {
     int const M = cl->p0 * cl->p1;
     int b0 = cl->p0, b1 = cl->p1, bv = cl->var, v;
     double best_t = -1.0;
-    if (cl->p0 == 0) continue;
+    if (cl->p0 == 0 || cl->own) continue;
     /* untimed pass first: the first candidate timed on a cold device
      * (clocks, caches, code) would read slow */
     if (time_time(p, reps) < 0.0) return 1;
@@ -2867,7 +2878,7 @@ EXPORT int agdx_n_time_classes(AgdProblem const *p) { return p->n_tclass; }
 
 EXPORT int agdx_set_time_factors(AgdProblem *p, int c, int m1, int m2) {
   int k;
-  if (c < 0 || c >= p->n_tclass || p->tclass[c].p0 == 0 ||
+  if (c < 0 || c >= p->n_tclass || p->tclass[c].p0 == 0 || p->tclass[c].own ||
       m1 * m2 != p->tclass[c].p0 * p->tclass[c].p1) {
     fprintf(stderr, "ERROR: no time class %d of half length %d\n", c, m1 * m2);
     return 1;
@@ -2883,7 +2894,8 @@ EXPORT int agdx_set_time_factors(AgdProblem *p, int c, int m1, int m2) {
 }
 
 EXPORT int agdx_set_time_variant(AgdProblem *p, int c, int var) {
-  if (c < 0 || c >= p->n_tclass || p->tclass[c].p0 == 0 || (var != 0 && var != 1)) {
+  if (c < 0 || c >= p->n_tclass || p->tclass[c].p0 == 0 || p->tclass[c].own ||
+      (var != 0 && var != 1)) {
     fprintf(stderr, "ERROR: no specialised time class %d or variant %d\n", c, var);
     return 1;
   }
@@ -2894,7 +2906,7 @@ EXPORT int agdx_set_time_variant(AgdProblem *p, int c, int var) {
 EXPORT int agdx_time_variants(AgdProblem const *p, int *out) {
   int c;
   if (out)
-    for (c = 0; c < p->n_tclass; c++) out[c] = p->tclass[c].var;
+    for (c = 0; c < p->n_tclass; c++) out[c] = p->tclass[c].own ? 0 : p->tclass[c].var;
   return p->n_tclass;
 }
 
@@ -2909,8 +2921,8 @@ EXPORT int agdx_time_factors(AgdProblem const *p, int *out) {
   int c;
   if (out)
     for (c = 0; c < p->n_tclass; c++) {
-      out[2 * c] = p->tclass[c].p0;
-      out[2 * c + 1] = p->tclass[c].p1;
+      out[2 * c] = p->tclass[c].own ? 0 : p->tclass[c].p0;
+      out[2 * c + 1] = p->tclass[c].own ? 0 : p->tclass[c].p1;
     }
   return p->n_tclass;
 }

@@ -69,9 +69,11 @@ static inline int allow_lds(void const *f) {
 // time windows are a serial chain, so below TIME_SPLIT_BLOCKS blocks (six
 // per CU) the chip waits on it: 30 blocks of 9 time windows (256 x 1024
 // line, windows 32 x 256) took 27 us forward and 34 adjoint as one run each
-// and take 15 and 11 split, 236 blocks of 14 (1510 x 1251 line) 113 and 132
-// against 67 and 52; above it the runs would only repeat the forward's
-// carry windows.
+// and take 15 and 11 split, 236 blocks of 14 (1510 x 1251 line, in lines; in
+// register FFTs 41 and 32) 113 and 132 against 67 and 52; above it the runs
+// would only repeat the forward's carry windows. (1024 to 3072 blocks, rounded
+// up or down, move that line by -6 % and 2400 x 2048 in windows of 48 x 64 by
+// +10 %, others by less than their spread.)
 static inline unsigned time_split(AgdClass const &c, int n, int least) {
   int const want = (TIME_SPLIT_BLOCKS + n - 1) / n, most = c.ntw / least;
   int const r = want < most ? want : most;

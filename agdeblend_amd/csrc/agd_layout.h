@@ -96,6 +96,7 @@ typedef struct {
   int hb;       /* run-time sized kernels: coefficient pairs held per line
                    (half the longest line, rounded up to an instance), or
                    AGD_FACTORED */
+  int own;      /* time classes: 1 beside a generic spatial size */
   int var;      /* time classes: forward kernel variant (0 register
                    prefetch, 1 lean tile); spatial classes: unused */
   int ntw;      /* time classes: most time windows of a block */

@@ -2034,7 +2034,6 @@ int agdu_upsample_bwd(void const *dy, void *dx, int N, int D, int H, int W, int 
     fprintf(stderr, "ERROR: upsampling channels %d at %d of %d unsupported\n", C, c0, Cy);
     return 1;
   }
-  int64_t const total = (int64_t)N * D * H * W * (C / 8);
   return row_launch("upsample_bwd", k_upsample_bwd, N, D, H, W * (int64_t)(C / 8), stream,
                     (uint16_t const *)dy, (uint16_t *)dx, D, H, W, C, Cy, c0);
 }
