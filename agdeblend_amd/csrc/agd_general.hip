@@ -15,7 +15,7 @@
 // traffic inside a line, and no dependence on how P factors. Lengths without
 // a prime factor above 13 take a register FFT instead (codelets). Where that
 // FFT's registers would leave few waves (above 33), P = A B folds into two
-// short ones in place (HB = 0).
+// short ones in place (FOLD).
 //
 // Measured (MI355X) on a 45 x 333 x 1500 volume in two patches, windows of
 // 17-18 x 24-25 x 200 (P = 22, 23 x 30, 32, Pt = 250; model 1.15 GB), us per
@@ -182,7 +182,7 @@ __device__ __forceinline__ int quot(int a, float inv) {
 typedef int i4 __attribute__((ext_vector_type(AGD_MAXSP)));
 struct Planes {
   int nsp, rows, pitch, rp;  // rows of a plane, row pitch, values of a plane
-  i4 ext, str, P, W, A;      // per space dim (A: lines' first factor, HB = 0)
+  i4 ext, str, P, W, A;      // per space dim (A: lines' first factor)
 };
 
 // a[i], uniform, without indexed registers
@@ -220,7 +220,7 @@ __device__ __forceinline__ bool codelets(int P, int total, int st, At const &at)
   return codelets<S, Ps...>(P, total, st, at);
 }
 
-// The two phases of a folded line (lines, HB = 0): `total` lines at(i), each
+// The two phases of a folded line (lines): `total` lines at(i), each
 // B (A) short lines, threads over (short line, line). rt[m] = exp(-2 pi i m /
 // P).
 template <int S, class At>
@@ -292,7 +292,7 @@ __device__ __forceinline__ void fold_b(int A, int B, int total, float it, int st
 
 // transforms every line along dim d of the nk planes in place; the other
 // dims run over their current extents g.ext
-template <int HB, int S>
+template <int HB, bool FOLD, int S>
 __device__ __forceinline__ void lines(float2 *sm, Planes &g, int nk, int d, int nin, int nout,
                                       cfloat const *tab, float2 const *rt) {
   int cnt = 1;
@@ -317,21 +317,23 @@ __device__ __forceinline__ void lines(float2 *sm, Planes &g, int nk, int d, int 
     }
     return At{sm + off};
   };
+  // P = A B in place: A-point lines over k1 (k = k1 B + k2), twiddle,
+  // then B-point lines over k2, whose outputs n = n1 + A n2 go to their
+  // natural places once every thread has read its inputs
+  // (1-D lines of 64 on 59 windows of 51 x 126: one FFT in 228 registers
+  // left 8 waves to a CU, three of four idle, 88 us; now 58, for 27 at
+  // the cached copy rate; the block's four barriers bound it)
+  int const A = pick(g.A, d), B = quot(P, 1.f / (float)A);
+  auto const fold = [&] {
+    float const it = 1.f / (float)total;
+    fold_a<S, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>(A, B, total, it, st, nin, at, rt);
+    __syncthreads();
+    fold_b<S, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>(A, B, total, it, st, nout, at);
+    if constexpr (HB > 0) fold_b<S, 25>(A, B, total, it, st, nout, at);
+    __syncthreads();
+  };
   if constexpr (HB == 0) {
-    if (!codelets<S, 2, 3, 4, 5, 7, 8, 9, 10, 12, 13, 14, 15>(P, total, st, at)) {
-      // P = A B in place: A-point lines over k1 (k = k1 B + k2), twiddle,
-      // then B-point lines over k2, whose outputs n = n1 + A n2 go to their
-      // natural places once every thread has read its inputs
-      // (1-D lines of 64 on 59 windows of 51 x 126: one FFT in 228 registers
-      // left 8 waves to a CU, three of four idle, 88 us; now 58, for 27 at
-      // the cached copy rate; the block's four barriers bound it)
-      int const A = pick(g.A, d), B = quot(P, 1.f / (float)A);
-      float const it = 1.f / (float)total;
-      fold_a<S, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>(A, B, total, it, st, nin, at, rt);
-      __syncthreads();
-      fold_b<S, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>(A, B, total, it, st, nout, at);
-      __syncthreads();
-    }
+    if (!codelets<S, 2, 3, 4, 5, 7, 8, 9, 10, 12, 13, 14, 15>(P, total, st, at)) fold();
   } else {
     bool done = codelets<S, 8, 9, 10, 12, 13, 14, 15>(P, total, st, at);
     if constexpr (HB >= 16)
@@ -340,6 +342,11 @@ __device__ __forceinline__ void lines(float2 *sm, Planes &g, int nk, int d, int 
       if (!done) done = codelets<S, 35, 39, 40, 42, 44, 45, 48, 49>(P, total, st, at);
     if constexpr (HB >= 32)
       if (!done) done = codelets<S, 50, 52, 54, 55, 60, 63, 64, 65>(P, total, st, at);
+    if constexpr (FOLD)
+      if (!done && A > 1) {
+        fold();
+        done = true;
+      }
     if (!done)
       block_lines<HB, S>(total, st, P, nin, nout, tab, at,
                          [&](At const &z, int q, float2 v) { z.p[q * st] = v; });
@@ -402,7 +409,9 @@ __device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr,
 
 // mode -1: forward only (X -> U); 0..5 as k_adj_spatial_t's MODE, followed by
 // the forward transform of the new model when fuse is set
-template <int HB>
+// FOLD: lines that have two factors fold (HB = 0: all that one FFT does not
+// hold; HB = 16: those beyond its codelets, beside lengths that do not fold)
+template <int HB, bool FOLD>
 __global__ __launch_bounds__(
     256, HB == 0 ? 5 : HB <= 16 ? 4 : HB <= 24 ? 3 : HB <= 32 ? 2 : 1) void k_spatial_g(
     AgdWin const *__restrict__ wins, AgdTask const *__restrict__ tasks, int task0,
@@ -438,10 +447,10 @@ __global__ __launch_bounds__(
   int64_t const uoff = w.u_off + (int64_t)t.tw * ((w.ntr + 15) / 16) * w.Ft * 16;
   float2 *const x = X + w.x_off + ((int64_t)t.tw * w.Ft + t.k0) * w.S;
   int const total = nk * w.S;
-  // HB = 0: the dims' roots [P_0] .. [P_{n-1}] after the planes (the longest
+  // FOLD: the dims' roots [P_0] .. [P_{n-1}] after the planes (the longest
   // task's: a class's LDS is its largest)
   float2 *const rts = sm + nk * g.rp;
-  if constexpr (HB == 0) {
+  if constexpr (FOLD) {
     int o = 0;
     for (int d = 0; d < nsp; ++d) {
       int const P = w.P[d];
@@ -464,7 +473,7 @@ __global__ __launch_bounds__(
     tiles_copy<true>(sm, g, w.ntr, w.Ft, const_cast<float2 *>(V) + uoff, t.k0, nk);
     __syncthreads();
     for (int d = nsp - 1; d >= 0; --d)
-      lines<HB, -1>(sm, g, nk, d, pick(g.W, d), pick(g.P, d), uniform(dft, w.sdft[d]), rt(d));
+      lines<HB, FOLD, -1>(sm, g, nk, d, pick(g.W, d), pick(g.P, d), uniform(dft, w.sdft[d]), rt(d));
   }
   // value i sits at LDS offset i + (row of i) (pitch - last)
   {
@@ -530,7 +539,7 @@ __global__ __launch_bounds__(
 #pragma unroll
     for (int e = 0; e < AGD_MAXSP; ++e) g.ext[e] = g.P[e];
     for (int d = 0; d < nsp; ++d)
-      lines<HB, +1>(sm, g, nk, d, pick(g.P, d), pick(g.W, d), uniform(dft, w.sdft[d]), rt(d));
+      lines<HB, FOLD, +1>(sm, g, nk, d, pick(g.P, d), pick(g.W, d), uniform(dft, w.sdft[d]), rt(d));
     tiles_copy<false>(sm, g, w.ntr, w.Ft, U + uoff, t.k0, nk);
   }
 }
@@ -854,15 +863,15 @@ __global__ __launch_bounds__(256, time_waves(HB)) void k_adj_time_g(
 // Instances of the run-time sized kernels by the coefficient pairs HB a line
 // holds in registers (lengths up to 2 HB + 1): the fewer, the more waves
 // share a SIMD. The host picks the smallest that fits a window's lines.
-template <int HB>
+template <int HB, bool FOLD>
 static int launch_spatial_g(AgdDev const *g, AgdClass const &c, float2 *X, float alpha,
                             float lamb, int mode, int fuse) {
-  static int const lds_ok = allow_lds((void const *)k_spatial_g<HB>);
+  static int const lds_ok = allow_lds((void const *)k_spatial_g<HB, FOLD>);
   (void)lds_ok;
   int first;
   int const n = class_range(g, c, &first);
   if (n <= 0) return 0;
-  return launch(mode < 0 ? "fwd_spatial" : "adj_spatial", k_spatial_g<HB>, dim3(n),
+  return launch(mode < 0 ? "fwd_spatial" : "adj_spatial", k_spatial_g<HB, FOLD>, dim3(n),
                 dim3(NTHR), c.lds, g->win, g->tasks, first, g->dft, g->plans,
                 (float2 const *)g->roots, (float2 const *)g->V, X,
                 (float2 *)g->U, alpha, lamb, (float const *)g->lamb_dev, mode, fuse, g->scalar);
@@ -870,13 +879,14 @@ static int launch_spatial_g(AgdDev const *g, AgdClass const &c, float2 *X, float
 int spatial_general(AgdDev const *g, AgdClass const &c, float2 *X, float alpha,
                            float lamb, int mode, int fuse) {
   switch (c.hb) {
-    case AGD_FACTORED: return launch_spatial_g<0>(g, c, X, alpha, lamb, mode, fuse);
-    case 8: return launch_spatial_g<8>(g, c, X, alpha, lamb, mode, fuse);
-    case 16: return launch_spatial_g<16>(g, c, X, alpha, lamb, mode, fuse);
-    case 24: return launch_spatial_g<24>(g, c, X, alpha, lamb, mode, fuse);
-    case 32: return launch_spatial_g<32>(g, c, X, alpha, lamb, mode, fuse);
-    case 48: return launch_spatial_g<48>(g, c, X, alpha, lamb, mode, fuse);
-    default: return launch_spatial_g<64>(g, c, X, alpha, lamb, mode, fuse);
+    case AGD_FACTORED: return launch_spatial_g<0, true>(g, c, X, alpha, lamb, mode, fuse);
+    case AGD_FOLDED_LINES: return launch_spatial_g<16, true>(g, c, X, alpha, lamb, mode, fuse);
+    case 8: return launch_spatial_g<8, false>(g, c, X, alpha, lamb, mode, fuse);
+    case 16: return launch_spatial_g<16, false>(g, c, X, alpha, lamb, mode, fuse);
+    case 24: return launch_spatial_g<24, false>(g, c, X, alpha, lamb, mode, fuse);
+    case 32: return launch_spatial_g<32, false>(g, c, X, alpha, lamb, mode, fuse);
+    case 48: return launch_spatial_g<48, false>(g, c, X, alpha, lamb, mode, fuse);
+    default: return launch_spatial_g<64, false>(g, c, X, alpha, lamb, mode, fuse);
   }
 }
 template <int HB>

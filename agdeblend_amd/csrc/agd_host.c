@@ -1132,8 +1132,8 @@ static int const kSpatialInst[] = {8, 16, 24, 32, 48, 64, 0};
 static int const kTimeInst[] = {8, 16, 32, 64, 0};
 
 /* The first factor of the padded length P in two register FFTs of 4 to 16
- * values, the smaller longest one first; 1 where one FFT holds it (the list
- * of lines<0>), 0 where none does */
+ * values, the smaller longest one first, or 5 of 5 x 25; 1 where one FFT
+ * holds it (the list of lines<0>), 0 where none does */
 static int line_factor(int P) {
   int a;
   if (P <= 5 || P == 7 || P == 8 || P == 9 || P == 10 || (P >= 12 && P <= 15)) return P > 1;
@@ -1144,7 +1144,7 @@ static int line_factor(int P) {
         if (P % c == 0 && c * c >= P) b = c;
       return b;
     }
-  return 0;
+  return P == 125 ? 5 : 0;
 }
 
 /* coefficient pairs of the window's run-time sized spatial kernel: lines up
@@ -1152,15 +1152,24 @@ static int line_factor(int P) {
  * generic kernel). Above 33 values the folded lines, where every dim has
  * them: the registers of one FFT leave two or three waves to a SIMD there
  * (P = 64: 88 us a launch, folded 58; 15 x 60: 2200, 1109; 15 x 35: 1031,
- * 819); up to 33 one FFT is as fast or faster (30 x 30: 498, folded 579). */
+ * 819); up to 33 one FFT is as fast or faster (30 x 30: 498, folded 579).
+ * Above 65, where no FFT holds a line, also beside dims up to 33 that do not
+ * fold, and 125 = 5 x 25 (whose 25 values take more registers): as plain sums
+ * such lines were slower than the LDS-resident kernel's radix passes. A line
+ * of windows of 100, us an iteration: LDS-resident 223, plain sum 660, folded
+ * 89; 96 x 14 (120 x 18): 5230, 11680, 1430; 60 x 14 (75 x 18): 3070, 1240,
+ * 780. (50 x 14, 63 x 18: one FFT 758, not moved.) */
 static int spatial_lines(AgdWin const *W) {
-  int d, m = 0, folded = 1;
+  int d, m = 0, whole = 0, wide = 0;
   if (W->S > AGD_LINES_VALUES || (size_t)2 * W->S * 8 > LDS_BUDGET) return 0;
   for (d = 0; d < W->nsp; d++) {
+    int const f = line_factor(W->P[d]);
     if (W->P[d] > m) m = W->P[d];
-    if (line_factor(W->P[d]) == 0) folded = 0;
+    if (f == 0 && W->P[d] > whole) whole = W->P[d];
+    if (f > 0 && W->P[d] / f > 16) wide = 1;
   }
-  if (folded && m > 33) return AGD_FACTORED;
+  if (m > 33 && whole == 0 && !wide) return AGD_FACTORED;
+  if (m > 65 && whole <= 33) return AGD_FOLDED_LINES;
   return line_instance(m, kSpatialInst);
 }
 
@@ -1329,7 +1338,7 @@ static int spatial_tasks(AgdProblem *p, AgdClass *cls, int ncls, int const *nk_r
       } else if (cl->hb) {
         int const last = W->P[W->nsp - 1];
         size_t l = (size_t)nk * (W->S / last) * (last | 1) * 8;
-        for (d = 0; cl->hb == AGD_FACTORED && d < W->nsp; d++) l += (size_t)W->P[d] * 8;
+        for (d = 0; cl->hb < kSpatialInst[0] && d < W->nsp; d++) l += (size_t)W->P[d] * 8;
         if (l > cl->lds) cl->lds = l;
       } else if ((size_t)2 * nk * W->S * 8 > *lds_sp) {
         *lds_sp = (size_t)2 * nk * W->S * 8;

@@ -29,6 +29,9 @@
 #define AGD_LINES_VALUES 4096
 /* AgdClass.hb of the run-time sized kernels on short register FFTs */
 #define AGD_FACTORED 4
+/* AgdClass.hb of the spatial kernel whose long lines are folded and whose
+ * other lines hold 16 coefficient pairs */
+#define AGD_FOLDED_LINES 5
 /* half lengths Mr / 2 of the wavelet convolution with a compile-time kernel
  * (k_wavelet_t); the host prefers them to the smallest 7-smooth length when
  * one is at most 25% longer */
@@ -65,7 +68,7 @@ typedef struct {
    * dim; Pt = gm1 * gm2 * gm3 in register FFTs, or (gm3 0) gm1 * gm2 in
    * lines with their coefficients' offsets (gm2 0: none) */
   int sdft[AGD_MAXSP];
-  int sfac[AGD_MAXSP]; /* first factor of P, both up to 16 (1: P up to 16) */
+  int sfac[AGD_MAXSP]; /* first factor of P, A B = P (1: P one FFT, 0: does not fold) */
   int gm1, gm2, gm3;
   int tdft1, tdft2;
   int64_t x_off;         /* model offset (complex) */
@@ -95,7 +98,7 @@ typedef struct {
                    classes: 1 when the time transform is specialised too */
   int hb;       /* run-time sized kernels: coefficient pairs held per line
                    (half the longest line, rounded up to an instance), or
-                   AGD_FACTORED */
+                   AGD_FACTORED, AGD_FOLDED_LINES */
   int own;      /* time classes: 1 beside a generic spatial size */
   int var;      /* time classes: forward kernel variant (0 register
                    prefetch, 1 lean tile); spatial classes: unused */
