@@ -357,14 +357,20 @@ __device__ __forceinline__ void lines(float2 *sm, Planes &g, int nk, int d, int 
 }
 
 // the window's traces of the nk planes, between LDS and the tiles of U / V
-// ([tile of 16 traces][Ft][16] per time window): a tile's nk planes are
-// contiguous. Indices by reciprocals (an integer division is ~35
+// ([tile of 16 traces][Ft][16] per time window, the last tile as wide as its
+// traces): a tile's nk planes are contiguous. Indices by reciprocals (an integer division is ~35
 // instructions, and these two loops were most of the kernel's).
-template <bool TO_LDS>
-__device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr, int Ft,
+// PART: the last tile is narrower (k = rem m / 2^16 divides its rows: rem <
+// 4096 and widths up to 16). Windows of 17 x 23 and 16 x 24 traces: 944 and
+// 477 us an iteration, 934 and 470 with last tiles padded to 16; as two loops
+// 1036 and 531.
+template <bool TO_LDS, bool PART>
+__device__ __forceinline__ void tiles_loop(float2 *sm, Planes const &g, int ntr, int Ft,
                                            float2 *utw, int k0, int nk) {
   constexpr int NB = 8;  // loads issued together
-  int const span = nk * 16, total = ((ntr + 15) >> 4) * span;
+  int const full = ntr >> 4, wl = ntr & 15;  // whole tiles, width of the last
+  int const span = nk * 16, total = nk * ntr;
+  unsigned const ml = PART ? 65535u / (unsigned)wl + 1u : 0u, Ft16 = (unsigned)Ft * 16u;
   float const is = 1.f / (float)span;
   float const i1 = 1.f / (float)g.W.y, i2 = 1.f / (float)g.W.z, i3 = 1.f / (float)g.W.w;
   for (int i0 = threadIdx.x; i0 < total; i0 += NB * 256) {
@@ -373,10 +379,12 @@ __device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr,
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       int const i = min(i0 + b * 256, total - 1);
-      int const t = quot(i, is), rem = i - t * span, k = rem >> 4;
-      int const tr = t * 16 + (rem & 15);
-      float2 *const u = utw + ((unsigned)t * (unsigned)Ft + (unsigned)k0) * 16u + (unsigned)rem;
-      int r = tr, off = k * g.rp;
+      int const t = quot(i, is), rem = i - t * span;
+      bool const last = PART && t >= full;
+      int const wt = last ? wl : 16;
+      int const k = PART ? (int)(__umul24(rem, last ? ml : 4096u) >> 16) : rem >> 4;
+      int r = t * 16 + rem - __mul24(k, wt), off = k * g.rp;
+      float2 *const u = utw + (__umul24(t, Ft16) + __umul24(k0, wt) + (unsigned)rem);
       if (g.nsp > 3) {
         int const q = quot(r, i3);
         off += (r - q * g.W.w) * g.str.w;
@@ -393,7 +401,7 @@ __device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr,
         r = q;
       }
       off += r * g.str.x;
-      lp[b] = i0 + b * 256 < total && tr < ntr ? off : -1;
+      lp[b] = i0 + b * 256 < total ? off : -1;
       if (TO_LDS)
         v[b] = *u;
       else if (lp[b] >= 0)
@@ -405,6 +413,14 @@ __device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr,
         if (lp[b] >= 0) sm[lp[b]] = v[b];
     }
   }
+}
+template <bool TO_LDS>
+__device__ __forceinline__ void tiles_copy(float2 *sm, Planes const &g, int ntr, int Ft,
+                                           float2 *utw, int k0, int nk) {
+  if (ntr & 15)
+    tiles_loop<TO_LDS, true>(sm, g, ntr, Ft, utw, k0, nk);
+  else
+    tiles_loop<TO_LDS, false>(sm, g, ntr, Ft, utw, k0, nk);
 }
 
 // mode -1: forward only (X -> U); 0..5 as k_adj_spatial_t's MODE, followed by
@@ -444,7 +460,7 @@ __global__ __launch_bounds__(
       }
     }
   }
-  int64_t const uoff = w.u_off + (int64_t)t.tw * ((w.ntr + 15) / 16) * w.Ft * 16;
+  int64_t const uoff = w.u_off + t.tw * (int64_t)w.uplane;
   float2 *const x = X + w.x_off + ((int64_t)t.tw * w.Ft + t.k0) * w.S;
   int const total = nk * w.S;
   // FOLD: the dims' roots [P_0] .. [P_{n-1}] after the planes (the longest
@@ -568,6 +584,11 @@ __global__ __launch_bounds__(
 // ---------------------------------------------------------------------------
 constexpr int kPairs = 8;
 __host__ __device__ constexpr int time_pitch(int Pt) { return (Pt + 3) / 8 * 8 + 4; }
+
+// rows of a tile are as wide as its nt traces: the pair p of row k starts at
+// value k nt + 2 p, which item i = k np + p (np pairs a row, the last of an odd
+// nt a single) finds at 2 i - (nt odd ? k : 0). 16 bytes aligned to 8.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
 
 struct TimeTables {
   float2 *Z, *TW, *TW2;
@@ -701,24 +722,31 @@ __global__ __launch_bounds__(256, time_waves(HB)) void k_fwd_time_g(
   for (int i = tid; i < Wt; i += 256) TP[i] = tapers[w.tt_off + i];
   for (int i = tid; i < 2 * kPairs * half; i += 256) CA[i] = 0.f;
   float *const Tb = T + w.t_off + (int64_t)t0 * nconv;
-  int64_t const tw_step = (int64_t)((w.ntr + 15) / 16) * Ft * kPairs;  // float4
-  float4 const *tile = (float4 const *)(U + w.u_off) + (int64_t)(t0 / 16) * Ft * kPairs;
+  float2 const *const tile = U + w.u_off + (int64_t)t0 * Ft;
+  int const np = (nt + 1) >> 1, odd = nt & 1;
+  float const ip = 1.f / (float)np;
   for (int tw = twa; tw < tw1; ++tw) {
-    float4 const *u = tile + tw * tw_step;
+    float2 const *const u = tile + tw * (int64_t)w.uplane;
     // Hermitian halves of both traces of a pair into z = x_a + i x_b (DC and
-    // Nyquist imaginary parts ignored); traces beyond the window are zero
+    // Nyquist imaginary parts ignored). A single's partner is zero: its load
+    // takes the next row's first value, or the one past the tile (the buffer
+    // has one more). Pairs beyond np transform what the tile holds, unused.
     constexpr int NB = 4;
-    for (int i0 = tid; i0 < Ft * kPairs; i0 += NB * 256) {
-      float4 v[NB];
+    for (int i0 = tid; i0 < Ft * np; i0 += NB * 256) {
+      f4u v[NB];
+      int kk[NB];
 #pragma unroll
-      for (int b = 0; b < NB; ++b) v[b] = u[min(i0 + b * 256, Ft * kPairs - 1)];
+      for (int b = 0; b < NB; ++b) {
+        int const i = min(i0 + b * 256, Ft * np - 1);
+        kk[b] = quot(i, ip);
+        v[b] = *(f4u const *)(u + 2 * i - (odd ? kk[b] : 0));
+      }
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         int const i = i0 + b * 256;
-        if (i < Ft * kPairs) {
-          int const k = i >> 3, p = i & 7;
+        if (i < Ft * np) {
+          int const k = kk[b], p = i - k * np;
           float2 xa = make_float2(v[b].x, v[b].y), xb = make_float2(v[b].z, v[b].w);
-          if (2 * p >= nt) xa = make_float2(0.f, 0.f);
           if (2 * p + 1 >= nt) xb = make_float2(0.f, 0.f);
           if (k == 0 || 2 * k == N) xa.y = xb.y = 0.f;
           float2 *const z = t.Z + p * pitch;
@@ -817,8 +845,9 @@ __global__ __launch_bounds__(256, time_waves(HB)) void k_adj_time_g(
   };
   float const two = plain ? 1.f : 2.f;
   int const kmax2 = (N - 1) / 2;
-  float4 *const vt = (float4 *)(V + w.u_off) + (int64_t)(t0 / 16) * Ft * kPairs;
-  int64_t const tw_step = (int64_t)((w.ntr + 15) / 16) * Ft * kPairs;
+  float2 *const vt = V + w.u_off + (int64_t)t0 * Ft;
+  int const np = (nt + 1) >> 1, odd = nt & 1;
+  float const ip = 1.f / (float)np;
   for (int tw = tw0; tw < tw1; ++tw) {
     constexpr int NB = 2;
     for (int s0 = lane; s0 < N; s0 += 64 * NB) {
@@ -847,14 +876,18 @@ __global__ __launch_bounds__(256, time_waves(HB)) void k_adj_time_g(
     __syncthreads();
     time_fft<HB, -1>(t, pitch, M1, M2, M3, dft, w.tdft1, w.tdft2);
     // half spectra of the two real traces of a pair, x2 on the interior bins
-    float4 *const vo = vt + tw * tw_step;
-    for (int i = tid; i < Ft * kPairs; i += 256) {
-      int const k = i >> 3, p = i & 7;
+    float2 *const vo = vt + tw * (int64_t)w.uplane;
+    for (int i = tid; i < Ft * np; i += 256) {
+      int const k = quot(i, ip), p = i - k * np;
       float2 const *const z = t.Z + p * pitch;
       float2 const z1 = z[t.pos[k]], z2 = z[t.pos[k ? N - k : 0]];
       float const s = (k >= 1 && k <= kmax2) ? 0.5f * two : 0.5f;
-      vo[i] = make_float4(s * (z1.x + z2.x), s * (z1.y - z2.y), s * (z1.y + z2.y),
-                          s * (z2.x - z1.x));
+      float2 *const o = vo + 2 * i - (odd ? k : 0);
+      float2 const va = make_float2(s * (z1.x + z2.x), s * (z1.y - z2.y));
+      if (2 * p + 1 < nt)
+        *(f4u *)o = f4u{va.x, va.y, s * (z1.y + z2.y), s * (z2.x - z1.x)};
+      else
+        *o = va;
     }
     __syncthreads();
   }

@@ -1111,9 +1111,6 @@ static void time_sizes(AgdWin const *W, int *m1, int *m2) {
  * of 6 x 8 x 10 x 128 took 141 and 109 us a launch in the run-time sized
  * kernels, 108 and 79 in these. */
 #define TIME_TILE 16
-static int tile_traces(AgdWin const *W) {
-  return (W->ntr + TIME_TILE - 1) / TIME_TILE * TIME_TILE;
-}
 static void time_key(AgdWin const *W, int *m1, int *m2) {
   *m1 = 0;
   *m2 = 0;
@@ -1693,11 +1690,18 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
             goto err;
         }
       }
+      /* time windows start at whole cache lines of U and V where that is at
+       * most 1.5 % of them, else at whole 16-byte loads */
+      {
+        int64_t const n = (int64_t)W->Ft * W->ntr, align = n >= 1024 ? 16 : 2;
+        W->uplane = (int)((n + align - 1) / align * align);
+        uo = (uo + align - 1) / align * align;
+      }
       W->x_off = xo;
       W->u_off = uo;
       W->t_off = to;
       xo += (int64_t)W->ntw * W->Ft * W->S;
-      uo += (int64_t)W->ntw * W->Ft * tile_traces(W);
+      uo += (int64_t)W->ntw * W->uplane;
       to += (int64_t)W->ntr * W->nconv;
       /* time taper */
       W->tt_off = (int)tapers.n;
@@ -1856,8 +1860,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
       p->n_chunk = 0;
       p->chunk[0] = 0;
       for (w = 0; w < p->n_win; w++) {
-        double const b =
-            2.0 * 8.0 * (double)p->win[w].ntw * p->win[w].Ft * tile_traces(&p->win[w]);
+        double const b = 2.0 * 8.0 * (double)p->win[w].ntw * p->win[w].uplane;
         if (cap > 0.0 && acc > 0.0 && acc + b > cap) {
           p->chunk[++p->n_chunk] = w;
           acc = 0.0;
@@ -1896,6 +1899,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
       p->dev.wavelet_mh = mh > 0 ? mh : 0;
     }
     p->dev.X = (float *)dev_alloc(p, (size_t)xo * 8);
+    uo += 1; /* the 16-byte load of a last single trace */
     p->dev.U = (float *)dev_alloc(p, (size_t)uo * 8);
     p->dev.V = (float *)dev_alloc(p, (size_t)uo * 8);
     p->u_len = (size_t)uo;

@@ -116,12 +116,12 @@ __device__ __forceinline__ float2 rootf(float2 const *roots, int n, int e, int s
   return w;
 }
 
-// element of trace tr, plane k of one time window's tiles of U / V
-// ([tile of 16 traces][Ft][16]); ntr16: complex values per plane and window
-__device__ __forceinline__ int64_t tile_at(int tr, int k, int Ft) {
-  return ((int64_t)(tr >> 4) * Ft + k) * 16 + (tr & 15);
+// element of trace tr, plane k of one time window of U / V (tiles of 16 of
+// the window's ntr traces, [Ft][16]; the last as wide as its traces)
+__device__ __forceinline__ int64_t tile_at(int tr, int k, int Ft, int ntr) {
+  int const t0 = tr & ~15;
+  return (int64_t)t0 * Ft + (int64_t)k * min(16, ntr - t0) + (tr - t0);
 }
-__device__ __forceinline__ int tile_plane(int ntr) { return (ntr + 15) & ~15; }
 
 // ---------------------------------------------------------------------------
 // Line geometries for LDS-resident batched FFTs
@@ -319,8 +319,7 @@ __global__ __launch_bounds__(NTHR) void k_fwd_spatial(
       r /= w.W[e];
       off += c * g.str[e];
     }
-    U[w.u_off + (int64_t)t.tw * w.Ft * tile_plane(ntr) + tile_at(tr, t.k0 + k, w.Ft)] =
-        A[k * S + off];
+    U[w.u_off + t.tw * (int64_t)w.uplane + tile_at(tr, t.k0 + k, w.Ft, ntr)] = A[k * S + off];
   }
 }
 
@@ -353,11 +352,11 @@ __global__ __launch_bounds__(NTHR) void k_fwd_time(
   for (int i = threadIdx.x; i < tb * Wt; i += blockDim.x) acc[i] = 0.f;
   LinesContig lc{M};
   for (int tw = 0; tw < w.ntw; ++tw) {
-    float2 const *u = U + w.u_off + (int64_t)tw * Ft * tile_plane(w.ntr);
+    float2 const *u = U + w.u_off + tw * (int64_t)w.uplane;
     for (int i = threadIdx.x; i < Ft * tb; i += blockDim.x) {
       int const k = i / tb;
       int const j = i - k * tb;
-      H[j * Ft + k] = j < nt ? u[tile_at(t0 + j, k, Ft)] : make_float2(0.f, 0.f);
+      H[j * Ft + k] = j < nt ? u[tile_at(t0 + j, k, Ft, w.ntr)] : make_float2(0.f, 0.f);
     }
     __syncthreads();
     if (even) {
@@ -609,7 +608,7 @@ __global__ __launch_bounds__(NTHR) void k_adj_time(
         X.x *= 2.f;
         X.y *= 2.f;
       }
-      V[w.u_off + (int64_t)tw * Ft * tile_plane(w.ntr) + tile_at(t0 + j, k, Ft)] = X;
+      V[w.u_off + tw * (int64_t)w.uplane + tile_at(t0 + j, k, Ft, w.ntr)] = X;
     }
     (void)out;
     __syncthreads();
@@ -659,8 +658,7 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial(
       r /= w.W[e];
       off += c * g.str[e];
     }
-    A[k * S + off] =
-        V[w.u_off + (int64_t)t.tw * w.Ft * tile_plane(ntr) + tile_at(tr, t.k0 + k, w.Ft)];
+    A[k * S + off] = V[w.u_off + t.tw * (int64_t)w.uplane + tile_at(tr, t.k0 + k, w.Ft, ntr)];
   }
   __syncthreads();
   for (int e = 0; e < nsp; ++e) g.ext[e] = w.W[e];
@@ -1288,18 +1286,20 @@ __device__ __forceinline__ void rows_fft(float2 *sm, int nk) {
 }
 
 // LDS rows of the nk planes <-> the window traces of the planes in U / V
-// ([tile of 16 traces][Ft][16] per time window); the element order below
-// walks each tile's nk planes contiguously. Utw points at the task's time
-// window, k0 is its first plane.
+// ([tile of 16 traces][Ft][16] per time window; one tile as wide as the
+// window where it has fewer); the element order below walks each tile's nk
+// planes contiguously. Utw points at the task's time window, k0 is its first
+// plane.
 template <int P0, int P1, bool TO_LDS>
 __device__ __forceinline__ void planes_copy(float2 *sm, float2 *Utw, int k0, int Ft, int nk) {
   constexpr int LD = P1 + 1;
   constexpr int W0 = win_len<P0>();
   constexpr int W1 = win_len<P1>();
-  constexpr int NTR = W0 * W1, NTP = (NTR + TG - 1) / TG * TG;  // padded last tile
+  constexpr int TW = W0 * W1 < TG ? W0 * W1 : TG;
+  static_assert(W0 * W1 % TW == 0, "tiles of one width");
   constexpr int NB = 8;  // loads issued together per thread
-  int const span = nk * TG;
-  int const total = nk * NTP;
+  int const span = nk * TW;
+  int const total = nk * W0 * W1;
   for (int base = 0; base < total; base += NB * NTHR) {
     float2 v[NB];
     int lp[NB];
@@ -1308,22 +1308,20 @@ __device__ __forceinline__ void planes_copy(float2 *sm, float2 *Utw, int k0, int
       int const i = min(base + (int)threadIdx.x + b * NTHR, total - 1);
       int const g = i / span;
       int const rem = i - g * span;
-      int const k = rem / TG;
-      int const tr = g * TG + (rem - k * TG);
+      int const k = rem / TW;
+      int const tr = g * TW + (rem - k * TW);
       int const row = tr / W1;
       lp[b] = (k * W0 + row) * LD + (tr - row * W1);
-      if (NTR < NTP && tr >= NTR) lp[b] = -1;
-      float2 *u = Utw + ((int64_t)g * Ft + k0) * TG + rem;
+      float2 *u = Utw + ((int64_t)g * Ft + k0) * TW + rem;
       if (TO_LDS)
         v[b] = *u;
-      else if (base + (int)threadIdx.x + b * NTHR < total && (NTR == NTP || lp[b] >= 0))
+      else if (base + (int)threadIdx.x + b * NTHR < total)
         *u = sm[lp[b]];
     }
     if (TO_LDS) {
 #pragma unroll
       for (int b = 0; b < NB; ++b)
-        if (base + (int)threadIdx.x + b * NTHR < total && (NTR == NTP || lp[b] >= 0))
-          sm[lp[b]] = v[b];
+        if (base + (int)threadIdx.x + b * NTHR < total) sm[lp[b]] = v[b];
     }
   }
 }
@@ -1354,8 +1352,7 @@ __global__ __launch_bounds__(NTHR) void k_fwd_spatial_t(
   __syncthreads();
   rows_fft<P0, P1, +1, P1, W1>(sm, nk);
   __syncthreads();
-  planes_copy<P0, P1, false>(sm, U + w.u_off + (int64_t)t.tw * w.Ft * tile_plane(W0 * W1),
-                             t.k0, w.Ft, nk);
+  planes_copy<P0, P1, false>(sm, U + w.u_off + t.tw * (int64_t)w.uplane, t.k0, w.Ft, nk);
 }
 
 // Adjoint spatial transform of V and the model update, by MODE:
@@ -1384,7 +1381,7 @@ __global__ __launch_bounds__(NTHR) void k_adj_spatial_t(
   AgdTask const t = tasks[task0 + blockIdx.x];
   AgdWin const &w = wins[t.win];
   int const nk = t.nk;
-  int64_t const uoff = w.u_off + (int64_t)t.tw * w.Ft * tile_plane(W0 * W1);
+  int64_t const uoff = w.u_off + t.tw * (int64_t)w.uplane;
   planes_copy<P0, P1, true>(sm, const_cast<float2 *>(V) + uoff, t.k0, w.Ft, nk);
   __syncthreads();
   rows_fft<P0, P1, -1, W1, P1>(sm, nk);

@@ -9,10 +9,11 @@
  *             fastest). Mathematically the same coefficients as the
  *             reference's [ntw][P_space...][Ft] (fk.c:256-262), transposed.
  *   inter U   complex float, per window [ntw][ntr/16][Ft][16] (tiles of 16
- *             traces, one contiguous block per time window; the last tile of
- *             a window is padded): spatial transform of X cropped to the
- *             window's traces (forward), or time transform of the traces
- *             (adjoint); ntr = prod(W_space).
+ *             traces, the last of a window as wide as its traces; one
+ *             contiguous block of uplane >= Ft ntr values per time window):
+ *             spatial transform of X cropped to the window's traces
+ *             (forward), or time transform of the traces (adjoint);
+ *             ntr = prod(W_space).
  *   traces T  float, per window [ntr][nconv] (the reference's temp_1 trace
  *             buffer, fk.c:330-331).
  *   record    float, all (channel, interval) continuous records concatenated
@@ -61,6 +62,7 @@ typedef struct {
   int wplan;             /* wavelet convolution FFT plan (-1: none) */
   int wplan_full;        /* plan holding roots of the wavelet length M */
   int wM;                /* wavelet convolution length M */
+  int uplane;            /* complex values of a time window in U / V */
   int trace0;            /* first global window-trace index */
   int patch;
   float scaler;          /* 1 / sqrt(prod P) (fk.c:157-163) */
