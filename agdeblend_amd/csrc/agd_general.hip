@@ -926,7 +926,7 @@ template <int HB>
 static int launch_fwd_time_g(AgdDev const *g, AgdClass const &c, int first, int n) {
   static int const lds_ok = allow_lds((void const *)k_fwd_time_g<HB>);
   (void)lds_ok;
-  return launch("fwd_time", k_fwd_time_g<HB>, dim3(n, time_split(c, n, 2)), dim3(NTHR), c.lds, g->win,
+  return launch("fwd_time", k_fwd_time_g<HB>, dim3(n, time_split(g, c, n, 2)), dim3(NTHR), c.lds, g->win,
                 g->tblocks, first, g->dft, g->plans, (float2 const *)g->roots, g->tapers,
                 g->tscale, (float2 const *)g->U, g->T);
 }
@@ -944,7 +944,7 @@ static int launch_adj_time_g(AgdDev const *g, AgdClass const &c, int first, int 
                              float const *Tin, int plain) {
   static int const lds_ok = allow_lds((void const *)k_adj_time_g<HB>);
   (void)lds_ok;
-  return launch("adj_time", k_adj_time_g<HB>, dim3(n, time_split(c, n, 1)), dim3(NTHR), c.lds, g->win,
+  return launch("adj_time", k_adj_time_g<HB>, dim3(n, time_split(g, c, n, 1)), dim3(NTHR), c.lds, g->win,
                 g->tblocks, first, g->dft, g->plans, (float2 const *)g->roots, g->tapers,
                 g->tscale, g->went, (float const *)g->r, Tin, (float2 *)g->V, plain,
                 first == c.begin && n == c.count ? g->tadj : (int const *)nullptr);

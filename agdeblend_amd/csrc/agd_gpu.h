@@ -47,6 +47,7 @@ typedef struct {
   int const *tadj;            /* [n_tblocks]: per class, its blocks sorted by
                                  their first trace (the adjoint time kernel's
                                  launch order), or NULL */
+  int split_time;             /* launches of few time blocks split their runs */
   int tb;                     /* traces per time block */
   size_t lds_time;            /* bytes (generic kernel) */
   AgdClass const *tclass;     /* host array */

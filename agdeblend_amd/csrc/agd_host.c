@@ -1392,7 +1392,8 @@ static int *adj_time_order(AgdProblem const *p, int const *tb, int n) {
  * window's (0) for the whole-volume order, where each block streams a
  * trace tile's time windows one after the other; 4 with the window-chunk
  * order (AGD_CHUNK_MB), so that a chunk of a few windows still makes
- * thousands of blocks; AGD_TIME_TW overrides */
+ * thousands of blocks; AGD_TIME_TW overrides, and its runs are not split
+ * further by launches of few blocks (dev.split_time) */
 static int time_tw_run(void) {
   char const *e = getenv("AGD_TIME_TW");
   if (e != NULL) return atoi(e) > 0 ? atoi(e) : 0;
@@ -1874,6 +1875,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
     if (p->tblk == NULL) goto err;
     memcpy(p->tblk, tblocks.p, tblocks.n * TB_INTS * sizeof(int));
     p->n_tblk = (int)tblocks.n;
+    p->dev.split_time = getenv("AGD_TIME_TW") == NULL;
     p->dev.n_tblocks = (int)tblocks.n;
     {
       int *ord = adj_time_order(p, (int const *)tblocks.p, (int)tblocks.n);

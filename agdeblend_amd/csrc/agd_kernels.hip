@@ -2486,13 +2486,13 @@ int agdg_fwd_time(AgdDev const *g) {
 #define FT_CASE(a, b)                                                                   \
     if (!done && c.p0 == a && c.p1 == b) {                                              \
       if (n > 0 && c.var == 0 &&                                                        \
-          launch("fwd_time", k_fwd_time_t<a, b, false>, dim3(n, time_split(c, n, 2)),                        \
+          launch("fwd_time", k_fwd_time_t<a, b, false>, dim3(n, time_split(g, c, n, 2)), \
                  dim3(time_threads<a * b>()), fwd_time_lds<a * b, false>(), g->win,     \
                  g->tblocks, first, g->plans, (float2 const *)g->roots, g->tapers,      \
                  g->tscale, (float2 const *)g->U, g->T))                                \
         return 1;                                                                       \
       if (n > 0 && c.var != 0 &&                                                        \
-          launch("fwd_time", k_fwd_time_t<a, b, true>, dim3(n, time_split(c, n, 2)),                         \
+          launch("fwd_time", k_fwd_time_t<a, b, true>, dim3(n, time_split(g, c, n, 2)), \
                  dim3(time_threads<a * b>()), fwd_time_lds<a * b, true>(), g->win,      \
                  g->tblocks, first, g->plans, (float2 const *)g->roots, g->tapers,      \
                  g->tscale, (float2 const *)g->U, g->T))                                \
@@ -2543,7 +2543,7 @@ int agdg_adj_time(AgdDev const *g, float const *Tin, int plain) {
 #define AT_CASE(a, b)                                                                   \
     if (!done && c.p0 == a && c.p1 == b) {                                              \
       if (n > 0 &&                                                                      \
-          launch("adj_time", k_adj_time_t<a, b>, dim3(n, time_split(c, n, 1)),                                 \
+          launch("adj_time", k_adj_time_t<a, b>, dim3(n, time_split(g, c, n, 1)), \
                  dim3(time_threads<a * b>()), adj_time_lds<a * b>(), g->win, g->tblocks,   \
                  first, g->plans, (float2 const *)g->roots, g->tapers, g->tscale,        \
                  g->went, (float const *)g->r, Tin, (float2 *)g->V, plain,              \

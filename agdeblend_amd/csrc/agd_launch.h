@@ -73,8 +73,10 @@ static inline int allow_lds(void const *f) {
 // register FFTs 41 and 32) 113 and 132 against 67 and 52; above it the runs
 // would only repeat the forward's carry windows. (1024 to 3072 blocks, rounded
 // up or down, move that line by -6 % and 2400 x 2048 in windows of 48 x 64 by
-// +10 %, others by less than their spread.)
-static inline unsigned time_split(AgdClass const &c, int n, int least) {
+// +10 %, others by less than their spread.) Runs given by AGD_TIME_TW are
+// left as they are.
+static inline unsigned time_split(AgdDev const *g, AgdClass const &c, int n, int least) {
+  if (!g->split_time) return 1;
   int const want = (TIME_SPLIT_BLOCKS + n - 1) / n, most = c.ntw / least;
   int const r = want < most ? want : most;
   return r > 1 ? r : 1;

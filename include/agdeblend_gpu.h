@@ -156,7 +156,8 @@ int agdx_set_time_factors(AgdProblem *p, int c, int m1, int m2);
  * trace, and the run [tw0, tw1) of the window's time windows the block
  * transforms (all of them unless AGD_TIME_TW sets runs, or the window-chunk
  * order AGD_CHUNK_MB does: runs of 4; a launch of few blocks splits them
- * further, with the same results). Returns their number. */
+ * further, with the same results, but not those of AGD_TIME_TW, whose 0 is
+ * one run). Returns their number. */
 int agdx_time_blocks(AgdProblem const *p, int *out);
 /* Device copy of the patch data set by agdx_set_data: all patches
  * concatenated in patch order, agdx_data_len floats (valid until
