@@ -1225,8 +1225,9 @@ static int time_instance(AgdWin const *W) {
 }
 
 /* whether W is served by time class cl (own: a specialised time length
- * beside a spatial size without a specialised kernel; the interface treats
- * such a class as generic: no factors to set, one run per block) */
+ * beside a spatial size without a specialised kernel, whose factors, variant
+ * and runs are not the caller's to set, as before these windows had a
+ * specialised time kernel) */
 static int time_match(AgdWin const *W, AgdClass const *cl) {
   int a, b, s0, s1;
   time_key(W, &a, &b);
@@ -2921,7 +2922,7 @@ EXPORT int agdx_set_time_variant(AgdProblem *p, int c, int var) {
 EXPORT int agdx_time_variants(AgdProblem const *p, int *out) {
   int c;
   if (out)
-    for (c = 0; c < p->n_tclass; c++) out[c] = p->tclass[c].own ? 0 : p->tclass[c].var;
+    for (c = 0; c < p->n_tclass; c++) out[c] = p->tclass[c].var;
   return p->n_tclass;
 }
 

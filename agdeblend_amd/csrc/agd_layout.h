@@ -101,7 +101,8 @@ typedef struct {
   int hb;       /* run-time sized kernels: coefficient pairs held per line
                    (half the longest line, rounded up to an instance), or
                    AGD_FACTORED, AGD_FOLDED_LINES */
-  int own;      /* time classes: 1 beside a generic spatial size */
+  int own;      /* time classes: 1 for a specialised kernel beside a spatial
+                   size without one (default factors and variant, one run) */
   int var;      /* time classes: forward kernel variant (0 register
                    prefetch, 1 lean tile); spatial classes: unused */
   int ntw;      /* time classes: most time windows of a block */

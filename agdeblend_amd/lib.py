@@ -348,8 +348,8 @@ class Problem:
         return nk[:n].tolist(), ms[:n].tolist()
 
     def time_factors(self):
-        """Current (M1, M2) factorization of each time class ((0, 0): the
-        generic kernels)."""
+        """Current (M1, M2) factorization of each time class ((0, 0): it
+        cannot be set, see agdx_time_factors)."""
         n = int(self.L.agdx_n_time_classes(self.h))
         out = np.zeros(2 * max(n, 1), C_INT)
         self.L.agdx_time_factors(self.h, _p(out))

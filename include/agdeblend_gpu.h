@@ -139,14 +139,19 @@ int agdx_autotune(AgdProblem *p, int reps, int *nk_out, double *ms_out);
 /* Number of spatial kernel classes of the problem. */
 int agdx_n_spatial_classes(AgdProblem const *p);
 /* Number of time kernel classes, and their current (M1, M2) factorization
- * (out: 2 ints per class, or NULL; 0 0 for classes of the generic
- * kernels). agdx_time_factors returns the number of classes. */
+ * (out: 2 ints per class, or NULL; 0 0 for classes whose factorization
+ * cannot be set: those of the generic kernels, and specialised ones of
+ * windows whose spatial size has no specialised kernel, which keep the
+ * default factors and variant, form a class of their own and have one run
+ * per block; the autotuner leaves both alone). agdx_time_factors returns
+ * the number of classes. */
 int agdx_n_time_classes(AgdProblem const *p);
 int agdx_time_factors(AgdProblem const *p, int *out);
 /* Forward time kernel variant per time class (out: one int per class):
  * 0 the next time window's tile prefetched into registers, 1 the lean tile
  * (one LDS tile for input and transform, the carry in registers, more
- * blocks per CU). The autotuner times both with every factorization. */
+ * blocks per CU). The autotuner times both with every factorization. Set for
+ * classes whose factorization can be set; 0 for the generic kernels. */
 int agdx_time_variants(AgdProblem const *p, int *out);
 int agdx_set_time_variant(AgdProblem *p, int c, int var);
 /* Sets time class c to the factorization m1 x m2 of its half length (one
@@ -154,10 +159,11 @@ int agdx_set_time_variant(AgdProblem *p, int c, int var);
 int agdx_set_time_factors(AgdProblem *p, int c, int m1, int m2);
 /* The time kernels' blocks, 4 ints each into out (or NULL): window, first
  * trace, and the run [tw0, tw1) of the window's time windows the block
- * transforms (all of them unless AGD_TIME_TW sets runs, or the window-chunk
- * order AGD_CHUNK_MB does: runs of 4; a launch of few blocks splits them
- * further, with the same results, but not those of AGD_TIME_TW, whose 0 is
- * one run). Returns their number. */
+ * transforms: all of them, unless the block's class has a factorization to
+ * set and AGD_TIME_TW sets runs, or the window-chunk order AGD_CHUNK_MB does
+ * (runs of 4). A launch of few blocks splits the runs of every class further,
+ * with the same results, unless AGD_TIME_TW is set (0: one run). Returns
+ * their number. */
 int agdx_time_blocks(AgdProblem const *p, int *out);
 /* Device copy of the patch data set by agdx_set_data: all patches
  * concatenated in patch order, agdx_data_len floats (valid until
