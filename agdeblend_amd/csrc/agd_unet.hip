@@ -1453,99 +1453,110 @@ __device__ __forceinline__ u16x8 ld8(uint16_t const *p) { return *(u16x8 const *
 __device__ __forceinline__ void st8(uint16_t *p, u16x8 v) { *(u16x8 *)p = v; }
 
 // The training pass's resampling kernels take one (n, d, h) row of their
-// output per block: the row's indices are divided out once, a thread only
-// splits its (w, 8 channels), in 32 bits (64-bit divisions per 16 bytes had
-// these kernels at 1.5 TB/s).
+// output per block (and, beyond the grid, the rows a grid apart): the row's
+// indices are divided out once, a thread only splits its (w, 8 channels), in
+// 32 bits (64-bit divisions per 16 bytes had these kernels at 1.5 TB/s); I is
+// 64 bits for tensors whose rows or items per row need them.
 struct Row {
   int n, d, h;
 };
-__device__ __forceinline__ Row out_row(int D, int H) {
-  int const r = blockIdx.x, nd = r / H;
-  return Row{nd / D, nd % D, r - nd * H};
+template <typename I>
+__device__ __forceinline__ Row out_row(I row, int D, int H) {
+  I const nd = row / (I)H, n = nd / (I)D;
+  return Row{(int)n, (int)(nd - n * D), (int)(row - nd * H)};
 }
 
 // 2x2x2 max pool: y[n][d][h][w][c] over x[n][2d..][2h..][2w..][c]; arg holds
 // the winning offset (first maximum in (a, b, e) order). D, H, W: of y
+template <typename I>
 __global__ void k_maxpool(uint16_t const *__restrict__ x, uint16_t *__restrict__ y,
-                          uint8_t *__restrict__ arg, int D, int H, int W, int C) {
-  Row const r = out_row(D, H);
-  int const C8 = C / 8;
-  int64_t const out0 = (int64_t)blockIdx.x * W * C;
-  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
-    int const w = idx / C8, c = (idx - w * C8) * 8;
-    float best[8];
-    int barg[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      best[k] = -INFINITY;
-      barg[k] = 0;
-    }
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-      int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
-      int64_t const row = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
-      u16x8 const v = ld8(x + (row * 2 * W + 2 * w + e) * C + c);
+                          uint8_t *__restrict__ arg, int D, int H, int W, int C, I rows) {
+  I const C8 = C / 8;
+  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
+    Row const r = out_row(row, D, H);
+    int64_t const out0 = (int64_t)row * W * C;
+    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
+      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
+      float best[8];
+      int barg[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        float const f = bf2f(v[k]);
-        if (f > best[k]) {
-          best[k] = f;
-          barg[k] = o;
+        best[k] = -INFINITY;
+        barg[k] = 0;
+      }
+#pragma unroll
+      for (int o = 0; o < 8; ++o) {
+        int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
+        int64_t const xrow = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
+        u16x8 const v = ld8(x + (xrow * 2 * W + 2 * w + e) * C + c);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          float const f = bf2f(v[k]);
+          if (f > best[k]) {
+            best[k] = f;
+            barg[k] = o;
+          }
         }
       }
-    }
-    u16x8 out;
-    u8x8 ar;
+      u16x8 out;
+      u8x8 ar;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      out[k] = f2bf(best[k]);
-      ar[k] = (uint8_t)barg[k];
+      for (int k = 0; k < 8; ++k) {
+        out[k] = f2bf(best[k]);
+        ar[k] = (uint8_t)barg[k];
+      }
+      st8(y + out0 + (int64_t)idx * 8, out);
+      *(u8x8 *)(arg + out0 + (int64_t)idx * 8) = ar;
     }
-    st8(y + out0 + (int64_t)idx * 8, out);
-    *(u8x8 *)(arg + out0 + (int64_t)idx * 8) = ar;
   }
 }
 
 // gradient of the pooling, D, H, W: of dx. add (or NULL): a second gradient of
 // the pooled tensor's input, its channels [c0, c0 + C) of Ca, added in fp32 and
 // rounded once (as k_copy_channels mode 1 on the written dx)
+template <typename I>
 __global__ void k_maxpool_bwd(uint16_t const *__restrict__ dy, uint8_t const *__restrict__ arg,
                               uint16_t *__restrict__ dx, int D, int H, int W, int C,
-                              uint16_t const *__restrict__ add, int Ca, int c0) {
-  Row const r = out_row(D, H);
-  int const C8 = C / 8;
-  int64_t const prow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
-  int const mine = ((r.d & 1) << 2) | ((r.h & 1) << 1);
-  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
-    int const w = idx / C8, c = (idx - w * C8) * 8;
-    int64_t const o = (prow * (W / 2) + w / 2) * C + c;
-    u16x8 const g = ld8(dy + o);
-    u8x8 const a = *(u8x8 const *)(arg + o);
-    u16x8 out;
+                              uint16_t const *__restrict__ add, int Ca, int c0, I rows) {
+  I const C8 = C / 8;
+  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
+    Row const r = out_row(row, D, H);
+    int64_t const prow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
+    int const mine = ((r.d & 1) << 2) | ((r.h & 1) << 1);
+    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
+      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
+      int64_t const o = (prow * (W / 2) + w / 2) * C + c;
+      u16x8 const g = ld8(dy + o);
+      u8x8 const a = *(u8x8 const *)(arg + o);
+      u16x8 out;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) out[k] = a[k] == (mine | (w & 1)) ? g[k] : (uint16_t)0;
-    if (add != nullptr) {
-      u16x8 const s = ld8(add + ((int64_t)blockIdx.x * W + w) * Ca + c0 + c);
+      for (int k = 0; k < 8; ++k) out[k] = a[k] == (mine | (w & 1)) ? g[k] : (uint16_t)0;
+      if (add != nullptr) {
+        u16x8 const s = ld8(add + ((int64_t)row * W + w) * Ca + c0 + c);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) out[k] = f2bf(bf2f(s[k]) + bf2f(out[k]));
+        for (int k = 0; k < 8; ++k) out[k] = f2bf(bf2f(s[k]) + bf2f(out[k]));
+      }
+      st8(dx + ((int64_t)row * W + w) * C + c, out);
     }
-    st8(dx + ((int64_t)blockIdx.x * W + w) * C + c, out);
   }
 }
 
 // y = [upsample(xu), xs]: the nearest x2 upsampling of xu (CU channels) and xs
 // (CS channels) side by side, whole voxels of y [n][D][H][W][CU + CS] at a time
+template <typename I>
 __global__ void k_concat_up(uint16_t const *__restrict__ xu, uint16_t const *__restrict__ xs,
-                            uint16_t *__restrict__ y, int D, int H, int W, int CU, int CS) {
-  Row const r = out_row(D, H);
-  int const C8 = (CU + CS) / 8;
-  int64_t const urow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
-  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
-    int const w = idx / C8, c = (idx - w * C8) * 8;
-    uint16_t const *const q = c < CU
-                                  ? xu + (urow * (W / 2) + w / 2) * CU + c
-                                  : xs + ((int64_t)blockIdx.x * W + w) * CS + (c - CU);
-    st8(y + (int64_t)blockIdx.x * W * (CU + CS) + (int64_t)idx * 8, ld8(q));
+                            uint16_t *__restrict__ y, int D, int H, int W, int CU, int CS, I rows) {
+  I const C8 = (CU + CS) / 8;
+  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
+    Row const r = out_row(row, D, H);
+    int64_t const urow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
+    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
+      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
+      uint16_t const *const q = c < CU
+                                    ? xu + (urow * (W / 2) + w / 2) * CU + c
+                                    : xs + ((int64_t)row * W + w) * CS + (c - CU);
+      st8(y + (int64_t)row * W * (CU + CS) + (int64_t)idx * 8, ld8(q));
+    }
   }
 }
 
@@ -1572,27 +1583,30 @@ __global__ void k_upsample(uint16_t const *__restrict__ x, uint16_t *__restrict_
 
 // gradient of the upsampling: dx[v][c] = sum of the 8 children's
 // dy[..][c0 + c], in a fixed order; accumulated in fp32. D, H, W: of dx
+template <typename I>
 __global__ void k_upsample_bwd(uint16_t const *__restrict__ dy, uint16_t *__restrict__ dx, int D,
-                               int H, int W, int C, int Cy, int c0) {
-  Row const r = out_row(D, H);
-  int const C8 = C / 8;
-  for (int idx = threadIdx.x; idx < W * C8; idx += blockDim.x) {
-    int const w = idx / C8, c = (idx - w * C8) * 8;
-    float s[8];
+                               int H, int W, int C, int Cy, int c0, I rows) {
+  I const C8 = C / 8;
+  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
+    Row const r = out_row(row, D, H);
+    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
+      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
+      float s[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) s[k] = 0.f;
+      for (int k = 0; k < 8; ++k) s[k] = 0.f;
 #pragma unroll
-    for (int o = 0; o < 8; ++o) {
-      int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
-      int64_t const row = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
-      u16x8 const g = ld8(dy + (row * 2 * W + 2 * w + e) * Cy + c0 + c);
+      for (int o = 0; o < 8; ++o) {
+        int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
+        int64_t const yrow = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
+        u16x8 const g = ld8(dy + (yrow * 2 * W + 2 * w + e) * Cy + c0 + c);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) s[k] += bf2f(g[k]);
+        for (int k = 0; k < 8; ++k) s[k] += bf2f(g[k]);
+      }
+      u16x8 out;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) out[k] = f2bf(s[k]);
+      st8(dx + (int64_t)row * W * C + (int64_t)idx * 8, out);
     }
-    u16x8 out;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) out[k] = f2bf(s[k]);
-    st8(dx + (int64_t)blockIdx.x * W * C + (int64_t)idx * 8, out);
   }
 }
 
@@ -1723,18 +1737,18 @@ static inline int64_t blocks_capped(int64_t n, int t) {
   return b < (1 << 20) ? b : (1 << 20);
 }
 
-// a kernel with one block per (n, d, h) row of `items` 16-byte items
-template <typename K, typename... A>
-static int row_launch(char const *name, K kernel, int N, int D, int H, int64_t items,
+// a kernel of (n, d, h) rows of `items` 16-byte items, a block each up to 2^20
+// blocks (a launch holds less than 2^32 threads); small: the instance with
+// 32-bit indices, large: 64-bit
+template <typename K, typename L, typename... A>
+static int row_launch(char const *name, K small, L large, int N, int D, int H, int64_t items,
                       void *stream, A... args) {
   int64_t const rows = (int64_t)N * D * H;
-  if (rows > 0x7fffffff || items > 0x7fffffff / 2) {
-    fprintf(stderr, "ERROR: %s of %lld rows of %lld items unsupported\n", name, (long long)rows,
-            (long long)items);
-    return 1;
-  }
   int const t = items >= UT ? UT : (int)((items + 63) / 64 * 64);
-  return ulaunch(name, kernel, dim3((unsigned)rows), dim3(t > 0 ? t : 64), stream, args...);
+  dim3 const grid((unsigned)(rows < (1 << 20) ? rows : 1 << 20)), block(t > 0 ? t : 64);
+  if (rows < 0x7fffffff && items < 0x7fffffff)
+    return ulaunch(name, small, grid, block, stream, args..., (unsigned)rows);
+  return ulaunch(name, large, grid, block, stream, args..., (uint64_t)rows);
 }
 
 extern "C" {
@@ -1975,7 +1989,8 @@ int agdu_maxpool(void const *x, void *y, void *arg, int N, int D, int H, int W, 
     fprintf(stderr, "ERROR: channel count %d is not a multiple of 8\n", C);
     return 1;
   }
-  return row_launch("maxpool", k_maxpool, N, D / 2, H / 2, (W / 2) * (int64_t)(C / 8), stream,
+  return row_launch("maxpool", k_maxpool<unsigned>, k_maxpool<uint64_t>, N, D / 2, H / 2,
+                    (W / 2) * (int64_t)(C / 8), stream,
                     (uint16_t const *)x, (uint16_t *)y, (uint8_t *)arg, D / 2, H / 2, W / 2, C);
 }
 
@@ -1993,7 +2008,8 @@ int agdu_maxpool_bwd_add(void const *dy, void const *arg, void const *add, int C
     fprintf(stderr, "ERROR: added channels %d at %d of %d unsupported\n", C, c0, Ca);
     return 1;
   }
-  return row_launch("maxpool_bwd", k_maxpool_bwd, N, D, H, W * (int64_t)(C / 8), stream,
+  return row_launch("maxpool_bwd", k_maxpool_bwd<unsigned>, k_maxpool_bwd<uint64_t>, N, D, H,
+                    W * (int64_t)(C / 8), stream,
                     (uint16_t const *)dy, (uint8_t const *)arg, (uint16_t *)dx, D, H, W, C,
                     (uint16_t const *)add, Ca, c0);
 }
@@ -2013,7 +2029,8 @@ int agdu_concat_up(void const *xu, void const *xs, void *y, int N, int D, int H,
     fprintf(stderr, "ERROR: concatenating %d and %d channels unsupported\n", CU, CS);
     return 1;
   }
-  return row_launch("concat_up", k_concat_up, N, D, H, W * (int64_t)((CU + CS) / 8), stream,
+  return row_launch("concat_up", k_concat_up<unsigned>, k_concat_up<uint64_t>, N, D, H,
+                    W * (int64_t)((CU + CS) / 8), stream,
                     (uint16_t const *)xu, (uint16_t const *)xs, (uint16_t *)y, D, H, W, CU, CS);
 }
 
@@ -2034,7 +2051,8 @@ int agdu_upsample_bwd(void const *dy, void *dx, int N, int D, int H, int W, int 
     fprintf(stderr, "ERROR: upsampling channels %d at %d of %d unsupported\n", C, c0, Cy);
     return 1;
   }
-  return row_launch("upsample_bwd", k_upsample_bwd, N, D, H, W * (int64_t)(C / 8), stream,
+  return row_launch("upsample_bwd", k_upsample_bwd<unsigned>, k_upsample_bwd<uint64_t>, N, D,
+                    H, W * (int64_t)(C / 8), stream,
                     (uint16_t const *)dy, (uint16_t *)dx, D, H, W, C, Cy, c0);
 }
 
