@@ -162,9 +162,6 @@ struct ConvWaves {
 // and per row of a block), the 27 taps become 4 (a, b) pairs x 3 w taps for
 // each of the 4 (pd, ph) parities: 48 combined taps, entry
 // ((pd * 2 + ph) * 4 + a * 2 + b) * 3 + kw.
-__host__ __device__ constexpr int up_tap(int pd, int ph, int a, int b, int kw) {
-  return (((pd * 2 + ph) * 4 + a * 2 + b) * 3) + kw;
-}
 
 // CU > 0: the input is the concatenation [upsample(xu), x] without being
 // formed: input channels [0, CU) are xu's ([n][D/2][H/2][W/2][CU], nearest
@@ -895,7 +892,7 @@ __global__ __launch_bounds__(UT, 2) void k_conv3s(uint16_t const *__restrict__ x
 }
 
 // Combined taps of the first CU input channels of wt ([27][CO][CI]):
-// wcu[up_tap(pd, ph, a, b, kw)][co][cu] = bf16(sum over the d taps kd of
+// wcu[((pd 2 + ph) 4 + a 2 + b) 3 + kw][co][cu] = bf16(sum over the d taps kd of
 // (pd, a) and the h taps kh of (ph, b) of wt[(kd * 3 + kh) * 3 + kw][co][cu]),
 // summed in fp32 in tap order. Taps of parity p and pair index a: p = 0:
 // {0}, {1, 2}; p = 1: {0, 1}, {2}.
@@ -1928,8 +1925,8 @@ int agdu_flip_weights(void const *wt, void *wtt, int CI, int CO, void *stream) {
   X(16, 16, 3) X(16, 32, 3) X(32, 32, 3) X(48, 16, 3) X(32, 16, 3) X(32, 64, 9) X(64, 64, 9) \
   X(96, 32, 9) X(64, 32, 9) X(16, 64, 3)
 
-// launch shape of the weight gradient: tile pairs (grid.y), rows per block
-// and blocks (grid.x); 0 when the channel pair has no kernel
+// launch shape of the weight gradient: tile pairs, rows per row chunk and row
+// chunks (each of 3 pairs blocks); 0 when the channel pair has no kernel
 static int wgrad_plan(int N, int D, int H, int W, int CI, int CO, int *pairs, int *rb,
                       int64_t *nblk) {
   int share = 0;
@@ -1953,8 +1950,7 @@ int64_t agdu_wgrad_part_len(int N, int D, int H, int W, int CI, int CO) {
   int pairs, rb;
   int64_t nblk;
   if (!wgrad_plan(N, D, H, W, CI, CO, &pairs, &rb, &nblk)) return -1;
-  int64_t const ng = (nblk + RED_PER - 1) / RED_PER;
-  return nblk * (27 * CI * CO + CO) + ng * (27 * CI * CO + CO);
+  return nblk * (27 * CI * CO + CO);
 }
 
 int agdu_conv3_wgrad(void const *x, void const *dy, float *part, float *dw, float *db, int N,
