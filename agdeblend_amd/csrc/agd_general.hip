@@ -5,7 +5,7 @@
 // or a few samples longer than asked for, so padded lengths such as 23, 42
 // or 43 are the usual case, not the exception. These kernels take the
 // lengths at run time. Every 1-D transform is a line held by one thread in
-// registers (line_dft): the DFT of P values on the pairs
+// registers (Line): the DFT of P values on the pairs
 //   a_k = x_k + x_{P-k},  b_k = x_k - x_{P-k},   0 < k < P / 2,
 //   X_q, X_{P-q} = (x_0 + (-1)^q x_{P/2} + sum a_k cos(2 pi q k / P))
 //                  +- i S sum b_k sin(2 pi q k / P),

@@ -28,7 +28,7 @@ typedef struct {
   AgdWin const *win;          /* [n_win] */
   AgdFftPlan const *plans;    /* FFT plans */
   float const *roots;         /* complex roots pool (interleaved) */
-  float const *dft;           /* line_dft coefficient pool */
+  float const *dft;           /* coefficients of the lines (Line::dft) */
   float const *tapers;        /* time taper pool */
   float const *tscale;        /* per global window trace: scaler * space tapers */
   float const *tconst;        /* per global window trace: space tapers only */
@@ -140,7 +140,8 @@ int agdg_adj_time(AgdDev const *g, float const *Tin, int plain);
  * without reading X. fuse: also write the forward spatial transform of the new X
  * into U (the next iteration's first forward stage). */
 int agdg_adj_spatial(AgdDev const *g, float alpha, float lamb, int mode, int fuse);
-/* 1 when every spatial class has a specialised kernel (fusion available) */
+/* 1 when every spatial class has a specialised or run-time sized kernel
+ * (fusion available; not in split precision) */
 int agdg_can_fuse(AgdDev const *g);
 /* number of spatial classes the split-precision transforms can serve */
 int agdg_x3_classes(AgdDev const *g);

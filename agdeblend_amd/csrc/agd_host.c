@@ -558,7 +558,7 @@ static void trace_coord(BlendCfg const *c, long shot, int ntimes, int channel,
 typedef struct {
   vec plans; /* AgdFftPlan */
   vec roots; /* float pairs */
-  vec dft;   /* line_dft coefficients (floats) */
+  vec dft;   /* the lines' coefficients (floats) */
 } PlanSet;
 
 static int planset_get(PlanSet *s, int n) {
@@ -602,7 +602,7 @@ static int planset_get(PlanSet *s, int n) {
   return (int)(s->plans.n - 1);
 }
 
-/* Offset of line_dft's coefficients of length n (agd_general.h), n > 0: for
+/* Offset of the coefficients of lines of length n (Line::dft), n > 0: for
  * q = 1 .. (n - 1) / 2 a row of the pairs cos, sin(2 pi q k / n), k = 1 ..
  * (n - 1) / 2, padded with zeros to groups of 4. -1 on error. */
 static int dft_get(PlanSet *s, int n) {

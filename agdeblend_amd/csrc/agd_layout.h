@@ -45,7 +45,7 @@ typedef struct {
   int nstage;
   int radix[AGD_MAXSTAGE];
   int roots_off; /* complex offset in the roots pool */
-  int dft_off;   /* float offset of line_dft's coefficients in the dft pool */
+  int dft_off;   /* float offset of the lines' coefficients (Line::dft) in the dft pool */
 } AgdFftPlan;
 
 typedef struct {
