@@ -26,6 +26,8 @@
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// four biases, of any float pointer
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -556,7 +558,7 @@ __global__ __launch_bounds__(UT, (ConvWaves<CO, UPC>::W)) void k_conv3(
     auto rows = [&](auto relu) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        f32x4 const b = (mode & 1) ? *(f32x4 const *)(bias + t * 16 + 4 * kq)
+        f32x4 const b = (mode & 1) ? *(f32x4u const *)(bias + t * 16 + 4 * kq)
                                    : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < 4; ++m)
@@ -756,7 +758,7 @@ __global__ __launch_bounds__(UT, 2) void k_conv3s(uint16_t const *__restrict__ x
   // loaded once: a load in the loop would be issued after the next plane's
   // prefetch, and waiting for it would wait for the prefetch too
   f32x4 const b =
-      (mode & 1) ? *(f32x4 const *)(bias + 4 * kq) : f32x4{0.f, 0.f, 0.f, 0.f};
+      (mode & 1) ? *(f32x4u const *)(bias + 4 * kq) : f32x4{0.f, 0.f, 0.f, 0.f};
   // LDS byte offsets of the lane's voxels in a plane, per step and (POOL)
   // tile row: the loop adds constants only
   int aof[POOL ? 2 : 1][5];
@@ -1448,6 +1450,7 @@ typedef uint8_t u8x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ u16x8 ld8(uint16_t const *p) { return *(u16x8 const *)p; }
 __device__ __forceinline__ void st8(uint16_t *p, u16x8 v) { *(u16x8 *)p = v; }
+typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
 
 // The training pass's resampling kernels take one (n, d, h) row of their
 // output per block (and, beyond the grid, the rows a grid apart): the row's
@@ -1675,7 +1678,7 @@ __global__ __launch_bounds__(UT) void k_l2_loss(uint16_t const *__restrict__ y,
     if (C % 8 == 0) {
       u16x8 o = {g, 0, 0, 0, 0, 0, 0, 0};
       for (int c = 0; c < C; c += 8) {
-        st8(dy + v * C + c, o);
+        *(u16x8u *)(dy + v * C + c) = o;  // any bf16 pointer, as below
         o[0] = 0;
       }
     } else {
