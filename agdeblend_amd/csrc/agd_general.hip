@@ -22,10 +22,10 @@
 // iteration: spatial transforms and update 15480 by the LDS-resident kernels
 // (radix passes through LDS with table roots, forward and adjoint apart) ->
 // 1640 lines as above -> 1620 with the codelets -> 990 with reciprocals for
-// integer divisions; it moves 3.9 GB, 820 us at this card's copy rate. Time
-// transforms 1460 and 1670 -> 480 and 500 -> 291 and 278. Prefetching the model's values
-// ahead of the transforms changed nothing (the lines' registers are worth
-// more as waves).
+// integer divisions (1000 with last tiles as wide as their traces); it moves
+// 3.9 GB, 820 us at this card's copy rate. Time transforms 1460 and 1670 ->
+// 480 and 500 -> 291 and 278. Prefetching the model's values ahead of the
+// transforms changed nothing (the lines' registers are worth more as waves).
 #include <hip/hip_runtime.h>
 
 #include "agd_fft.h"

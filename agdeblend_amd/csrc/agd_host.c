@@ -1271,7 +1271,7 @@ static int lines_nk(AgdWin const *W) {
  * within a 48 KB LDS tile of spec_len(a) rows of b + 1 per plane. One space
  * dim (a = 1): a plane is one row transform, a thread's work, so planes are
  * what fills a wave: up to 32, in tasks of equal size (256 x 1024 line,
- * windows 32 x 256: 30 us per launch with 6 planes, 12 with 27).
+ * windows 32 x 256: 30 us per launch with 6 planes, 16 with 27).
  * AGD_SPATIAL_NK overrides */
 static int default_nk(int a, int b, int Ft) {
   size_t const plane = (size_t)spec_len(a) * (b + 1) * 8;
