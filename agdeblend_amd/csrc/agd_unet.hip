@@ -1452,111 +1452,136 @@ __device__ __forceinline__ u16x8 ld8(uint16_t const *p) { return *(u16x8 const *
 __device__ __forceinline__ void st8(uint16_t *p, u16x8 v) { *(u16x8 *)p = v; }
 typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
 
-// The training pass's resampling kernels take one (n, d, h) row of their
-// output per block (and, beyond the grid, the rows a grid apart): the row's
-// indices are divided out once, a thread only splits its (w, 8 channels), in
-// 32 bits (64-bit divisions per 16 bytes had these kernels at 1.5 TB/s); I is
-// 64 bits for tensors whose rows or items per row need them.
-struct Row {
-  int n, d, h;
+// The training pass's resampling kernels: a thread per 16-byte item (n, d, h,
+// w, 8 channels) of their output, its indices by multiplication with the
+// sizes' reciprocals where there are fewer than 2^31 items. Pooling and its
+// gradient on 64 channels, us: 64-bit divisions per item 58 and 93 at 64 x 64 x
+// 512, 20 and 31 at 2 x 2 x 2 x 100000; one block per (n, d, h) row 65 and 87,
+// and 4530 and 1440 (the chip idle but for eight blocks); so 58 and 82, 19 and
+// 27.
+// n / d = n m >> s for n < 2^31: 2^(s - 31) >= d, m = ceil(2^s / d)
+struct Div {
+  uint32_t m, s, d;
 };
-template <typename I>
-__device__ __forceinline__ Row out_row(I row, int D, int H) {
-  I const nd = row / (I)H, n = nd / (I)D;
-  return Row{(int)n, (int)(nd - n * D), (int)(row - nd * H)};
+struct Item {
+  int n, d, h, w, c;
+};
+// sizes of an output in items: 8-channel groups, W, H, D
+struct Sizes32 {
+  typedef uint32_t Index;
+  Div c, w, h, d;
+};
+struct Sizes64 {
+  typedef uint64_t Index;
+  uint64_t c, w, h, d;
+};
+__device__ __forceinline__ uint32_t div_rem(uint32_t n, Div v, int &rem) {
+  uint32_t const q = (uint32_t)(((uint64_t)n * v.m) >> v.s);
+  rem = (int)(n - q * v.d);
+  return q;
 }
+__device__ __forceinline__ uint64_t div_rem(uint64_t n, uint64_t v, int &rem) {
+  rem = (int)(n % v);
+  return n / v;
+}
+template <typename S>
+__device__ __forceinline__ Item item_at(typename S::Index i, S const &z) {
+  Item r;
+  i = div_rem(i, z.c, r.c);
+  r.c *= 8;
+  i = div_rem(i, z.w, r.w);
+  i = div_rem(i, z.h, r.h);
+  r.n = (int)div_rem(i, z.d, r.d);
+  return r;
+}
+#define ITEMS(idx, S, total)                                                        \
+  for (typename S::Index idx = (typename S::Index)blockIdx.x * UT + threadIdx.x; idx < total; \
+       idx += (typename S::Index)gridDim.x * UT)
 
 // 2x2x2 max pool: y[n][d][h][w][c] over x[n][2d..][2h..][2w..][c]; arg holds
 // the winning offset (first maximum in (a, b, e) order). D, H, W: of y
-template <typename I>
-__global__ void k_maxpool(uint16_t const *__restrict__ x, uint16_t *__restrict__ y,
-                          uint8_t *__restrict__ arg, int D, int H, int W, int C, I rows) {
-  I const C8 = C / 8;
-  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
-    Row const r = out_row(row, D, H);
-    int64_t const out0 = (int64_t)row * W * C;
-    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
-      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
-      float best[8];
-      int barg[8];
+template <typename S>
+__global__ __launch_bounds__(UT) void k_maxpool(uint16_t const *__restrict__ x,
+                                                uint16_t *__restrict__ y,
+                                                uint8_t *__restrict__ arg, int D, int H, int W,
+                                                int C, S z, typename S::Index total) {
+  ITEMS(idx, S, total) {
+    Item const r = item_at(idx, z);
+    float best[8];
+    int barg[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      best[k] = -INFINITY;
+      barg[k] = 0;
+    }
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
+      int64_t const row = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
+      u16x8 const v = ld8(x + (row * 2 * W + 2 * r.w + e) * C + r.c);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        best[k] = -INFINITY;
-        barg[k] = 0;
-      }
-#pragma unroll
-      for (int o = 0; o < 8; ++o) {
-        int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
-        int64_t const xrow = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
-        u16x8 const v = ld8(x + (xrow * 2 * W + 2 * w + e) * C + c);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          float const f = bf2f(v[k]);
-          if (f > best[k]) {
-            best[k] = f;
-            barg[k] = o;
-          }
+        float const f = bf2f(v[k]);
+        if (f > best[k]) {
+          best[k] = f;
+          barg[k] = o;
         }
       }
-      u16x8 out;
-      u8x8 ar;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        out[k] = f2bf(best[k]);
-        ar[k] = (uint8_t)barg[k];
-      }
-      st8(y + out0 + (int64_t)idx * 8, out);
-      *(u8x8 *)(arg + out0 + (int64_t)idx * 8) = ar;
     }
+    u16x8 out;
+    u8x8 ar;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      out[k] = f2bf(best[k]);
+      ar[k] = (uint8_t)barg[k];
+    }
+    st8(y + (int64_t)idx * 8, out);
+    *(u8x8 *)(arg + (int64_t)idx * 8) = ar;
   }
 }
 
 // gradient of the pooling, D, H, W: of dx. add (or NULL): a second gradient of
 // the pooled tensor's input, its channels [c0, c0 + C) of Ca, added in fp32 and
 // rounded once (as k_copy_channels mode 1 on the written dx)
-template <typename I>
-__global__ void k_maxpool_bwd(uint16_t const *__restrict__ dy, uint8_t const *__restrict__ arg,
-                              uint16_t *__restrict__ dx, int D, int H, int W, int C,
-                              uint16_t const *__restrict__ add, int Ca, int c0, I rows) {
-  I const C8 = C / 8;
-  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
-    Row const r = out_row(row, D, H);
+template <typename S>
+__global__ __launch_bounds__(UT) void k_maxpool_bwd(
+    uint16_t const *__restrict__ dy, uint8_t const *__restrict__ arg, uint16_t *__restrict__ dx,
+    int D, int H, int W, int C, uint16_t const *__restrict__ add, int Ca, int c0, S z,
+    typename S::Index total) {
+  ITEMS(idx, S, total) {
+    Item const r = item_at(idx, z);
     int64_t const prow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
-    int const mine = ((r.d & 1) << 2) | ((r.h & 1) << 1);
-    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
-      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
-      int64_t const o = (prow * (W / 2) + w / 2) * C + c;
-      u16x8 const g = ld8(dy + o);
-      u8x8 const a = *(u8x8 const *)(arg + o);
-      u16x8 out;
+    int64_t const o = (prow * (W / 2) + r.w / 2) * C + r.c;
+    int const mine = ((r.d & 1) << 2) | ((r.h & 1) << 1) | (r.w & 1);
+    u16x8 const g = ld8(dy + o);
+    u8x8 const a = *(u8x8 const *)(arg + o);
+    u16x8 out;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) out[k] = a[k] == (mine | (w & 1)) ? g[k] : (uint16_t)0;
-      if (add != nullptr) {
-        u16x8 const s = ld8(add + ((int64_t)row * W + w) * Ca + c0 + c);
+    for (int k = 0; k < 8; ++k) out[k] = a[k] == mine ? g[k] : (uint16_t)0;
+    if (add != nullptr) {
+      int64_t const v = (((int64_t)r.n * D + r.d) * H + r.h) * W + r.w;
+      u16x8 const s = ld8(add + v * Ca + c0 + r.c);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) out[k] = f2bf(bf2f(s[k]) + bf2f(out[k]));
-      }
-      st8(dx + ((int64_t)row * W + w) * C + c, out);
+      for (int k = 0; k < 8; ++k) out[k] = f2bf(bf2f(s[k]) + bf2f(out[k]));
     }
+    st8(dx + (int64_t)idx * 8, out);
   }
 }
 
 // y = [upsample(xu), xs]: the nearest x2 upsampling of xu (CU channels) and xs
 // (CS channels) side by side, whole voxels of y [n][D][H][W][CU + CS] at a time
-template <typename I>
-__global__ void k_concat_up(uint16_t const *__restrict__ xu, uint16_t const *__restrict__ xs,
-                            uint16_t *__restrict__ y, int D, int H, int W, int CU, int CS, I rows) {
-  I const C8 = (CU + CS) / 8;
-  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
-    Row const r = out_row(row, D, H);
+template <typename S>
+__global__ __launch_bounds__(UT) void k_concat_up(uint16_t const *__restrict__ xu,
+                                                  uint16_t const *__restrict__ xs,
+                                                  uint16_t *__restrict__ y, int D, int H, int W,
+                                                  int CU, int CS, S z, typename S::Index total) {
+  ITEMS(idx, S, total) {
+    Item const r = item_at(idx, z);
     int64_t const urow = ((int64_t)r.n * (D / 2) + r.d / 2) * (H / 2) + r.h / 2;
-    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
-      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
-      uint16_t const *const q = c < CU
-                                    ? xu + (urow * (W / 2) + w / 2) * CU + c
-                                    : xs + ((int64_t)row * W + w) * CS + (c - CU);
-      st8(y + (int64_t)row * W * (CU + CS) + (int64_t)idx * 8, ld8(q));
-    }
+    int64_t const v = (((int64_t)r.n * D + r.d) * H + r.h) * W + r.w;
+    uint16_t const *const q = r.c < CU ? xu + (urow * (W / 2) + r.w / 2) * CU + r.c
+                                       : xs + v * CS + (r.c - CU);
+    st8(y + (int64_t)idx * 8, ld8(q));
   }
 }
 
@@ -1583,30 +1608,28 @@ __global__ void k_upsample(uint16_t const *__restrict__ x, uint16_t *__restrict_
 
 // gradient of the upsampling: dx[v][c] = sum of the 8 children's
 // dy[..][c0 + c], in a fixed order; accumulated in fp32. D, H, W: of dx
-template <typename I>
-__global__ void k_upsample_bwd(uint16_t const *__restrict__ dy, uint16_t *__restrict__ dx, int D,
-                               int H, int W, int C, int Cy, int c0, I rows) {
-  I const C8 = C / 8;
-  for (I row = blockIdx.x; row < rows; row += gridDim.x) {
-    Row const r = out_row(row, D, H);
-    for (I idx = threadIdx.x; idx < (I)W * C8; idx += blockDim.x) {
-      int const w = (int)(idx / C8), c = (int)(idx - (I)w * C8) * 8;
-      float s[8];
+template <typename S>
+__global__ __launch_bounds__(UT) void k_upsample_bwd(uint16_t const *__restrict__ dy,
+                                                     uint16_t *__restrict__ dx, int D, int H,
+                                                     int W, int Cy, int c0, S z,
+                                                     typename S::Index total) {
+  ITEMS(idx, S, total) {
+    Item const r = item_at(idx, z);
+    float s[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) s[k] = 0.f;
+    for (int k = 0; k < 8; ++k) s[k] = 0.f;
 #pragma unroll
-      for (int o = 0; o < 8; ++o) {
-        int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
-        int64_t const yrow = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
-        u16x8 const g = ld8(dy + (yrow * 2 * W + 2 * w + e) * Cy + c0 + c);
+    for (int o = 0; o < 8; ++o) {
+      int const a = o >> 2, b = (o >> 1) & 1, e = o & 1;
+      int64_t const row = ((int64_t)r.n * 2 * D + 2 * r.d + a) * 2 * H + 2 * r.h + b;
+      u16x8 const g = ld8(dy + (row * 2 * W + 2 * r.w + e) * Cy + c0 + r.c);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) s[k] += bf2f(g[k]);
-      }
-      u16x8 out;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) out[k] = f2bf(s[k]);
-      st8(dx + (int64_t)row * W * C + (int64_t)idx * 8, out);
+      for (int k = 0; k < 8; ++k) s[k] += bf2f(g[k]);
     }
+    u16x8 out;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) out[k] = f2bf(s[k]);
+    st8(dx + (int64_t)idx * 8, out);
   }
 }
 
@@ -1737,18 +1760,28 @@ static inline int64_t blocks_capped(int64_t n, int t) {
   return b < (1 << 20) ? b : (1 << 20);
 }
 
-// a kernel of (n, d, h) rows of `items` 16-byte items, a block each up to 2^20
-// blocks (a launch holds less than 2^32 threads); small: the instance with
-// 32-bit indices, large: 64-bit
+static Div div_by(uint32_t d) {
+  Div v = {0, 31, d};
+  while (((uint64_t)1 << (v.s - 31)) < d) ++v.s;
+  v.m = (uint32_t)((((uint64_t)1 << v.s) + d - 1) / d);
+  return v;
+}
+
+// a kernel of one thread per item of an [N][D][H][W][8 C8] output; small: its
+// instance for fewer than 2^31 items, large: for any number
 template <typename K, typename L, typename... A>
-static int row_launch(char const *name, K small, L large, int N, int D, int H, int64_t items,
-                      void *stream, A... args) {
-  int64_t const rows = (int64_t)N * D * H;
-  int const t = items >= UT ? UT : (int)((items + 63) / 64 * 64);
-  dim3 const grid((unsigned)(rows < (1 << 20) ? rows : 1 << 20)), block(t > 0 ? t : 64);
-  if (rows < 0x7fffffff && items < 0x7fffffff)
-    return ulaunch(name, small, grid, block, stream, args..., (unsigned)rows);
-  return ulaunch(name, large, grid, block, stream, args..., (uint64_t)rows);
+static int item_launch(char const *name, K small, L large, int N, int D, int H, int W, int C8,
+                       void *stream, A... args) {
+  int64_t const total = (int64_t)N * D * H * W * C8;
+  dim3 const grid((unsigned)blocks_capped(total, UT));
+  if (total <= 0) return 0;
+  if (total < 0x7fffffff)
+    return ulaunch(name, small, grid, dim3(UT), stream, args...,
+                   Sizes32{div_by((uint32_t)C8), div_by((uint32_t)W), div_by((uint32_t)H),
+                           div_by((uint32_t)D)},
+                   (uint32_t)total);
+  return ulaunch(name, large, grid, dim3(UT), stream, args...,
+                 Sizes64{(uint64_t)C8, (uint64_t)W, (uint64_t)H, (uint64_t)D}, (uint64_t)total);
 }
 
 extern "C" {
@@ -1988,9 +2021,9 @@ int agdu_maxpool(void const *x, void *y, void *arg, int N, int D, int H, int W, 
     fprintf(stderr, "ERROR: channel count %d is not a multiple of 8\n", C);
     return 1;
   }
-  return row_launch("maxpool", k_maxpool<unsigned>, k_maxpool<uint64_t>, N, D / 2, H / 2,
-                    (W / 2) * (int64_t)(C / 8), stream,
-                    (uint16_t const *)x, (uint16_t *)y, (uint8_t *)arg, D / 2, H / 2, W / 2, C);
+  return item_launch("maxpool", k_maxpool<Sizes32>, k_maxpool<Sizes64>, N, D / 2, H / 2, W / 2,
+                     C / 8, stream, (uint16_t const *)x, (uint16_t *)y, (uint8_t *)arg, D / 2,
+                     H / 2, W / 2, C);
 }
 
 int agdu_maxpool_bwd_add(void const *dy, void const *arg, void const *add, int Ca, int c0,
@@ -2007,10 +2040,9 @@ int agdu_maxpool_bwd_add(void const *dy, void const *arg, void const *add, int C
     fprintf(stderr, "ERROR: added channels %d at %d of %d unsupported\n", C, c0, Ca);
     return 1;
   }
-  return row_launch("maxpool_bwd", k_maxpool_bwd<unsigned>, k_maxpool_bwd<uint64_t>, N, D, H,
-                    W * (int64_t)(C / 8), stream,
-                    (uint16_t const *)dy, (uint8_t const *)arg, (uint16_t *)dx, D, H, W, C,
-                    (uint16_t const *)add, Ca, c0);
+  return item_launch("maxpool_bwd", k_maxpool_bwd<Sizes32>, k_maxpool_bwd<Sizes64>, N, D, H, W,
+                     C / 8, stream, (uint16_t const *)dy, (uint8_t const *)arg, (uint16_t *)dx, D,
+                     H, W, C, (uint16_t const *)add, Ca, c0);
 }
 
 int agdu_maxpool_bwd(void const *dy, void const *arg, void *dx, int N, int D, int H, int W,
@@ -2028,9 +2060,9 @@ int agdu_concat_up(void const *xu, void const *xs, void *y, int N, int D, int H,
     fprintf(stderr, "ERROR: concatenating %d and %d channels unsupported\n", CU, CS);
     return 1;
   }
-  return row_launch("concat_up", k_concat_up<unsigned>, k_concat_up<uint64_t>, N, D, H,
-                    W * (int64_t)((CU + CS) / 8), stream,
-                    (uint16_t const *)xu, (uint16_t const *)xs, (uint16_t *)y, D, H, W, CU, CS);
+  return item_launch("concat_up", k_concat_up<Sizes32>, k_concat_up<Sizes64>, N, D, H, W,
+                     (CU + CS) / 8, stream, (uint16_t const *)xu, (uint16_t const *)xs,
+                     (uint16_t *)y, D, H, W, CU, CS);
 }
 
 int agdu_upsample(void const *x, void *y, int N, int D, int H, int W, int C, int Cy, int c0,
@@ -2050,9 +2082,8 @@ int agdu_upsample_bwd(void const *dy, void *dx, int N, int D, int H, int W, int 
     fprintf(stderr, "ERROR: upsampling channels %d at %d of %d unsupported\n", C, c0, Cy);
     return 1;
   }
-  return row_launch("upsample_bwd", k_upsample_bwd<unsigned>, k_upsample_bwd<uint64_t>, N, D,
-                    H, W * (int64_t)(C / 8), stream,
-                    (uint16_t const *)dy, (uint16_t *)dx, D, H, W, C, Cy, c0);
+  return item_launch("upsample_bwd", k_upsample_bwd<Sizes32>, k_upsample_bwd<Sizes64>, N, D, H,
+                     W, C / 8, stream, (uint16_t const *)dy, (uint16_t *)dx, D, H, W, Cy, c0);
 }
 
 int agdu_copy_channels(void const *x, void *y, int64_t nvox, int Cx, int cx0, int Cy,

@@ -1,6 +1,7 @@
-"""The resampling kernels on more rows than a launch has blocks for: one block
-per row of a volume of 2 x (2^25 + 2) rows would be more threads than a
-launch may have (2^32). Bit for bit against torch (whole-voxel copies, one
+"""The resampling kernels on very many and on very few rows. One block per
+row of a volume of 2 x (2^25 + 2) rows would be more threads than a
+launch may have (2^32), and on eight rows of 100000 voxels it would leave the
+chip idle (ninety times the time of as many voxels in a cube). Bit for bit against torch (whole-voxel copies, one
 winner of a pooling window, the maximum itself; the upsampling's gradient of
 eight equal powers of two, exact in bf16)."""
 import pytest
@@ -67,3 +68,35 @@ def test_concatenation_and_upsampling_gradient():
     assert L.agdu_upsample_bwd(_p(dy), _p(dx), N, D, H, 1, 8, 8, 0, None) == 0
     torch.cuda.synchronize()
     assert torch.equal(dx, g * 8)
+
+
+def _us(call):
+    call()
+    best = 1e9
+    for _ in range(5):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in "ab")
+        a.record()
+        for _ in range(10):
+            assert call() == 0
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 100)
+    return best
+
+
+def test_few_long_rows_take_no_longer():
+    L = _lib()
+    times = []
+    for d, h, w in ((2, 2, 100000), (20, 20, 1000)):
+        x = _values(2, d, h, w, 32)
+        y = torch.empty(2, d // 2, h // 2, w // 2, 32, dtype=torch.bfloat16, device="cuda")
+        arg = torch.empty(y.shape, dtype=torch.uint8, device="cuda")
+        cat = torch.empty(2, d, h, w, 64, dtype=torch.bfloat16, device="cuda")
+        st = torch.cuda.current_stream().cuda_stream
+        times.append([
+            _us(lambda: L.agdu_maxpool(_p(x), _p(y), _p(arg), 2, d, h, w, 32, st)),
+            _us(lambda: L.agdu_maxpool_bwd(_p(y), _p(arg), _p(x), 2, d, h, w, 32, st)),
+            _us(lambda: L.agdu_concat_up(_p(y), _p(x), _p(cat), 2, d, h, w, 32, 32, st)),
+            _us(lambda: L.agdu_upsample_bwd(_p(x), _p(y), 2, d // 2, h // 2, w // 2, 32, 32, 0, st))])
+    print("us of eight rows", times[0], "of a cube", times[1], flush=True)
+    assert all(a < 3 * b + 5 for a, b in zip(*times))
