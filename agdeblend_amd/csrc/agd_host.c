@@ -1263,6 +1263,43 @@ static int lines_nk(AgdWin const *W) {
   return best;
 }
 
+/* The window's choices and coefficients for the run-time sized kernels; those
+ * of prev where its sizes are the same (neighbours' usually are: chosen anew
+ * for each of 12321 windows of 4 x 4 x 50 they took a fifth of the problem's
+ * creation) */
+static int run_time_sizes(PlanSet *s, AgdWin *W, AgdWin const *prev) {
+  int d, m1, m2, same = prev != NULL && prev->nsp == W->nsp && prev->Wt == W->Wt;
+  for (d = 0; same && d < W->nsp; d++) same = prev->W[d] == W->W[d] && prev->P[d] == W->P[d];
+  if (same) {
+    memcpy(W->sdft, prev->sdft, sizeof(W->sdft));
+    memcpy(W->sfac, prev->sfac, sizeof(W->sfac));
+    W->slines = prev->slines;
+    W->snk = prev->snk;
+    W->gm1 = prev->gm1;
+    W->gm2 = prev->gm2;
+    W->gm3 = prev->gm3;
+    W->tdft1 = prev->tdft1;
+    W->tdft2 = prev->tdft2;
+    return 0;
+  }
+  for (d = 0; d < W->nsp; d++) W->sfac[d] = line_factor(W->P[d]);
+  spatial_key(W, &m1, &m2);
+  W->slines = m1 ? 0 : spatial_lines(W);
+  if (W->slines) {
+    W->snk = lines_nk(W);
+    /* lines that fold need no coefficients */
+    for (d = 0; d < W->nsp; d++)
+      if (W->slines != AGD_FACTORED && (W->slines != AGD_FOLDED_LINES || W->sfac[d] <= 1) &&
+          (W->sdft[d] = dft_get(s, W->P[d])) < 0)
+        return 1;
+  }
+  time_key(W, &m1, &m2);
+  if (m1) return 0;
+  time_lines(W);
+  return W->gm2 && W->gm3 == 0 &&
+         ((W->tdft1 = dft_get(s, W->gm1)) < 0 || (W->tdft2 = dft_get(s, W->gm2)) < 0);
+}
+
 /* Spatial tasks (chunks of time-frequency planes) and time blocks (runs of
  * traces), each grouped into classes of windows with equal transform
  * sizes; a class is served by one kernel launch. */
@@ -1306,10 +1343,10 @@ static int spatial_tasks(AgdProblem *p, AgdClass *cls, int ncls, int const *nk_r
       wpos[w] = (int)tasks->n - cl->begin;
       spatial_key(W, &a, &b);
       time_key(W, &tm, &tn);
-      if (a != cl->p0 || b != cl->p1 || (a ? (tm > 0) != cl->tb : spatial_lines(W) != cl->hb))
+      if (a != cl->p0 || b != cl->p1 || (a ? (tm > 0) != cl->tb : W->slines != cl->hb))
         continue;
       if (cl->hb) {
-        nk = lines_nk(W);
+        nk = W->snk;
       } else if (a) {
         nk = (nk_req && nk_req[c] > 0) ? nk_req[c] : default_nk(a, b, W->Ft);
       } else {
@@ -1416,7 +1453,7 @@ static int build_classes(AgdProblem *p, vec *tasks, vec *tblocks, size_t *lds_sp
     AgdClass *cl = (AgdClass *)sc.p;
     spatial_key(W, &a, &b);
     time_key(W, &tm, &tn);
-    hb = a ? 0 : spatial_lines(W);
+    hb = W->slines;
     for (c = 0; c < (int)sc.n; c++)
       if (cl[c].p0 == a && cl[c].p1 == b && (a ? cl[c].tb == (tm > 0) : cl[c].hb == hb)) found = 1;
     if (!found) {
@@ -1672,26 +1709,7 @@ static AgdProblem *create_impl(int np, int const *volumes, int const *n_dims,
       if (W->tplan < 0 || W->tplan_full < 0) goto err;
       W->wplan = -1;
       W->wplan_full = -1;
-      {
-        /* coefficients of the run-time sized kernels */
-        int m1, m2;
-        spatial_key(W, &m1, &m2);
-        for (d = 0; d < nsp; d++) {
-          W->sdft[d] = 0;
-          W->sfac[d] = line_factor(W->P[d]);
-        }
-        if (m1 == 0 && spatial_lines(W))
-          for (d = 0; d < nsp; d++)
-            if ((W->sdft[d] = dft_get(&ps, W->P[d])) < 0) goto err;
-        time_key(W, &m1, &m2);
-        if (m1 == 0) {
-          time_lines(W);
-          if (W->gm2 && W->gm3 == 0 &&
-              ((W->tdft1 = dft_get(&ps, W->gm1)) < 0 ||
-               (W->tdft2 = dft_get(&ps, W->gm2)) < 0))
-            goto err;
-        }
-      }
+      if (run_time_sizes(&ps, W, w > 0 ? W - 1 : NULL)) goto err;
       /* time windows start at whole cache lines of U and V where that is at
        * most 1.5 % of them, else at whole 16-byte loads */
       {

@@ -70,6 +70,7 @@ typedef struct {
    * dim; Pt = gm1 * gm2 * gm3 in register FFTs, or (gm3 0) gm1 * gm2 in
    * lines with their coefficients' offsets (gm2 0: none) */
   int sdft[AGD_MAXSP];
+  int slines, snk;     /* the class's hb and the planes per task (host) */
   int sfac[AGD_MAXSP]; /* first factor of P, A B = P (1: P one FFT, 0: does not fold) */
   int gm1, gm2, gm3;
   int tdft1, tdft2;
