@@ -926,7 +926,11 @@ template <int HB>
 static int launch_fwd_time_g(AgdDev const *g, AgdClass const &c, int first, int n) {
   static int const lds_ok = allow_lds((void const *)k_fwd_time_g<HB>);
   (void)lds_ok;
-  return launch("fwd_time", k_fwd_time_g<HB>, dim3(n, time_split(g, c, n, 2)), dim3(NTHR), c.lds, g->win,
+  // by registers, and by the LDS of a CU
+  static int const held = agd_resident((void const *)k_fwd_time_g<HB>, NTHR, 0);
+  int const fits = agd_compute_units() * (int)(160 * 1024 / c.lds);
+  int const runs = time_split_fwd(g, c, n, held < fits ? held : fits);
+  return launch("fwd_time", k_fwd_time_g<HB>, dim3(n, runs), dim3(NTHR), c.lds, g->win,
                 g->tblocks, first, g->dft, g->plans, (float2 const *)g->roots, g->tapers,
                 g->tscale, (float2 const *)g->U, g->T);
 }

@@ -64,20 +64,44 @@ static inline int allow_lds(void const *f) {
   return 1;
 }
 
-// Runs that a launch of n time blocks of class c splits each block's time
+// the card's compute units, and the blocks of `threads` threads and lds bytes of
+// dynamic LDS that it holds at once of a kernel (asked once per instance)
+int agd_compute_units(void);
+int agd_resident(void const *kernel, int threads, size_t lds);
+
+// Most runs that a launch of n time blocks of class c splits each block's time
 // windows into (grid y), at least `least` time windows to a run. A block's
 // time windows are a serial chain, so below TIME_SPLIT_BLOCKS blocks (six
 // per CU) the chip waits on it: 30 blocks of 9 time windows (256 x 1024
 // line, windows 32 x 256) took 27 us forward and 34 adjoint as one run each
-// and take 15 and 11 split, 236 blocks of 14 (1510 x 1251 line, in lines; in
-// register FFTs 41 and 32) 113 and 132 against 67 and 52; above it the runs
-// would only repeat the forward's carry windows. (1024 to 3072 blocks, rounded
-// up or down, move that line by -6 % and 2400 x 2048 in windows of 48 x 64 by
-// +10 %, others by less than their spread.) Runs given by AGD_TIME_TW are
-// left as they are.
-static inline unsigned time_split(AgdDev const *g, AgdClass const &c, int n, int least) {
+// and take 15 and 11 split, 236 blocks of 14 (1510 x 1251 line, windows 50 x
+// 200) 143 and 169 and 36 and 33. Runs given by AGD_TIME_TW are left as they
+// are.
+static inline int time_split(AgdDev const *g, AgdClass const &c, int n, int least) {
   if (!g->split_time) return 1;
   int const want = (TIME_SPLIT_BLOCKS + n - 1) / n, most = c.ntw / least;
   int const r = want < most ? want : most;
   return r > 1 ? r : 1;
+}
+
+// The forward's runs, each of which repeats the time window before it for its
+// carry: of the counts up to the most, the one whose rounds of resident blocks
+// take the fewest time windows one after the other. By the count of blocks
+// alone, 1280 runs of 2 of 4 time windows (40 x 96 x 384 in windows of 16 x 32 x
+// 256, 768 blocks resident) took 29 us, the 640 blocks as one run each 25; the
+// line of 1510 x 1251 43 us in runs of 2, 36 in runs of 3; 1800 x 2000 in windows
+// of 18 x 500 197 and, as one run each, 148.
+static inline int time_split_fwd(AgdDev const *g, AgdClass const &c, int n, int resident) {
+  int const most = time_split(g, c, n, 2);
+  int best = 1;
+  int64_t best_cost = 0;
+  for (int r = 1; r <= most; ++r) {
+    int64_t const rounds = ((int64_t)n * r + resident - 1) / resident;
+    int64_t const cost = rounds * ((c.ntw + r - 1) / r + (r > 1));
+    if (r == 1 || cost < best_cost) {
+      best = r;
+      best_cost = cost;
+    }
+  }
+  return best;
 }

@@ -1,0 +1,40 @@
+"""The forward's split pays for the time window that every run repeats: on
+launches that fill the card it takes no longer than one run per block."""
+import numpy as np
+import pytest
+
+from agdeblend_amd import lib as L
+from tests.test_gpu_parity import _kw, _spec_geometry
+
+pytestmark = pytest.mark.gpu
+
+
+def _forward_us(kw, one_run, monkeypatch):
+    if one_run:
+        monkeypatch.setenv("AGD_TIME_TW", "0")
+    else:
+        monkeypatch.delenv("AGD_TIME_TW", raising=False)
+    pm = L.Problem(**kw)
+    try:
+        x = np.ones(pm.model_len, np.complex64)
+        pm.forward(x)
+        best = 1e9
+        for _ in range(12):
+            L.timing(True)
+            pm.forward(x)
+            L.timing(False)
+            ms, n = L.timing_get("fwd_time")
+            best = min(best, ms / n)
+        return best * 1e3
+    finally:
+        pm.close()
+
+
+@pytest.mark.parametrize("shape,windows", [((40, 96, 384), (16, 32, 256)),
+                                           ((36, 144, 384), (8, 32, 256)),
+                                           ((1800, 2000), (18, 500))])
+def test_split_forward_is_no_slower_than_one_run(shape, windows, monkeypatch):
+    kw = _kw(_spec_geometry(shape, windows, 3))
+    one, split = (_forward_us(kw, v, monkeypatch) for v in (True, False))
+    print(shape, windows, "one run %.1f us, split %.1f us" % (one, split), flush=True)
+    assert split <= 1.08 * one
